@@ -607,25 +607,25 @@ __device__ __forceinline__ int32_t recombine(int32_t hh, int32_t mid, int32_t ll
 
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-// Store one wave's 64 x 64 results.  A lane holds D[8 (r / 4) + 4 lh + r % 4][l32] of each
-// 32 x 32 block.  With PAIRS, lanes 2c and 2c + 1 swap one result per row pair (DPP
+// Store one wave's (32 RB) x (32 CB) results.  A lane holds D[8 (r / 4) + 4 lh + r % 4][l32] of
+// each 32 x 32 block.  With PAIRS, lanes 2c and 2c + 1 swap one result per row pair (DPP
 // quad_perm [1,0,3,2]) so that the even lane stores columns (2c, 2c + 1) of row r and the
 // odd lane the same columns of row r + 1, as one 4-byte store each.
-template <uint32_t MODE, bool PAIRS, class Epi>
-__device__ __forceinline__ void store_wave_tile(const v16i (&hh)[2][2], const v16i (&mid)[2][2],
-                                                const v16i (&ll)[2][2], const int2* rterm, const int2* cterm,
+template <uint32_t MODE, bool PAIRS, int RB, int CB, class Epi>
+__device__ __forceinline__ void store_wave_tile(const v16i (&hh)[RB][CB], const v16i (&mid)[RB][CB],
+                                                const v16i (&ll)[RB][CB], const int2* rterm, const int2* cterm,
                                                 uint32_t bt, uint32_t row0, uint32_t col0, uint32_t wr,
                                                 uint32_t wc, uint32_t l32, uint32_t lh, const Epi& epi) {
     const uint32_t odd = l32 & 1;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const uint32_t cl = wc * 64 + j * 32 + l32, col = col0 + cl;
+    for (int j = 0; j < CB; j++) {
+        const uint32_t cl = wc * (32 * CB) + j * 32 + l32, col = col0 + cl;
         const int2 ct = cterm[cl];
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < RB; i++) {
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
-                const uint32_t rl = wr * 64 + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+                const uint32_t rl = wr * (32 * RB) + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
                 const int2 r0 = rterm[rl], r1 = rterm[rl + 1];
                 const int32_t q0 = recombine<MODE>(hh[i][j][r], mid[i][j][r], ll[i][j][r], r0.x + ct.x, r0.y + ct.y,
                                                    epi.lo, epi.hi);
@@ -648,7 +648,7 @@ __device__ __forceinline__ void store_wave_tile(const v16i (&hh)[2][2], const v1
                 }
                 // one row pair at a time: hoisting the term loads of later pairs would
                 // need more registers than the accumulators leave
-                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (RB * CB >= 4) __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
@@ -656,21 +656,21 @@ __device__ __forceinline__ void store_wave_tile(const v16i (&hh)[2][2], const v1
 
 // store_wave_tile for a tile wholly inside the output with plain rows (tile_base): the lane's
 // offset from the tile's first element in 32 bits, the row offsets uniform, no bounds checks.
-template <uint32_t MODE>
-__device__ __forceinline__ void store_wave_fast(const v16i (&hh)[2][2], const v16i (&mid)[2][2],
-                                                const v16i (&ll)[2][2], const int2* rterm, const int2* cterm,
+template <uint32_t MODE, int RB, int CB>
+__device__ __forceinline__ void store_wave_fast(const v16i (&hh)[RB][CB], const v16i (&mid)[RB][CB],
+                                                const v16i (&ll)[RB][CB], const int2* rterm, const int2* cterm,
                                                 int16_t* __restrict__ base, uint32_t ld, uint32_t wr, uint32_t wc,
                                                 uint32_t l32, uint32_t lh, int32_t lo, int32_t hi) {
     const uint32_t odd = l32 & 1;
-    const uint32_t lane_off = (wr * 64 + 4 * lh + odd) * ld + wc * 64 + l32 - odd;
+    const uint32_t lane_off = (wr * (32 * RB) + 4 * lh + odd) * ld + wc * (32 * CB) + l32 - odd;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int2 ct = cterm[wc * 64 + j * 32 + l32];
+    for (int j = 0; j < CB; j++) {
+        const int2 ct = cterm[wc * (32 * CB) + j * 32 + l32];
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < RB; i++) {
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
-                const uint32_t rl = wr * 64 + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+                const uint32_t rl = wr * (32 * RB) + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
                 const int2 r0 = rterm[rl], r1 = rterm[rl + 1];
                 const int32_t q0 = recombine<MODE>(hh[i][j][r], mid[i][j][r], ll[i][j][r], r0.x + ct.x, r0.y + ct.y,
                                                    lo, hi);
@@ -682,16 +682,16 @@ __device__ __forceinline__ void store_wave_fast(const v16i (&hh)[2][2], const v1
                 const uint32_t lo = (uint32_t)(odd ? got : q0), hi = (uint32_t)(odd ? q1 : got);
                 const uint32_t roff = (uint32_t)(i * 32 + 8 * (r >> 2) + (r & 3)) * ld + j * 32;
                 *reinterpret_cast<uint32_t*>(base + lane_off + roff) = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (RB * CB >= 4) __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
 }
 
 // kSplitFix: this slice's partial of its wave's 64 x 64 outputs, in the accumulators' own
-// layout (a tile's nz slices are consecutive blocks of TM x 128 int32 at `tile_part`; in a
-// block, wave w's accumulator (i, j) rows 4q .. 4q + 3 sit at 1 KiB row (4 (2i + j) + q) of
-// the wave's 16 KiB, 16 bytes a lane), written and read with agent-scope 16-byte buffer
+// layout (a tile's nz slices are consecutive blocks of NW RB CB KiB x 4 at `tile_part`, NW the
+// workgroup's waves; in a block, wave w's accumulator (i, j) rows 4q .. 4q + 3 sit at 1 KiB row
+// (4 (CB i + j) + q) of the wave's 4 RB CB KiB, 16 bytes a lane), written and read with agent-scope 16-byte buffer
 // accesses (sc1) so that a workgroup on another XCD reads them; then the tile's arrival count.
 // The slice that arrives last (ticket nz - 1) resets the count for the next launch, adds the
 // other slices' partials (all were stored, and their stores had completed, before their slices
@@ -699,29 +699,29 @@ __device__ __forceinline__ void store_wave_fast(const v16i (&hh)[2][2], const v1
 // MID = (T >> 8) & 255, LL = T & 255, 2^16 HH + 2^8 MID + LL = T exactly -- for the kWrap
 // store; the other slices return false.  No workgroup waits for another.  Every wave of the
 // workgroup calls it (two barriers).
-template <int TM>
-__device__ __forceinline__ bool split_fixup(v16i (&hh)[2][2], v16i (&mid)[2][2], v16i (&ll)[2][2],
+template <int NW, int RB, int CB>
+__device__ __forceinline__ bool split_fixup(v16i (&hh)[RB][CB], v16i (&mid)[RB][CB], v16i (&ll)[RB][CB],
                                             int32_t* tile_part, uint32_t nz, uint32_t kz, uint32_t wave,
                                             uint32_t lane, uint32_t* cnt, uint32_t* ticket) {
-    constexpr uint32_t kBlock = TM * 128 * 4;                  // bytes of one slice's tile
+    constexpr uint32_t kWave = 4096 * RB * CB, kBlock = NW * kWave;   // bytes of one slice's wave, tile
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(tile_part, 0, (int)(nz * kBlock), 0x00020000);
-    const uint32_t wbase = wave * 16384 + lane * 16;
+    const uint32_t wbase = wave * kWave + lane * 16;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < CB; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++)
                 ll[i][j][r] = (int32_t)(((uint32_t)hh[i][j][r] << 16) + ((uint32_t)mid[i][j][r] << 8) +
                                         (uint32_t)ll[i][j][r]);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < CB; j++)
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const v4i v = {ll[i][j][4 * q], ll[i][j][4 * q + 1], ll[i][j][4 * q + 2], ll[i][j][4 * q + 3]};
-                __builtin_amdgcn_raw_buffer_store_b128(v, rs, kz * kBlock + wbase + (4 * (2 * i + j) + q) * 1024, 0, 16);
+                __builtin_amdgcn_raw_buffer_store_b128(v, rs, kz * kBlock + wbase + (4 * (CB * i + j) + q) * 1024, 0, 16);
             }
     __builtin_amdgcn_s_waitcnt(0x0070);      // this wave's partial stores complete
     __syncthreads();
@@ -732,21 +732,21 @@ __device__ __forceinline__ bool split_fixup(v16i (&hh)[2][2], v16i (&mid)[2][2],
     for (uint32_t z = 0; z < nz; z++) {
         if (z == kz) continue;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < RB; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < CB; j++)
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    const v4i v = __builtin_amdgcn_raw_buffer_load_b128(rs, z * kBlock + wbase + (4 * (2 * i + j) + q) * 1024, 0, 16);
+                    const v4i v = __builtin_amdgcn_raw_buffer_load_b128(rs, z * kBlock + wbase + (4 * (CB * i + j) + q) * 1024, 0, 16);
 #pragma unroll
                     for (int e = 0; e < 4; e++)
                         ll[i][j][4 * q + e] = (int32_t)((uint32_t)ll[i][j][4 * q + e] + (uint32_t)v[e]);
                 }
     }
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < CB; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int32_t tot = ll[i][j][r];
@@ -783,12 +783,29 @@ __device__ __forceinline__ void lds_copy16(const int8_t* g, int8_t* lds_wave_bas
     __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
 
+// The output tile of workgroup `x` of a slice.  Workgroups are dealt round-robin to the 8 XCDs, each
+// with its own L2: the ones of one residue mod 8 take a contiguous run of an order that walks
+// strips of `xw` tile columns row by row, so that a run is a block of about xw x xw tiles (xw is
+// near the square root of a run's length, gemm_strip) and an XCD reads each operand line once.
+// With whole columns as runs (every XCD reading all of A) BERT's 3072-row linears took 29.1 (768 x
+// 2304), 15.9 (768 x 768) and 50.2 us (3072 x 768, unsplit); with blocks 28.9, 14.0 and 44.4.
+struct TilePos {
+    uint32_t id, tr, tc;
+};
+__device__ __forceinline__ TilePos tile_pos(uint32_t x, uint32_t tiles_r, uint32_t tiles_c, uint32_t xw) {
+    const uint32_t ntiles = tiles_r * tiles_c, q = ntiles >> 3, res = x & 7;
+    const uint32_t p = res * q + min(res, ntiles & 7) + (x >> 3);
+    const uint32_t strip = p / (tiles_r * xw), in = p - strip * tiles_r * xw;
+    const uint32_t w = min(xw, tiles_c - strip * xw), row = in / w;
+    return TilePos{p, row, strip * xw + in - row * w};
+}
+
 template <int WR, int NST, class Epi>
-__global__ __launch_bounds__(128 * WR, WR == 1 ? 1 : 8 / (2 * WR)) void gemm_planes_kernel(
+__global__ __launch_bounds__(128 * WR, 8 / (2 * WR)) void gemm_planes_kernel(
     const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
     uint64_t a_slice, uint64_t rp_slice, uint32_t a_lines, const int8_t* __restrict__ Bhi,
     const int8_t* __restrict__ Blo, const int32_t* __restrict__ cpart, uint64_t b_slice, uint64_t cp_slice,
-    uint32_t b_lines, uint32_t nslab, uint32_t nsum_a, uint32_t tiles_r, uint32_t tiles_c, uint32_t kp, int32_t k64,
+    uint32_t b_lines, uint32_t nslab, uint32_t nsum_a, uint32_t tiles_r, uint32_t tiles_c, uint32_t xw, uint32_t kp, int32_t k64,
     uint32_t mode, int32_t* __restrict__ pout, uint32_t ksteps, uint32_t* __restrict__ tcnt, Epi epi) {
     constexpr int TM = 64 * WR;                  // tile rows
     constexpr int NT = 128 * WR;                 // threads
@@ -807,13 +824,8 @@ __global__ __launch_bounds__(128 * WR, WR == 1 ? 1 : 8 / (2 * WR)) void gemm_pla
     __shared__ int2 rterm[TM], cterm[BN];        // (h, l) halves
     __shared__ uint32_t ticket;                  // kSplitFix: the tile's arrival ticket
 
-    // XCD-aware tile order: workgroups are dispatched round-robin over the 8 XCDs, so
-    // give each XCD a contiguous range of tiles (column-major: tiles sharing a B column
-    // strip run on one XCD and share its L2).
-    const uint32_t ntiles = tiles_r * tiles_c;
-    uint32_t g = blockIdx.x;
-    if ((ntiles & 7) == 0) g = (g & 7) * (ntiles >> 3) + (g >> 3);
-    const uint32_t tr = g % tiles_r, tc = g / tiles_r;
+    const TilePos tp = tile_pos(blockIdx.x, tiles_r, tiles_c, xw);
+    const uint32_t tr = tp.tr, tc = tp.tc;
     const uint32_t bt = blockIdx.y, kz = blockIdx.z;
     const uint32_t kbeg = ksteps ? kz * ksteps : 0;
 
@@ -891,12 +903,9 @@ __global__ __launch_bounds__(128 * WR, WR == 1 ? 1 : 8 / (2 * WR)) void gemm_pla
             lds_copy16(bl_src + ((q) - 4 - BCP) * kp16 + k_, &SM[2 * A_T + B_T + b_dst + 1024 * ((q) - 4 - BCP)]); \
     }
     // The copies of slot s (after the s-th group of four MFMAs, 0..7): waves of copy group
-    // g issue theirs in slots 4g .. 4g + 3, two, two, then the rest; with 2 waves (12 copies)
-    // the one group issues two in each of slots 0 .. 5.
+    // g issue theirs in slots 4g .. 4g + 3, two, two, then the rest.
 #define CM_COPIES(SM, step, slot)                                                 \
     if (!cp_) {                                                                   \
-    } else if (NW == 2) {                                                         \
-        if ((slot) < 6) { CM_COPY(SM, step, 2 * (slot)) CM_COPY(SM, step, 2 * (slot) + 1) } \
     } else if (((slot) >> 2) == cgrp) {                                           \
         constexpr int s_ = (slot) & 3;                                            \
         if (s_ < 2) { CM_COPY(SM, step, 2 * s_) CM_COPY(SM, step, 2 * s_ + 1) }   \
@@ -987,19 +996,19 @@ __global__ __launch_bounds__(128 * WR, WR == 1 ? 1 : 8 / (2 * WR)) void gemm_pla
     const uint32_t row0 = tr * TM, col0 = tc * BN;
     if (mode == kSplitFix) {
         // the slices' partials meet in the last slice to arrive; the others are done
-        const uint64_t tile_id = (uint64_t)bt * ntiles + g;
-        if (!split_fixup<TM>(hh, mid, ll, pout + tile_id * gridDim.z * (TM * BN), gridDim.z, kz, wave, lane,
+        const uint64_t tile_id = (uint64_t)bt * tiles_r * tiles_c + tp.id;
+        if (!split_fixup<NW, 2, 2>(hh, mid, ll, pout + tile_id * gridDim.z * (TM * BN), gridDim.z, kz, wave, lane,
                              tcnt + tile_id, &ticket))
             return;
         mode = kWrap;
     }
-#define CM_STORE(M, P) store_wave_tile<M, P>(hh, mid, ll, rterm, cterm, bt, row0, col0, wr, wc, l32, lh, epi)
+#define CM_STORE(M, P) store_wave_tile<M, P, 2, 2>(hh, mid, ll, rterm, cterm, bt, row0, col0, wr, wc, l32, lh, epi)
     const TileBase tb = epi.tile_base(bt, row0, col0, TM, BN);
     if (tb.base != nullptr) {           // a whole tile: the lean store
-        if (mode == kWrap) store_wave_fast<kWrap>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi);
+        if (mode == kWrap) store_wave_fast<kWrap, 2, 2>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi);
         else if (mode == kSatNarrow)
-            store_wave_fast<kSatNarrow>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi);
-        else store_wave_fast<kSatWide>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi);
+            store_wave_fast<kSatNarrow, 2, 2>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi);
+        else store_wave_fast<kSatWide, 2, 2>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi);
     } else if (mode == kSatNarrow) {
         if (epi.pairs) CM_STORE(kSatNarrow, true); else CM_STORE(kSatNarrow, false);
     } else if (mode == kWrap) {
@@ -1007,6 +1016,251 @@ __global__ __launch_bounds__(128 * WR, WR == 1 ? 1 : 8 / (2 * WR)) void gemm_pla
     } else {
         if (epi.pairs) CM_STORE(kSatWide, true); else CM_STORE(kSatWide, false);
     }
+#undef CM_STORE
+}
+
+// ---------------------------------------------------------------- the plane GEMM, few tiles
+// The same product for outputs of few tiles (a 128-token layer, a prompt's projections, a
+// network's 7 x 7 and 14 x 14 planes), where the kernel above is bound by latency: its two-stage
+// ring gives a copy less than one k step to arrive, a wavefront's fragment reads stall its own
+// MFMAs, and its 128 x 128 tiles leave most compute units idle.  Here a workgroup of WR x WC
+// waves computes (32 RB WR) x (32 CB WC) outputs over a ring of NST stages:
+//   - copies run NST - 1 steps ahead, so that with few steps nearly all of k is in flight at once;
+//   - a wavefront reads the next step's fragments (both 32-k substeps) while its MFMAs of this step
+//     run, from a stage that landed one step earlier: one barrier a step, and no MFMA waits on LDS.
+// Stage, plane and swizzle layout as above; the 1 KiB copies of a stage (16 rows each: A hi, A lo,
+// B hi, B lo) are dealt to the waves in equal runs, each from its own uniform base address.
+template <int N>
+__device__ __forceinline__ void wait_copies() {            // at most N of this wave's copies outstanding, LDS reads done
+    static_assert(N >= 0 && N < 64, "vmcnt is six bits");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
+}
+
+// The copies (NC a step) of all but the newest `later` (at most MAX) steps have landed.
+template <int NC, int MAX>
+__device__ __forceinline__ void wait_steps(uint32_t later) {
+    if constexpr (MAX == 0) wait_copies<0>();
+    else if (later >= MAX) wait_copies<MAX * NC>();
+    else wait_steps<NC, MAX - 1>(later);
+}
+
+template <int RB, int CB, int WR, int WC, int NST, class Epi>
+__global__ __launch_bounds__(64 * WR * WC, 2) void gemm_ring_kernel(
+    const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
+    uint64_t a_slice, uint64_t rp_slice, uint32_t a_lines, const int8_t* __restrict__ Bhi,
+    const int8_t* __restrict__ Blo, const int32_t* __restrict__ cpart, uint64_t b_slice, uint64_t cp_slice,
+    uint32_t b_lines, uint32_t nslab, uint32_t nsum_a, uint32_t tiles_r, uint32_t tiles_c, uint32_t xw, uint32_t kp, int32_t k64,
+    uint32_t mode, int32_t* __restrict__ pout, uint32_t ksteps, uint32_t* __restrict__ tcnt, Epi epi) {
+    constexpr int TM = 32 * RB * WR, TN = 32 * CB * WC;
+    constexpr int NW = WR * WC, NT = 64 * NW;
+    constexpr int A_T = TM * BK, B_T = TN * BK;        // plane tile bytes
+    constexpr int STAGE = 2 * A_T + 2 * B_T;           // Ah, Al, Bh, Bl
+    constexpr int NC = STAGE / 1024 / NW;              // copies per wave and step
+    static_assert(STAGE % (1024 * NW) == 0, "equal copies per wave");
+    static_assert(NST >= 4 && NST <= 8 && (NST & 1) == 0, "an even ring (the fragment registers alternate)");
+    static_assert(NC * (NST - 1) < 64, "vmcnt is six bits");
+    // separate arrays: the compiler then tells the copies in flight from the fragment reads
+    __shared__ __attribute__((aligned(1024))) int8_t sm0[STAGE], sm1[STAGE], sm2[STAGE], sm3[STAGE];
+    __shared__ __attribute__((aligned(1024))) int8_t sm4[NST > 4 ? STAGE : 16], sm5[NST > 4 ? STAGE : 16];
+    __shared__ __attribute__((aligned(1024))) int8_t sm6[NST > 6 ? STAGE : 16], sm7[NST > 6 ? STAGE : 16];
+    __shared__ int2 rterm[TM], cterm[TN];              // (h, l) halves
+    __shared__ uint32_t ticket;                        // kSplitFix: the tile's arrival ticket
+
+    const TilePos tp = tile_pos(blockIdx.x, tiles_r, tiles_c, xw);
+    const uint32_t tr = tp.tr, tc = tp.tc;
+    const uint32_t bt = blockIdx.y, kz = blockIdx.z;
+    const uint32_t kbeg = ksteps ? kz * ksteps : 0;
+    const uint32_t nk = ksteps ? min(ksteps, kp / BK - kbeg) : kp / BK;
+
+    const uint32_t t = threadIdx.x, lane = t & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t wr = wave / WC, wc = wave % WC, l32 = lane & 31, lh = lane >> 5;
+
+    // copies: wave w takes the 16-row blocks NC w .. NC w + NC - 1 of a stage; lane l row l / 4,
+    // physical chunk l % 4 = logical chunk (l % 4) ^ swizzle
+    const uint32_t lrow = lane >> 2, cchunk = ((lane & 3) ^ ((lrow >> 2) & 3)) * 16;
+    const uint32_t voff = lrow * kp + cchunk;
+    const uint64_t a_base = bt * a_slice + (uint64_t)tr * TM * kp + (uint64_t)kbeg * BK;
+    const uint64_t b_base = bt * b_slice + (uint64_t)tc * TN * kp + (uint64_t)kbeg * BK;
+    const int8_t* src[NC];
+#pragma unroll
+    for (int q = 0; q < NC; q++) {
+        uint32_t blk = NC * wave + q;
+        if (blk < 2 * TM / 16) {
+            const bool low = blk >= TM / 16;
+            blk -= low ? TM / 16 : 0;
+            src[q] = (low ? Alo : Ahi) + a_base + (uint64_t)blk * 16 * kp;
+        } else {
+            blk -= 2 * TM / 16;
+            const bool low = blk >= TN / 16;
+            blk -= low ? TN / 16 : 0;
+            src[q] = (low ? Blo : Bhi) + b_base + (uint64_t)blk * 16 * kp;
+        }
+    }
+    auto issue = [&](int8_t* sm, uint32_t step) {
+#pragma unroll
+        for (int q = 0; q < NC; q++) lds_copy16(src[q] + (uint64_t)step * BK + voff, sm + (NC * wave + q) * 1024);
+    };
+    // the partial line sums: the first twelve of a line are loaded before the copies go out and used
+    // after them (a load issued behind the copies would be waited for behind them)
+    constexpr int TE = (TM + TN + NT - 1) / NT, TP = 12;
+    int32_t tpart[TE][TP];
+    auto term_src = [&](uint32_t e, uint32_t& stride, uint32_t& ns) -> const int32_t* {
+        const bool is_row = e < TM;
+        stride = is_row ? a_lines : b_lines;
+        ns = is_row ? nsum_a : nslab;
+        return is_row ? rpart + bt * rp_slice + tr * TM + e : cpart + bt * cp_slice + tc * TN + (e - TM);
+    };
+#pragma unroll
+    for (int q = 0; q < TE; q++) {
+        const uint32_t e = t + q * NT;
+        if (e >= TM + TN) continue;
+        uint32_t stride, ns;
+        const int32_t* pp = term_src(e, stride, ns);
+#pragma unroll
+        for (int i = 0; i < 4; i++) tpart[q][i] = pp[(uint64_t)min((uint32_t)i, ns - 1) * stride];
+        if (ns > 4) {
+#pragma unroll
+            for (int i = 4; i < TP; i++) tpart[q][i] = pp[(uint64_t)min((uint32_t)i, ns - 1) * stride];
+        }
+    }
+#define CM_ST(i) ((i) % NST == 0 ? sm0 : (i) % NST == 1 ? sm1 : (i) % NST == 2 ? sm2 : (i) % NST == 3 ? sm3 \
+                  : (i) % NST == 4 ? sm4 : (i) % NST == 5 ? sm5 : (i) % NST == 6 ? sm6 : sm7)
+    issue(sm0, 0);
+    if (1 < nk) issue(sm1, 1);
+    if (2 < nk) issue(sm2, 2);
+    if (NST > 4 && 3 < nk) issue(sm3, 3);
+    if (NST > 4 && 4 < nk) issue(sm4, 4);
+    if (NST > 6 && 5 < nk) issue(sm5, 5);
+    if (NST > 6 && 6 < nk) issue(sm6, 6);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < TE; q++) {
+        const uint32_t e = t + q * NT;
+        if (e >= TM + TN) continue;
+        uint32_t stride, ns;
+        const int32_t* pp = term_src(e, stride, ns);
+        int32_t sum = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum += (uint32_t)i < ns ? tpart[q][i] : 0;
+        if (ns > 4) {
+#pragma unroll
+            for (int i = 4; i < TP; i++) sum += (uint32_t)i < ns ? tpart[q][i] : 0;
+            for (uint32_t sl = TP; sl < ns; sl++) sum += pp[(uint64_t)sl * stride];
+        }
+        if (e < TM) rterm[e] = make_int2(epi.row_bias(tr * TM + e) - k64 + (sum >> 1), (sum & 1) << 7);
+        else cterm[e - TM] = make_int2(sum >> 1, (sum & 1) << 7);
+    }
+
+    const uint32_t sw = (l32 >> 2) & 3;
+    const uint32_t fa_row = (wr * (32 * RB) + l32) * BK, fb_row = (wc * (32 * CB) + l32) * BK;
+    const uint32_t ch[2] = {((0 + lh) ^ sw) * 16, ((2 + lh) ^ sw) * 16};
+    struct Frags { v4i ah[2][RB], al[2][RB], bh[2][CB], bl[2][CB]; };
+    auto read = [&](const int8_t* sm, Frags& f) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+#pragma unroll
+            for (int b = 0; b < RB; b++) {
+                f.ah[s][b] = *reinterpret_cast<const v4i*>(sm + fa_row + b * 32 * BK + ch[s]);
+                f.al[s][b] = *reinterpret_cast<const v4i*>(sm + A_T + fa_row + b * 32 * BK + ch[s]);
+            }
+#pragma unroll
+            for (int b = 0; b < CB; b++) {
+                f.bh[s][b] = *reinterpret_cast<const v4i*>(sm + 2 * A_T + fb_row + b * 32 * BK + ch[s]);
+                f.bl[s][b] = *reinterpret_cast<const v4i*>(sm + 2 * A_T + B_T + fb_row + b * 32 * BK + ch[s]);
+            }
+        }
+    };
+    v16i hh[RB][CB], mid[RB][CB], ll[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < CB; j++) hh[i][j] = mid[i][j] = ll[i][j] = v16i{};
+    auto mfma = [&](const Frags& f) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+#define CM_MFMAS(ACC, X, Y)                                                       \
+    _Pragma("unroll") for (int i = 0; i < RB; i++) _Pragma("unroll") for (int j = 0; j < CB; j++) \
+        ACC[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.X[s][i], f.Y[s][j], ACC[i][j], 0, 0, 0);
+            CM_MFMAS(hh, ah, bh)
+            CM_MFMAS(mid, ah, bl)
+            CM_MFMAS(ll, al, bl)
+            CM_MFMAS(mid, al, bh)
+#undef CM_MFMAS
+        }
+    };
+    // Every wave waits for its copies of step kt + 1 (those of up to NST - 3 later steps stay in
+    // flight) and its fragment reads of step kt, then for the other waves: stage kt + 1 is
+    // whole, and stage kt - 1, whose fragments every wave has consumed, takes step kt + NST - 1.
+    auto meet = [&](uint32_t kt) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        wait_steps<NC, NST - 3>(nk - 2 - kt);          // kt + 1 < nk
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+    };
+    Frags f0, f1;
+    {   // stage 0: the copies of at most NST - 2 later steps stay in flight
+        __builtin_amdgcn_sched_barrier(0);
+        wait_steps<NC, NST - 2>(nk - 1);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+    }
+    read(sm0, f0);
+    // (the wait for CUR stands outside the branch, where the compiler sees it on every path)
+#define CM_RSTEP(I, CUR, NXT)                                                     \
+    __builtin_amdgcn_s_waitcnt(0xC07F);                                           \
+    if (kt + 1 < nk) {                                                            \
+        meet(kt);                                                                 \
+        if (kt + NST - 1 < nk) issue(CM_ST((I) + NST - 1), kt + NST - 1);         \
+        read(CM_ST((I) + 1), NXT);                                                \
+    }                                                                             \
+    mfma(CUR);                                                                    \
+    if (++kt >= nk) break;
+    for (uint32_t kt = 0;;) {
+        CM_RSTEP(0, f0, f1)
+        CM_RSTEP(1, f1, f0)
+        CM_RSTEP(2, f0, f1)
+        CM_RSTEP(3, f1, f0)
+        if constexpr (NST > 4) {
+            CM_RSTEP(4, f0, f1)
+            CM_RSTEP(5, f1, f0)
+        }
+        if constexpr (NST > 6) {
+            CM_RSTEP(6, f0, f1)
+            CM_RSTEP(7, f1, f0)
+        }
+    }
+#undef CM_RSTEP
+#undef CM_ST
+
+    // ---- epilogue (every copy has landed: the last step waited for it)
+    const uint32_t row0 = tr * TM, col0 = tc * TN;
+    if (mode == kSplitFix) {
+        const uint64_t tile_id = (uint64_t)bt * tiles_r * tiles_c + tp.id;
+        if (!split_fixup<NW, RB, CB>(hh, mid, ll, pout + tile_id * gridDim.z * (TM * TN), gridDim.z, kz, wave, lane,
+                                     tcnt + tile_id, &ticket))
+            return;
+        mode = kWrap;
+    }
+#define CM_STORE(M, P) store_wave_tile<M, P, RB, CB>(hh, mid, ll, rterm, cterm, bt, row0, col0, wr, wc, l32, lh, epi)
+#define CM_STORE_FAST(M) \
+    store_wave_fast<M, RB, CB>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi)
+    const TileBase tb = epi.tile_base(bt, row0, col0, TM, TN);
+    if (tb.base != nullptr) {
+        if (mode == kWrap) CM_STORE_FAST(kWrap);
+        else if (mode == kSatNarrow) CM_STORE_FAST(kSatNarrow);
+        else CM_STORE_FAST(kSatWide);
+    } else if (mode == kSatNarrow) {
+        if (epi.pairs) CM_STORE(kSatNarrow, true); else CM_STORE(kSatNarrow, false);
+    } else if (mode == kWrap) {
+        if (epi.pairs) CM_STORE(kWrap, true); else CM_STORE(kWrap, false);
+    } else {
+        if (epi.pairs) CM_STORE(kSatWide, true); else CM_STORE(kSatWide, false);
+    }
+#undef CM_STORE_FAST
 #undef CM_STORE
 }
 
@@ -1892,13 +2146,20 @@ __global__ __launch_bounds__(64 * sp_max_waves(NB)) void skinny_mulact_kernel(co
 }
 
 // ---------------------------------------------------------------- drivers
+// The tile of a product: kernel variant, rows, columns and workgroups a compute unit holds.
+struct GemmPlan {
+    uint32_t id, tm, tn, per_cu;
+};
+constexpr GemmPlan kPlan128{0, 128, 128, 2}, kPlan256{1, 256, 128, 1};   // gemm_planes_kernel
+constexpr GemmPlan kRing64{2, 64, 64, 2}, kRing128{3, 128, 128, 1};      // gemm_ring_kernel
+
 // Byte planes [slices][lines_p][kp] of one operand and its partial line sums
 // [slices][nslab][lines_p].
 struct Planes {
     int8_t *hi, *lo;
     int32_t* part;
     uint32_t lines_p, kp, nslab, slices;
-    uint32_t tile = 128;                 // GEMM tile rows when this is the A operand
+    GemmPlan plan = kPlan128;            // the GEMM's tile when this is the A operand
     uint32_t rows = 0;                   // real lines (the rest up to lines_p are padding)
     uint32_t sums = 0;                   // partial line sums per line (0: one per slab)
     uint32_t nsum() const { return sums ? sums : nslab; }
@@ -1920,24 +2181,48 @@ int run_split(const Src& src, uint64_t src_slice, Planes& pl, hipStream_t s) {
     return CM_OK;
 }
 
-// Tile rows of the GEMM for an n x m output of `batch` slices.  A 256-row tile (8 waves, one
-// workgroup per compute unit) has the most operand reuse, but a grid of them that does not
-// fill the compute units in whole rounds leaves most of the last round idle; 128-row tiles
-// (two workgroups per unit) then finish sooner.  Outputs of at most 64 rows take 64-row tiles.
-uint32_t gemm_tile_rows(uint32_t n, uint32_t m, uint32_t batch, uint32_t cus) {
-    if (n <= 64) return 64;
-    if (n <= 128) return 128;
-    const uint64_t tiles = (uint64_t)ceil_div(n, 256) * ceil_div(m, BN) * batch;
-    return (tiles % cus == 0 || tiles >= 4ull * cus) ? 256 : 128;
+// k slices of a wrap-mode product of `tiles` tiles of a plan: as many as fill the workgroup slots
+// once, at least 12 k steps each (a slice's partials cost a round trip to the coherence point:
+// 128 x 3072 x 768 on 64 x 64 tiles takes 11.9 us in 2 slices, 9.7 in 4 (12 steps), 10.6 in 8).
+uint32_t gemm_slices(const GemmPlan& pl, uint64_t tiles, uint32_t nk, uint32_t cus) {
+    return (uint32_t)std::min<uint64_t>((uint64_t)cus * pl.per_cu / tiles, nk / 12);
+}
+
+// The tile of an n x m output of `batch` slices and nk k steps, where a product by the int32-wrap
+// rule (`wrap`) may be split over k; measured (us, k = 768 unless given):
+//   - 64 x 64 tiles on the four-stage ring while they fit the slots once (two workgroups a unit):
+//     128 x 2304 6.9 (128 x 128 tiles, two stages: 13.2), 1040 x 768 7.7 (15.2), 512 x 3072 10.0
+//     (13.6), 1536 x 768 of k 3072 24.5 (25.7 split in 3); and for outputs of at most 64 rows at any
+//     width: 24 x 100352 of k 192 18.9 (64 x 128 tiles, two stages: 23.6);
+//   - 128 x 128 tiles on the ring with 8 waves while they fit one to a unit: 1040 x 2304 15.1 (two
+//     stages 16.7), 576 x 6272 of k 128 8.0 (11.8), 3072 x 768 14.4 (14.3); but a wrap product that
+//     splits in 3 or more keeps the two-stage kernel, two workgroups a unit: 3072 x 768 of k 3072
+//     37.1 (ring unsplit 42.6), while 4992 x 768 of k 3072 takes 48.8 on the ring, 50.6 split in 2;
+//   - above, 256 x 128 tiles (one workgroup of 8 waves a unit, three stages) where their rounds
+//     over the units cost no more than the 128 x 128 tiles' (a round of them takes 22 - 25, of 128
+//     x 128 tiles 12.6 per tile a unit): 3072 x 2304 24.7 (26.7), 3072 x 3072 44.2 (37.8).
+GemmPlan gemm_plan(uint32_t n, uint32_t m, uint32_t batch, uint32_t nk, bool wrap, uint32_t cus) {
+    auto tiles = [&](const GemmPlan& pl) { return (uint64_t)ceil_div(n, pl.tm) * ceil_div(m, pl.tn) * batch; };
+    if (n <= 64 || tiles(kRing64) <= 2ull * cus) return kRing64;
+    const uint64_t t128 = tiles(kPlan128);
+    if (t128 <= cus) return wrap && gemm_slices(kPlan128, t128, nk, cus) >= 3 ? kPlan128 : kRing128;
+    return 2 * ((tiles(kPlan256) + cus - 1) / cus) <= (t128 + cus - 1) / cus ? kPlan256 : kPlan128;
+}
+
+// Tile columns of the strips tile_pos walks: the square root of an XCD's share of the tiles.
+uint32_t gemm_strip(uint32_t tiles, uint32_t tiles_c) {
+    uint32_t w = 1;
+    while ((w + 1) * (w + 1) * 8 <= tiles) w++;
+    return std::min(w, tiles_c);
 }
 
 template <class Epi>
 int run_gemm(const Planes& A, const Planes& B, uint32_t batch, uint32_t k, Epi epi, hipStream_t s,
              int32_t* pout = nullptr, uint32_t ksteps = 0, uint32_t* tcnt = nullptr) {
-    const uint32_t tm = A.tile;
-    const uint32_t tiles_r = ceil_div(A.rows, tm), tiles_c = B.lines_p / BN;
-    if (tm != 64 && tm != 128 && tm != 256) return fail(CM_EINVAL, "gemm: tile rows %u", tm);
-    if ((uint64_t)tiles_r * tm > A.lines_p) return fail(CM_EINVAL, "gemm: %u tile rows past %u plane rows", tm, A.lines_p);
+    const GemmPlan pl = A.plan;
+    const uint32_t tiles_r = ceil_div(A.rows, pl.tm), tiles_c = ceil_div(B.rows, pl.tn);
+    if ((uint64_t)tiles_r * pl.tm > A.lines_p || (uint64_t)tiles_c * pl.tn > B.lines_p)
+        return fail(CM_EINVAL, "gemm: %u x %u tiles past %u x %u plane lines", tiles_r, tiles_c, A.lines_p, B.lines_p);
     const uint64_t a_slice = A.slices > 1 ? (uint64_t)A.lines_p * A.kp : 0;
     const uint64_t b_slice = B.slices > 1 ? (uint64_t)B.lines_p * B.kp : 0;
     const uint64_t rp_slice = A.slices > 1 ? (uint64_t)A.nslab * A.lines_p : 0;
@@ -1945,31 +2230,26 @@ int run_gemm(const Planes& A, const Planes& B, uint32_t batch, uint32_t k, Epi e
     if (ksteps && tcnt == nullptr) return fail(CM_EINVAL, "gemm: a split over k needs the arrival counts");
     const uint32_t mode = ksteps ? kSplitFix : (epi.wrap ? kWrap : (k <= 8192 ? kSatNarrow : kSatWide));
     const uint32_t nz = ksteps ? ceil_div(A.kp / BK, ksteps) : 1;
+    const uint32_t xw = gemm_strip(tiles_r * tiles_c, tiles_c);
     const dim3 grid(tiles_r * tiles_c, batch, nz);
-    if (tm == 256) {
-        CM_LAUNCH("gemm_planes_kernel", (gemm_planes_kernel<4, 3, Epi>), grid, dim3(512), 0, s, A.hi, A.lo, A.part,
-                  a_slice, rp_slice, A.lines_p, B.hi, B.lo, B.part, b_slice, cp_slice, B.lines_p, B.nslab, A.nsum(),
-                  tiles_r, tiles_c, A.kp, (int32_t)(64 * k), mode, pout, ksteps, tcnt, epi);
-    } else if (tm == 64) {
-        CM_LAUNCH("gemm_planes_kernel", (gemm_planes_kernel<1, 2, Epi>), grid, dim3(128), 0, s, A.hi, A.lo, A.part,
-                  a_slice, rp_slice, A.lines_p, B.hi, B.lo, B.part, b_slice, cp_slice, B.lines_p, B.nslab, A.nsum(),
-                  tiles_r, tiles_c, A.kp, (int32_t)(64 * k), mode, pout, ksteps, tcnt, epi);
-    } else {
-        CM_LAUNCH("gemm_planes_kernel", (gemm_planes_kernel<2, 2, Epi>), grid, dim3(256), 0, s, A.hi, A.lo, A.part,
-                  a_slice, rp_slice, A.lines_p, B.hi, B.lo, B.part, b_slice, cp_slice, B.lines_p, B.nslab, A.nsum(),
-                  tiles_r, tiles_c, A.kp, (int32_t)(64 * k), mode, pout, ksteps, tcnt, epi);
+#define CM_GEMM(NT, ...)                                                                                             \
+    CM_LAUNCH("gemm_planes_kernel", (__VA_ARGS__), grid, dim3(NT), 0, s, A.hi, A.lo, A.part, a_slice, rp_slice,       \
+              A.lines_p, B.hi, B.lo, B.part, b_slice, cp_slice, B.lines_p, B.nslab, A.nsum(), tiles_r, tiles_c, xw,   \
+              A.kp, (int32_t)(64 * k), mode, pout, ksteps, tcnt, epi)
+    switch (pl.id) {
+    case kPlan256.id: CM_GEMM(512, gemm_planes_kernel<4, 3, Epi>); break;
+    case kRing64.id: CM_GEMM(256, gemm_ring_kernel<1, 1, 2, 2, 4, Epi>); break;
+    case kRing128.id: CM_GEMM(512, gemm_ring_kernel<1, 2, 4, 2, 4, Epi>); break;
+    default: CM_GEMM(256, gemm_planes_kernel<2, 2, Epi>); break;
     }
+#undef CM_GEMM
     return CM_OK;
 }
 
-// k steps per slice for a wrap-mode matmul whose output tiles leave most workgroup slots
-// idle (0: no split): slices until the grid about fills the slots, at least 4 steps each.
-uint32_t gemm_ksteps(uint32_t tm, uint32_t tiles, uint32_t kp, const DeviceState* st) {
-    const uint32_t slots = st->cus * (tm == 256 ? 1u : 2u), nk = kp / BK;
-    if (tiles * 2 > slots || nk < 16) return 0;
-    const uint32_t nz = std::min(slots / tiles, nk / 4);
-    if (nz < 2) return 0;
-    return ceil_div(nk, nz);
+// k steps per slice of a wrap-mode product (0: no split).
+uint32_t gemm_ksteps(const GemmPlan& pl, uint32_t tiles, uint32_t kp, const DeviceState* st) {
+    const uint32_t nk = kp / BK, nz = gemm_slices(pl, tiles, nk, st->cus);
+    return nz < 2 ? 0 : ceil_div(nk, nz);
 }
 
 Planes make_planes(uint32_t lines, uint32_t kp, uint32_t slices, uint32_t align = 128) {
@@ -1979,7 +2259,13 @@ Planes make_planes(uint32_t lines, uint32_t kp, uint32_t slices, uint32_t align 
     p.kp = kp;
     p.nslab = ceil_div(kp, SLAB);
     p.slices = slices;
-    p.tile = align;
+    return p;
+}
+
+// A's planes for a product by `plan`.
+Planes make_a_planes(uint32_t lines, uint32_t kp, uint32_t slices, const GemmPlan& plan) {
+    Planes p = make_planes(lines, kp, slices, plan.tm);
+    p.plan = plan;
     return p;
 }
 
@@ -2101,10 +2387,10 @@ int skinny_wrap(const int16_t* a, const int16_t* b, int16_t* c, uint32_t n, uint
 // bytes of its int32 partials.
 uint32_t matmul_ksteps(const Planes& A, const Planes& B, uint32_t n, uint32_t m, uint32_t batch, uint32_t wrap32,
                        const DeviceState* st, size_t* bytes) {
-    const uint32_t tiles = ceil_div(n, A.tile) * (B.lines_p / BN) * batch;
-    const uint32_t ks = wrap32 ? gemm_ksteps(A.tile, tiles, A.kp, st) : 0;
+    const uint32_t tiles = ceil_div(n, A.plan.tm) * ceil_div(m, A.plan.tn) * batch;
+    const uint32_t ks = wrap32 ? gemm_ksteps(A.plan, tiles, A.kp, st) : 0;
     // the partials of every slice, whole tiles (split_fixup's layout)
-    *bytes = ks ? (size_t)ceil_div(A.kp / BK, ks) * tiles * A.tile * BN * 4 : 0;
+    *bytes = ks ? (size_t)ceil_div(A.kp / BK, ks) * tiles * A.plan.tm * A.plan.tn * 4 : 0;
     return ks;
 }
 
@@ -2115,7 +2401,7 @@ int gemm_out(const Planes& A, const Planes& B, int16_t* c, uint32_t n, uint32_t 
     EpiMatmul epi{c, (uint64_t)c_bs, n, m, wrap32 ? 1u : 0u, pairs ? 1u : 0u};
     // a split product is finished by the last slice of each tile (one launch): an arrival
     // count per tile (a split has at most one tile per compute unit, gemm_ksteps)
-    const uint64_t tiles = (uint64_t)ceil_div(A.rows, A.tile) * (B.lines_p / BN) * batch;
+    const uint64_t tiles = (uint64_t)ceil_div(A.rows, A.plan.tm) * ceil_div(m, A.plan.tn) * batch;
     if (ksteps && tiles > st->split_cnt_n)
         return fail(CM_EINVAL, "gemm: %llu split tiles past the %u arrival counts", (unsigned long long)tiles,
                     st->split_cnt_n);
@@ -2142,9 +2428,15 @@ int matmul_run(const int16_t* a, const int16_t* b, int16_t* c, uint32_t n, uint3
         return skinny_wrap(a, b, c, n, k, m, batch, a_bs, b_bs, c_bs, b_packed, st, s, fixed);
     const uint32_t kp = (uint32_t)round_up(k, BK);
     const uint32_t sa = (batch > 1 && a_bs != 0) ? batch : 1, sb = (batch > 1 && b_bs != 0) ? batch : 1;
-    Planes A = make_planes(n, kp, sa, gemm_tile_rows(n, m, batch, st->cus)), B = make_planes(m, kp, sb);
+    Planes A = make_a_planes(n, kp, sa, gemm_plan(n, m, batch, kp / BK, wrap32, st->cus)), B = make_planes(m, kp, sb);
     size_t pbytes;
-    const uint32_t ksteps = matmul_ksteps(A, B, n, m, batch, wrap32, st, &pbytes);
+    uint32_t ksteps = matmul_ksteps(A, B, n, m, batch, wrap32, st, &pbytes);
+    if (fixed != nullptr && A.bytes() + B.bytes() + pbytes > fixed->cap) {
+        // the least a product needs: rows rounded up to 64, no partials
+        A = make_a_planes(n, kp, sa, kRing64);
+        ksteps = 0;
+        pbytes = 0;
+    }
     void* ws;
     rc = take_workspace(st, fixed, A.bytes() + B.bytes() + pbytes, &ws, s);
     if (rc) return rc;
@@ -2253,7 +2545,7 @@ extern "C" int cm_matmul_planes(const int16_t* a, const void* b_planes, int16_t*
     hipStream_t s = as_stream(stream);
     const uint32_t kp = (uint32_t)round_up(k, BK);
     const uint32_t sa = (batch > 1 && a_bs != 0) ? batch : 1;
-    Planes A = make_planes(n, kp, sa, gemm_tile_rows(n, m, batch, st->cus)), B = make_planes(m, kp, b_slices);
+    Planes A = make_a_planes(n, kp, sa, gemm_plan(n, m, batch, kp / BK, wrap32, st->cus)), B = make_planes(m, kp, b_slices);
     size_t pbytes;
     const uint32_t ksteps = matmul_ksteps(A, B, n, m, batch, wrap32, st, &pbytes);
     void* ws;
@@ -2286,7 +2578,7 @@ extern "C" int cm_matmul_aplanes(const void* a_planes, uint32_t nsum, const void
         return fail(CM_EALIGN, "matmul: planes not 256-byte aligned");
     hipStream_t s = as_stream(stream);
     const APlanes ap = a_planes_view(const_cast<void*>(a_planes), n, k, nsum);
-    Planes A = make_planes(n, k, 1, gemm_tile_rows(n, m, 1, st->cus)), B = make_planes(m, k, 1);
+    Planes A = make_a_planes(n, k, 1, gemm_plan(n, m, 1, k / BK, wrap32, st->cus)), B = make_planes(m, k, 1);
     A.hi = ap.hi;
     A.lo = ap.lo;
     A.part = ap.part;
@@ -2328,8 +2620,8 @@ Planes conv_b_planes(const ConvGeom& g, uint32_t kp) {
     return g.fold() ? make_planes(g.batch * g.plane(), kp, 1) : make_planes(g.plane(), kp, g.batch);
 }
 
-uint32_t conv_tile(const ConvGeom& g, const Planes& B, const DeviceState* st) {
-    return gemm_tile_rows(g.out_ch, B.rows, B.slices, st->cus);
+GemmPlan conv_plan(const ConvGeom& g, const Planes& B, const DeviceState* st) {
+    return gemm_plan(g.out_ch, B.rows, B.slices, B.kp / BK, false, st->cus);
 }
 
 // The weights' planes: rows = output channels in the packed tile-major order (ConvKernel.h:136-159).
@@ -2500,7 +2792,7 @@ int conv_run(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y
                      dilation_w, pad_top, pad_left, cs, y_cn, y_gs, wrap32 ? 1u : 0u};
     const uint32_t kp = conv_kp(in_ch, kh, kw);
     Planes B = conv_b_planes(g, kp);
-    Planes A = make_planes(out_ch, kp, 1, conv_tile(g, B, st));
+    Planes A = make_a_planes(out_ch, kp, 1, conv_plan(g, B, st));
     void* ws;
     rc = workspace(st, A.bytes() + B.bytes(), &ws, s);
     if (rc) return rc;
@@ -2594,7 +2886,7 @@ int conv_planes_run(const int16_t* x, const void* w_planes, const int16_t* bias,
     Planes A = make_planes(out_ch, kp, 1, 256);
     char* q = static_cast<char*>(const_cast<void*>(w_planes));
     A.carve(q);
-    A.tile = conv_tile(g, B, st);
+    A.plan = conv_plan(g, B, st);
     void* ws;
     rc = workspace(st, B.bytes(), &ws, s);
     if (rc) return rc;
@@ -2646,7 +2938,7 @@ extern "C" int cm_matmul_strided(const int16_t* a, const int16_t* b, int16_t* c,
     if (lda < k || ldb < (b_trans ? k : m) || ldc < m) return fail(CM_EINVAL, "matmul: row strides below the rows");
     hipStream_t s = as_stream(stream);
     const uint32_t kp = (uint32_t)round_up(k, BK);
-    Planes A = make_planes(n, kp, batch, gemm_tile_rows(n, m, batch, st->cus)), B = make_planes(m, kp, batch);
+    Planes A = make_a_planes(n, kp, batch, gemm_plan(n, m, batch, kp / BK, false, st->cus)), B = make_planes(m, kp, batch);
     void* ws;
     rc = workspace(st, A.bytes() + B.bytes(), &ws, s);
     if (rc) return rc;
