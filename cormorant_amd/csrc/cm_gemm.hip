@@ -49,15 +49,8 @@ __device__ __forceinline__ uint32_t pack_lo(const int16_t* v) {   // 4 low bytes
 }
 
 // ---------------------------------------------------------------- operand sources
-// A side: rows of the output (matmul rows of A; conv output channels = weights).
-struct SrcRowMajor {             // A[i][kk] = a[i * lda + kk]
-    const int16_t* p;
-    uint32_t rows, k;
-    uint64_t lda;
-    __device__ bool real(uint32_t i, uint32_t kk) const { return i < rows && kk < k; }
-    __device__ int16_t at(uint32_t i, uint32_t kk) const { return p[i * lda + kk]; }
-};
-// B side: columns of the output; B(kk, j) for the three matmul images.
+// B side: columns of the output; B(kk, j) of the matmul images (the GEMV image of more than one
+// column group; the others have their own kernels).
 struct SrcMatB {
     const int16_t* p;
     uint32_t cols, k, m, layout, kw;   // layout 0 row-major, 1 packed, 2 gemv, 3 transposed [m][k]
@@ -88,27 +81,16 @@ struct SrcConvW {
     }
 };
 // im2col of one NCHW image as GEMM columns: column p = oh * out_w + ow.
-struct SrcIm2col {
+struct Im2col {
     const int16_t* p;
+    uint64_t img;                    // elements per image
     uint32_t in_ch, in_h, in_w, out_w, kh, kw, sh, sw, dh, dw, pt, pl, cols;
-    __device__ bool real(uint32_t col, uint32_t kk) const {
-        uint32_t lane = kk & 15, ict = (kk >> 4) / (kh * kw);
-        return col < cols && ict * 16 + lane < in_ch;
-    }
-    __device__ int16_t at(uint32_t col, uint32_t kk) const {
-        uint32_t lane = kk & 15, t = kk >> 4, ict = t / (kh * kw), pos = t - ict * kh * kw;
-        uint32_t khi = pos / kw, kwi = pos - khi * kw, ic = ict * 16 + lane;
-        uint32_t oh = col / out_w, ow = col - oh * out_w;
-        int ih = (int)(oh * sh + khi * dh) - (int)pt, iw = (int)(ow * sw + kwi * dw) - (int)pl;
-        if (ih < 0 || ih >= (int)in_h || iw < 0 || iw >= (int)in_w) return 0;
-        return p[((uint64_t)ic * in_h + ih) * in_w + iw];
-    }
 };
 
 // Split one operand into byte planes [lines][kp] (lines = rows for A, columns for B) and
 // partial line sums per SLAB of k.  Workgroup: 64 lines x one SLAB; the 64x64 element tiles
-// pass through LDS so that the reads follow the source's fast dimension (`KFast`: k for a
-// row-major A; the line index for B images and im2col).
+// pass through LDS so that the reads follow the source's fast dimension (`KFast`: k for conv
+// weights; the line index for B images).
 template <class Src, bool KFast>
 __global__ __launch_bounds__(256) void split_kernel(Src src, uint64_t src_slice, int8_t* __restrict__ hi,
                                                     int8_t* __restrict__ lo, int32_t* __restrict__ part,
@@ -163,9 +145,18 @@ __global__ __launch_bounds__(256) void split_kernel(Src src, uint64_t src_slice,
 // Padding is written as the value 128 (A' = 0: the byte pair (0, 0)) and left out of the sums.
 constexpr int16_t kPad = 128;
 
-// Rows with k contiguous (the matmul A, row stride lda, 16-byte aligned rows): one wavefront
+// 8 elements at any element alignment (one 16-byte load: global loads need no more than 2 bytes).
+__device__ __forceinline__ int4 load8(const int16_t* p) {
+    int4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
+// Rows with k contiguous (the matmul A, row stride lda, rows at any alignment): one wavefront
 // per row and SLAB of k, 8 k per lane per 16-byte load, the slab's loads all in flight
-// before the first is used; grid (ceil(lines_p / 4), nslab, slices).
+// before the first is used; only the lane at the end of a row loads single elements.  Rows of 771
+// (3000 of them) took 59 us through the general kernel's 2-byte loads, 8.5 here.
+// Grid (ceil(lines_p / 4), nslab, slices).
 __global__ __launch_bounds__(256) void split_rows_kernel(const int16_t* __restrict__ src, Slices slice,
                                                          uint64_t lda, uint32_t rows, uint32_t k,
                                                          int8_t* __restrict__ hi, int8_t* __restrict__ lo,
@@ -181,11 +172,15 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const int16_t* __restri
     int4 v[U];
     if (real_row && (slab + 1) * SLAB <= k) {          // the whole slab is real: no branches
 #pragma unroll
-        for (int u = 0; u < U; u++) v[u] = *reinterpret_cast<const int4*>(r + slab * SLAB + 512 * u + 8 * lane);
+        for (int u = 0; u < U; u++) v[u] = load8(r + slab * SLAB + 512 * u + 8 * lane);
     } else {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const uint32_t k0 = slab * SLAB + 512 * u + 8 * lane;
+            if (real_row && k0 + 8 <= k) {
+                v[u] = load8(r + k0);
+                continue;
+            }
             int16_t e[8];
 #pragma unroll
             for (int q = 0; q < 8; q++) e[q] = (real_row && k0 + q < k) ? r[k0 + q] : kPad;
@@ -234,7 +229,7 @@ __global__ __launch_bounds__(256) void split_rows_short_kernel(const int16_t* __
     if (in) {
         const int16_t* r = src + slice.off(bt) + (uint64_t)row * lda;
         if (real_row && k0 + 8 <= k) {
-            v = *reinterpret_cast<const int4*>(r + k0);
+            v = load8(r + k0);
             sum = sum8(v);
         } else {
             int16_t e[8];
@@ -258,8 +253,8 @@ __global__ __launch_bounds__(256) void split_rows_short_kernel(const int16_t* __
     if (g == 0) part[(uint64_t)bt * lines_p + row] = sum;
 }
 
-// Columns of a k-major image (row-major B [k][m] with m % 8 == 0, or the packed 32-column
-// tiles).  A wavefront takes 32 columns and 256 k of one SLAB: lane = (r4, c8) with
+// Columns of a k-major image (row-major B [k][m] at any width and alignment, or the packed
+// 32-column tiles; 771 x 1235 71 us through the general kernel, 11 here).  A wavefront takes 32 columns and 256 k of one SLAB: lane = (r4, c8) with
 // r4 = lane / 4 picking 4 consecutive k of each 64-k group and c8 = lane % 4 picking 8
 // columns, so one load instruction reads 16 rows x 64 contiguous bytes.  Each lane loads
 // its 4 groups x 4 rows x 8 columns at once, then transposes every 4 x 8 block in registers
@@ -290,7 +285,37 @@ __global__ __launch_bounds__(256) void split_cols_kernel(const int16_t* __restri
 #pragma unroll
         for (int g = 0; g < 4; g++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[g][r] = *reinterpret_cast<const int4*>(p0 + (64 * g + r) * rs);
+            for (int r = 0; r < 4; r++) v[g][r] = load8(p0 + (64 * g + r) * rs);
+    } else if (cols_real || packed || m >= 8) {
+        // whole loads for the real k rows.  The lane at the last columns: a packed tile holds all its
+        // 32 columns, and the ones past m become padding; of row-major rows it loads the last 8 and
+        // shifts out the ones its left neighbour holds.  The lanes past m hold padding alone.
+        const uint32_t nv = cols_real ? 8 : (j0 < m ? m - j0 : 0);           // real columns
+        const uint32_t jl = cols_real || packed ? j0 : m - 8;
+        const int4 pad = make_int4(0x00800080, 0x00800080, 0x00800080, 0x00800080);
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const uint32_t kk = kq + 64 * g + 4 * r4 + r;
+                v[g][r] = pad;
+                if (kk < k && nv) v[g][r] = load8(b + at(kk, jl));
+            }
+        if (nv && nv < 8) {
+            const unsigned __int128 mask = ((unsigned __int128)1 << (16 * nv)) - 1;
+            const uint32_t sh = packed ? 0 : 16 * (8 - nv);
+            unsigned __int128 fill;
+            __builtin_memcpy(&fill, &pad, 16);
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    unsigned __int128 w;
+                    __builtin_memcpy(&w, &v[g][r], 16);
+                    w = ((w >> sh) & mask) | (fill & ~mask);
+                    if (kq + 64 * g + 4 * r4 + r < k) __builtin_memcpy(&v[g][r], &w, 16);
+                }
+        }
     } else {
 #pragma unroll
         for (int g = 0; g < 4; g++)
@@ -454,7 +479,65 @@ __global__ __launch_bounds__(1024) void split_fold16_kernel(const int16_t* __res
     }
 }
 
-// The same operand for planes with many lines: a workgroup takes 64 lines and one SLAB of
+// im2col planes of NCHW images, k in the packed weight order (16-channel tiles x kernel positions):
+// as split_fold16_kernel, 16 columns (output pixels) a workgroup, wave w the slab's 64 k from 64 w;
+// lane (column l % 16, chunk l / 16) loads its pixel's 16 channels at the chunk's kernel position
+// (16 loads in flight, one address and one bounds test a chunk) and writes 16 bytes a plane, the
+// four chunk lanes of a column 64 contiguous bytes.  Bound by the planes' bytes: 8 images of 64
+// channels at 56 x 56, 3 x 3 (29 MB of planes) took 67 us with a division and bounds
+// tests per element, 12.8 here.  Grid (lines_p / 16, nslab, images).
+__global__ __launch_bounds__(1024) void split_im2col_kernel(Im2col g, int8_t* __restrict__ hi,
+                                                            int8_t* __restrict__ lo, int32_t* __restrict__ part,
+                                                            uint32_t lines_p, uint32_t kp, uint32_t nslab) {
+    __shared__ int32_t wsum[16][16];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const uint32_t ln = lane & 15, ch = lane >> 4;
+    const uint32_t j = blockIdx.x * 16 + ln, slab = blockIdx.y, bt = blockIdx.z;
+    const uint32_t k0 = slab * SLAB + 64 * wave + 16 * ch;
+    int32_t sum = 0;
+    if (k0 < kp) {
+        const uint32_t t = k0 >> 4, khw = g.kh * g.kw, ict = t / khw, pos = t - ict * khw;
+        const uint32_t khi = pos / g.kw, kwi = pos - khi * g.kw, c0 = ict * 16;
+        const uint32_t oh = j / g.out_w, ow = j - oh * g.out_w;
+        const int64_t ih = (int64_t)oh * g.sh + (int64_t)khi * g.dh - g.pt;
+        const int64_t iw = (int64_t)ow * g.sw + (int64_t)kwi * g.dw - g.pl;
+        const bool inside = ih >= 0 && ih < (int64_t)g.in_h && iw >= 0 && iw < (int64_t)g.in_w;
+        const uint32_t nc = j < g.cols && c0 < g.in_ch ? min(g.in_ch - c0, 16u) : 0;     // real channels
+        const uint64_t plane = (uint64_t)g.in_h * g.in_w;
+        const int16_t* src = g.p + bt * g.img + (inside ? c0 * plane + (uint64_t)ih * g.in_w + (uint64_t)iw : 0);
+        int16_t e[16];
+        if (nc == 16 && inside) {
+#pragma unroll
+            for (int q = 0; q < 16; q++) e[q] = src[q * plane];
+#pragma unroll
+            for (int q = 0; q < 16; q++) sum += e[q];
+        } else {
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const bool r = (uint32_t)q < nc;
+                e[q] = r ? (inside ? src[q * plane] : (int16_t)0) : kPad;
+                sum += r ? e[q] : 0;
+            }
+        }
+        uint2 h0, l0, h1, l1;
+        split8(*reinterpret_cast<const int4*>(e), h0, l0);
+        split8(*reinterpret_cast<const int4*>(e + 8), h1, l1);
+        const uint64_t off = ((uint64_t)bt * lines_p + j) * kp + k0;
+        *reinterpret_cast<uint4*>(hi + off) = make_uint4(h0.x, h0.y, h1.x, h1.y);
+        *reinterpret_cast<uint4*>(lo + off) = make_uint4(l0.x, l0.y, l1.x, l1.y);
+    }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (ch == 0) wsum[wave][ln] = sum;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        int32_t t = 0;
+        for (uint32_t w = 0; w < waves; w++) t += wsum[w][threadIdx.x];
+        part[((uint64_t)bt * nslab + slab) * lines_p + blockIdx.x * 16 + threadIdx.x] = t;
+    }
+}
+
+// The folded operand for planes with many lines: a workgroup takes 64 lines and one SLAB of
 // k in 64 x 64 tiles through LDS.  Thread t loads line t % 64 at 16 k (2-byte loads, the 64
 // lanes of one load on consecutive lines), then packs 16 consecutive k of line t / 4 into
 // 16-byte words: the four threads of a line write 64 contiguous bytes of each plane.
@@ -2287,8 +2370,7 @@ int matmul_check(uint32_t k, uint32_t gemv_kw, int64_t a_bs, int64_t b_bs, int64
     return CM_OK;
 }
 
-// Planes of rows with k contiguous (lda elements apart, 16-byte aligned): the short-row
-// kernel for kp <= 256, else a wavefront per row and slab.
+// Planes of rows with k contiguous (lda elements apart): the short-row kernel for kp <= 256, else a wavefront per row and slab.
 int split_row_lines(const int16_t* a, Slices a_slice, uint64_t lda, uint32_t n, uint32_t k, Planes& P,
                     hipStream_t s) {
     if (P.kp <= 256) {
@@ -2306,19 +2388,16 @@ int split_row_lines(const int16_t* a, Slices a_slice, uint64_t lda, uint32_t n, 
 
 // A's planes: row-major [n][k] slices at a_slice elements (0: one slice).
 int split_a(const int16_t* a, uint64_t a_slice, uint32_t n, uint32_t k, Planes& A, hipStream_t s) {
-    if (aligned16(a) && (k & 7) == 0 && (a_slice & 7) == 0) return split_row_lines(a, Slices{a_slice}, k, n, k, A, s);
-    return run_split<SrcRowMajor, true>(SrcRowMajor{a, n, k, k}, a_slice, A, s);
+    return split_row_lines(a, Slices{a_slice}, k, n, k, A, s);
 }
 
 // B's planes from its image (row-major, packed 32-column tiles or the GEMV image).
 int split_b(const int16_t* b, uint64_t b_slice, uint32_t k, uint32_t m, uint32_t b_packed, uint32_t gemv_kw,
             Planes& B, hipStream_t s) {
     const uint32_t layout = gemv_kw ? 2 : (b_packed == 2 ? 3 : (b_packed ? 1 : 0));
-    if (layout == 3 && aligned16(b) && (b_slice & 7) == 0 && (k & 7) == 0)
+    if (layout == 3)
         return split_row_lines(b, Slices{b_slice}, k, m, k, B, s);    // B's lines are rows with k contiguous
-    const bool fast_b = aligned16(b) && (b_slice & 7) == 0 &&
-                        (layout == 1 || (layout == 0 && (m & 7) == 0) || (layout == 2 && gemv_kw == 1 && (m & 7) == 0));
-    if (fast_b) {
+    if (layout <= 1 || (layout == 2 && gemv_kw == 1)) {
         CM_LAUNCH("split_cols_kernel", split_cols_kernel, dim3(B.lines_p / 32, B.nslab, B.slices), dim3(256), 0, s,
                   b, Slices{b_slice}, (uint64_t)m, layout == 1 ? 1u : 0u, m, k, B.hi, B.lo, B.part, B.lines_p, B.kp,
                   B.nslab);
@@ -2659,9 +2738,11 @@ int conv_gemm(const int16_t* x, const Planes& A, Planes& B, const int16_t* bptr,
         EpiConv epi{y, bptr, img, g.out_ch, cols, plane, 0, 0, g.wrap, pairs ? 1u : 0u, plane, lo, hi};
         return run_gemm(A, B, 1, g.in_ch * g.kh * g.kw, epi, s);
     }
-    SrcIm2col im{x, g.in_ch, g.in_h, g.in_w, g.out_w, g.kh, g.kw, g.sh, g.sw, g.dh, g.dw, g.pt, g.pl, plane};
-    int rc = run_split<SrcIm2col, false>(im, (uint64_t)g.in_ch * g.in_h * g.in_w, B, s);
-    if (rc) return rc;
+    const Im2col im{x, (uint64_t)g.in_ch * g.in_h * g.in_w, g.in_ch, g.in_h, g.in_w, g.out_w, g.kh, g.kw, g.sh, g.sw,
+                    g.dh, g.dw, g.pt, g.pl, plane};
+    const uint32_t waves = std::min<uint32_t>(16, ceil_div(std::min<uint32_t>(B.kp, SLAB), 64));
+    CM_LAUNCH("split_kernel", split_im2col_kernel, dim3(B.lines_p / 16, B.nslab, B.slices), dim3(64 * waves), 0, s, im,
+              B.hi, B.lo, B.part, B.lines_p, B.kp, B.nslab);
     const bool pairs = (reinterpret_cast<uintptr_t>(y) & 3) == 0 && (plane & 1) == 0 && (g.cs & 1) == 0 &&
                        (g.gs & 1) == 0 && (img & 1) == 0;
     EpiConv epi{y, bptr, img, g.out_ch, plane, g.cs, g.cn, g.gs, g.wrap, pairs ? 1u : 0u, 0, lo, hi};
