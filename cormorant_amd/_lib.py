@@ -56,6 +56,7 @@ SIGNATURES = {
     "cm_permute16": (_I32, [_P, _P] + [_U32] * 4 + [ctypes.c_uint64] * 4 + [_P]),
     "cm_copy16": (_I32, [_P, _P] + [_U32] * 4 + [ctypes.c_uint64] * 8 + [_P]),
     "cm_embed_rows": (_I32, [_P, _U32, _P, _P, _U32, _U32, _U32, _P]),
+    "cm_attention_strided": (_I32, [_P] * 4 + [_U32] * 5 + [ctypes.c_uint64] * 13 + [_U32] * 3 + [_P, _U32, _P]),
     "cm_attention": (_I32, [_P, _P] + [_U32] * 4 + [ctypes.c_uint64] + [_U32] * 3 + [ctypes.c_uint64] + [_U32] * 2 + [_P]),
     "cm_decode_attention": (_I32, [_P, _P, _P, _P] + [_U32] * 7 + [_P]),
     "cm_decode_prep": (_I32, [_P] * 6 + [_U32] * 6 + [_P, _P, _U32, _P, _U32, _P]),

@@ -388,6 +388,319 @@ int run_attention(const int16_t* qkv, int16_t* o, uint32_t batch, uint32_t seq, 
     return fail(CM_EINVAL, "attention: %u keys", seq);
 }
 
+// ---------------------------------------------------------------- attention over any keys
+// The same chain for any number of queries and keys that are multiples of 16 (at most 1024 keys),
+// with the softmax's mask register (causal: valid0 + q keys for query q) and every operand at its
+// own strides: an encoder's sequences that the kernel above has no instance for, and a prompt's
+// queries over a KV cache (q in the q.K^T image, d apart q_ds).  Node by node such a layer runs
+// head transposes, two operand splits a contraction, two GEMMs and the softmax, each a launch over
+// a few workgroups: 95 us at 5 sequences of 208 tokens and 12 heads, 75 us a KV group for 256
+// queries over 560 keys.
+//
+// A workgroup takes 16 queries of one (sequence, head) pair and its 4 wavefronts the keys: wave w
+// the 64-key steps w, w + 4, .. (at most NS), so that few queries still fill the chip and a lane's
+// scores (4 of each 16-key block for one query, as above) stay in registers.  K rows are the MFMA
+// operand as they lie in memory; the maximum and the sum of a query meet in LDS; V^T goes through
+// the wave's own LDS tile (64 keys a step, keys in the lane's own order); the waves' int32 partial
+// sums of o are added in LDS (the wrapped sum is one mod 2^32, so the order is free).  All offset
+// terms come from MFMAs against ones: sum_j P V = 2^16 HH + 2^8 MID + LL + 2^15 sum h_V + 2^7 sum l_V
+// + 128 sum P over every 64-key step, keys past the end taken as V = P = 0.
+struct AttnPairs {
+    const int16_t *q, *k, *v;
+    int16_t* o;
+    uint64_t q_ld, q_ds, q_bs, q_bs2, k_ld, k_bs, k_bs2, v_ld, v_bs, v_bs2, o_ld, o_bs, o_bs2;
+    uint32_t keys, inner, valid0, period, cm, cfg, dlim;
+    uint32_t p_rows, p_heads;                // plane row / head of an outer step (pair / inner)
+};
+constexpr uint32_t kVs = 80;                 // V^T plane row stride in bytes (64 keys, rows 20 banks apart)
+constexpr uint32_t kOs = 68;                 // partial o row stride in dwords
+
+template <uint32_t NS>
+__global__ __launch_bounds__(256, 2) void attention_pairs_kernel(AttnPairs a, const int32_t* __restrict__ tab,
+                                                                 APlanes po) {
+    __shared__ __attribute__((aligned(16))) int32_t stab[4096];
+    __shared__ __attribute__((aligned(16))) uint8_t vt[4][2 * kHd * kVs];          // [wave][hi, lo][64 d][kVs]
+    __shared__ int32_t redm[4][16], reds[4][16];
+    const uint32_t t = threadIdx.x, lane = t & 63, c16 = lane & 15, g = lane >> 4;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t pair = blockIdx.y, outer = pair / a.inner, in = pair - outer * a.inner;
+    const uint32_t q0 = blockIdx.x * 16, qi = q0 + c16;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++)
+        __builtin_amdgcn_global_load_lds(tab + 4 * (t + 256 * i),
+                                         (__attribute__((address_space(3))) void*)(stab + 4 * (64 * w + 256 * i)), 16, 0, 0);
+    const int16_t* kp = a.k + outer * a.k_bs + in * a.k_bs2 + 16 * g;
+    const int16_t* vp = a.v + outer * a.v_bs + in * a.v_bs2;
+    auto valid_of = [&](uint32_t q) { return min(a.valid0 + (a.period ? q % a.period : 0u), a.keys); };
+    const uint32_t valid = valid_of(qi);
+    // keys past every query's valid ones have P = 0: the last 16-key block any query of the tile needs
+    uint32_t kend = valid;
+#pragma unroll
+    for (uint32_t off = 1; off < 16; off <<= 1) kend = max(kend, (uint32_t)__shfl_xor((int)kend, off, 64));
+    kend = __builtin_amdgcn_readfirstlane((kend + 15) & ~15u);
+
+    // ---- the tile's queries (B of phase 1): query qi, d 16 g ..
+    v4i qh, ql;
+    {
+        const int16_t* qp = a.q + outer * a.q_bs + in * a.q_bs2 + (uint64_t)qi * a.q_ld + 16 * g * a.q_ds;
+        if (a.q_ds == 1) {
+            limbs16(qp, qh, ql);
+        } else {
+            __attribute__((aligned(16))) int16_t e[16];
+#pragma unroll
+            for (uint32_t i = 0; i < 16; i++) e[i] = qp[i * a.q_ds];
+            limbs16(e, qh, ql);
+        }
+    }
+    const v4i zero = {0, 0, 0, 0};
+    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    const v4i c20 = {1 << 20, 1 << 20, 1 << 20, 1 << 20};
+    const v4i qh1 = mfma(ones, qh, zero), ql1 = mfma(ones, ql, zero);
+
+    // ---- phase 1: the scores of the wave's steps; the unread ones stay below every score
+    int32_t sv[16 * NS];
+#pragma unroll
+    for (uint32_t s = 0; s < NS; s++) {
+        const uint32_t k0 = 64 * (w + 4 * s);
+        if (k0 < kend) {
+            int4 x[4][2];
+#pragma unroll
+            for (uint32_t kb = 0; kb < 4; kb++) {
+                const int16_t* kr = kp + (uint64_t)min(k0 + 16 * kb + c16, a.keys - 1) * a.k_ld;
+                x[kb][0] = *reinterpret_cast<const int4*>(kr);
+                x[kb][1] = *reinterpret_cast<const int4*>(kr + 8);
+            }
+#pragma unroll
+            for (uint32_t kb = 0; kb < 4; kb++) {
+                uint32_t h0, h1, h2, h3, l0, l1, l2, l3;
+                limbs8(x[kb][0], h0, h1, l0, l1);
+                limbs8(x[kb][1], h2, h3, l2, l3);
+                const v4i kh = {(int)h0, (int)h1, (int)h2, (int)h3}, kl = {(int)l0, (int)l1, (int)l2, (int)l3};
+                const v4i hh = mfma(kh, qh, zero);
+                v4i mid = mfma(kh, ql, zero);
+                mid = mfma(kl, qh, mid);
+                const v4i ll = mfma(kl, ql, c20);
+                const v4i ha = mfma(kh, ones, qh1), la = mfma(kl, ones, ql1);
+#pragma unroll
+                for (uint32_t r = 0; r < 4; r++) {
+                    const uint32_t acc = ((uint32_t)hh[r] << 16) + ((uint32_t)mid[r] << 8) + (uint32_t)ll[r] +
+                                         ((uint32_t)ha[r] << 15) + ((uint32_t)la[r] << 7);
+                    sv[16 * s + 4 * kb + r] = sat16_shr8((int32_t)acc);
+                }
+            }
+        } else {
+#pragma unroll
+            for (uint32_t n = 0; n < 16; n++) sv[16 * s + n] = 0;
+        }
+    }
+
+    // ---- phase 2: the softmax over the valid keys of the lane's query
+    auto key_of = [&](uint32_t s, uint32_t n) { return 64 * (w + 4 * s) + 16 * (n >> 2) + 4 * g + (n & 3); };
+    int32_t mx = -32768;
+#pragma unroll
+    for (uint32_t s = 0; s < NS; s++)
+#pragma unroll
+        for (uint32_t n = 0; n < 16; n++) mx = max(mx, key_of(s, n) < valid ? sv[16 * s + n] : -32768);
+    mx = max(mx, __shfl_xor(mx, 16, 64));
+    mx = max(mx, __shfl_xor(mx, 32, 64));
+    if (g == 0) redm[w][c16] = mx;
+    __builtin_amdgcn_s_waitcnt(0x0070);                // this wave's TAB copies and LDS writes
+    __syncthreads();
+    mx = max(max(redm[0][c16], redm[1][c16]), max(redm[2][c16], redm[3][c16]));
+    const uint32_t cs = a.cfg & 63u, fp = (a.cfg >> 8) & 31u;
+    const uint64_t cm24 = a.cm & 0xFFFFFFu;
+    uint32_t part = 0;
+#pragma unroll
+    for (uint32_t s = 0; s < NS; s++)
+#pragma unroll
+        for (uint32_t n = 0; n < 16; n++) {
+            const uint32_t d = (uint32_t)(mx - sv[16 * s + n]);      // of a key past valid: any, masked
+            const uint32_t y = (uint32_t)(((uint64_t)d * cm24) >> cs);
+            const bool on = key_of(s, n) < valid && d < a.dlim;
+            const uint32_t e = ((uint32_t)stab[y & 4095] >> ((y >> 12) & 31)) & (on ? ~0u : 0u);
+            sv[16 * s + n] = (int32_t)e;
+            part += e;
+        }
+    part += __shfl_xor(part, 16, 64);
+    part += __shfl_xor(part, 32, 64);
+    if (g == 0) reds[w][c16] = (int32_t)part;
+    __syncthreads();
+    const uint32_t S = (uint32_t)reds[0][c16] + (uint32_t)reds[1][c16] + (uint32_t)reds[2][c16] + (uint32_t)reds[3][c16];
+    const uint64_t R = ((uint64_t)1 << 40) / (uint64_t)(S ? S : 1u);
+    const double rd = __builtin_ldexp((double)R, (int)fp - 40);
+    int psum = 0;
+#pragma unroll
+    for (uint32_t n = 0; n < 16 * NS; n++) {
+        sv[n] = (int32_t)__builtin_fmin(__builtin_fma((double)(uint32_t)sv[n], rd, 0.5), 32767.0);
+        psum += sv[n];
+    }
+    psum += __shfl_xor(psum, 16, 64);
+    psum += __shfl_xor(psum, 32, 64);                  // sum of the wave's P of query qi
+
+    // ---- phase 3: the wave's part of o^T[d][qi], 4 blocks of 16 d
+    uint8_t* vth = vt[w];
+    uint8_t* vtl = vth + kHd * kVs;
+    v4i ohh[4], omid[4], oll[4], oha[4], ola[4];
+#pragma unroll
+    for (uint32_t m = 0; m < 4; m++) ohh[m] = omid[m] = oll[m] = oha[m] = ola[m] = zero;
+#pragma unroll
+    for (uint32_t s = 0; s < NS; s++) {
+        const uint32_t k0 = 64 * (w + 4 * s);
+        if (k0 >= kend) break;
+        // V^T of the step: a task is 4 keys (4 qd ..) x 8 d (8 c ..)
+        const uint32_t c = lane & 7;
+        int4 x[2][4];
+#pragma unroll
+        for (uint32_t it = 0; it < 2; it++) {
+            const uint32_t key = k0 + 4 * ((lane >> 3) + 8 * it);          // keys is a multiple of 16
+            const int16_t* vr = vp + (uint64_t)(key < a.keys ? key : 0) * a.v_ld + 8 * c;
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) {
+                x[it][r] = *reinterpret_cast<const int4*>(vr + r * a.v_ld);
+                if (key >= a.keys) x[it][r] = make_int4(0, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (uint32_t it = 0; it < 2; it++) {
+            const uint32_t qd = (lane >> 3) + 8 * it, p0 = 16 * (qd & 3) + 4 * (qd >> 2);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++) {
+                const uint32_t a0 = dword(x[it][0], q), a1 = dword(x[it][1], q), a2 = dword(x[it][2], q), a3 = dword(x[it][3], q);
+                const uint32_t th01 = __builtin_amdgcn_perm(a1, a0, 0x07030501u);
+                const uint32_t th23 = __builtin_amdgcn_perm(a3, a2, 0x07030501u);
+                const uint32_t tl01 = __builtin_amdgcn_perm(a1, a0, 0x06020400u);
+                const uint32_t tl23 = __builtin_amdgcn_perm(a3, a2, 0x06020400u);
+                const uint32_t d0 = 8 * c + 2 * q;
+                *reinterpret_cast<uint32_t*>(vth + d0 * kVs + p0) = __builtin_amdgcn_perm(th23, th01, 0x05040100u);
+                *reinterpret_cast<uint32_t*>(vth + (d0 + 1) * kVs + p0) = __builtin_amdgcn_perm(th23, th01, 0x07060302u);
+                *reinterpret_cast<uint32_t*>(vtl + d0 * kVs + p0) = __builtin_amdgcn_perm(tl23, tl01, 0x05040100u) ^ 0x80808080u;
+                *reinterpret_cast<uint32_t*>(vtl + (d0 + 1) * kVs + p0) =
+                    __builtin_amdgcn_perm(tl23, tl01, 0x07060302u) ^ 0x80808080u;
+            }
+        }
+        // the tile is the wave's own: LDS operations of a wave complete in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        uint32_t ph[4], pl[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) {
+            const uint32_t n = 16 * s + 4 * q;
+            const uint32_t p01 = (uint32_t)sv[n] | ((uint32_t)sv[n + 1] << 16);              // P in [0, 32767]
+            const uint32_t p23 = (uint32_t)sv[n + 2] | ((uint32_t)sv[n + 3] << 16);
+            ph[q] = __builtin_amdgcn_perm(p23, p01, 0x07050301u);
+            pl[q] = __builtin_amdgcn_perm(p23, p01, 0x06040200u) ^ 0x80808080u;
+        }
+        const v4i bh4 = {(int)ph[0], (int)ph[1], (int)ph[2], (int)ph[3]};
+        const v4i bl4 = {(int)pl[0], (int)pl[1], (int)pl[2], (int)pl[3]};
+#pragma unroll
+        for (uint32_t m = 0; m < 4; m++) {
+            const uint32_t off = (16 * m + c16) * kVs + 16 * g;
+            const v4i vh = *reinterpret_cast<const v4i*>(vth + off);
+            const v4i vl = *reinterpret_cast<const v4i*>(vtl + off);
+            ohh[m] = mfma(vh, bh4, ohh[m]);
+            omid[m] = mfma(vh, bl4, omid[m]);
+            oha[m] = mfma(vh, ones, oha[m]);
+            omid[m] = mfma(vl, bh4, omid[m]);
+            oll[m] = mfma(vl, bl4, oll[m]);
+            ola[m] = mfma(vl, ones, ola[m]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    }
+    // the wave's partials [query][d] over its own V^T tile (every read of it done)
+    int32_t* pw = reinterpret_cast<int32_t*>(vt[w]);
+#pragma unroll
+    for (uint32_t m = 0; m < 4; m++) {
+        v4i x;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++)
+            x[r] = (int32_t)(((uint32_t)ohh[m][r] << 16) + ((uint32_t)omid[m][r] << 8) + (uint32_t)oll[m][r] +
+                             ((uint32_t)oha[m][r] << 15) + ((uint32_t)ola[m][r] << 7) + 128u * (uint32_t)psum);
+        *reinterpret_cast<v4i*>(pw + c16 * kOs + 16 * m + 4 * g) = x;
+    }
+    __syncthreads();
+
+    // ---- o: lane (query 4 w + lane / 16, d 4 (lane % 16) ..) adds the four waves' partials
+    const uint32_t qr = 4 * w + g, d0 = 4 * c16, q = q0 + qr;
+    v4i x = zero;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+        const v4i y = *reinterpret_cast<const v4i*>(reinterpret_cast<const int32_t*>(vt[i]) + qr * kOs + d0);
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) x[r] = (int32_t)((uint32_t)x[r] + (uint32_t)y[r]);
+    }
+    uint32_t pk[2];
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r += 2)
+        pk[r / 2] = (uint32_t)(uint16_t)sat16_shr8(x[r]) | ((uint32_t)(uint16_t)sat16_shr8(x[r + 1]) << 16);
+    if (a.o != nullptr)
+        *reinterpret_cast<uint2*>(a.o + outer * a.o_bs + in * a.o_bs2 + (uint64_t)q * a.o_ld + d0) = make_uint2(pk[0], pk[1]);
+    if (po.hi != nullptr) {
+        const uint64_t prow = (uint64_t)outer * a.p_rows + q;
+        const uint32_t head = outer * a.p_heads + in;
+        *reinterpret_cast<uint32_t*>(po.hi + prow * po.k + kHd * head + d0) = __builtin_amdgcn_perm(pk[1], pk[0], 0x07050301u);
+        *reinterpret_cast<uint32_t*>(po.lo + prow * po.k + kHd * head + d0) =
+            __builtin_amdgcn_perm(pk[1], pk[0], 0x06040200u) ^ 0x80808080u;
+        int32_t sum = (int32_t)(int16_t)(pk[0] & 0xFFFF) + ((int32_t)pk[0] >> 16) + (int32_t)(int16_t)(pk[1] & 0xFFFF) +
+                      ((int32_t)pk[1] >> 16);
+#pragma unroll
+        for (uint32_t off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off, 64);
+        if (c16 == 0) po.part[(uint64_t)head * po.lines + prow] = sum;
+    }
+}
+
+int run_attention_pairs(AttnPairs a, uint32_t nq, uint32_t batch, uint32_t head_dim, uint32_t mask, void* planes,
+                        uint32_t planes_rows, hipStream_t s) {
+    DeviceState* st;
+    int rc = state(&st);
+    if (rc) return rc;
+    if (batch == 0 || nq == 0) return CM_OK;
+    if (a.q == nullptr || a.k == nullptr || a.v == nullptr || (a.o == nullptr && planes == nullptr))
+        return fail(CM_EINVAL, "attention: a null operand, or a null o without planes");
+    if (head_dim != kHd) return fail(CM_EINVAL, "attention: head_dim %u (the kernel takes 64)", head_dim);
+    if ((nq & 15) || (a.keys & 15) || a.keys == 0 || a.keys > 1024)
+        return fail(CM_EINVAL, "attention: %u queries, %u keys (multiples of 16, at most 1024 keys)", nq, a.keys);
+    if (a.inner == 0 || batch % a.inner) return fail(CM_EINVAL, "attention: %u pairs by %u", batch, a.inner);
+    if (batch > 65535) return fail(CM_EINVAL, "attention: %u pairs", batch);
+    const uint32_t fp = (a.cfg >> 8) & 31u;
+    if (fp == 0u) return fail(CM_EINVAL, "attention: softmax output bits %u", fp);
+    if (a.q_ds == 0) return fail(CM_EINVAL, "attention: q_ds 0");
+    const bool q_ok = a.q_ds != 1 || (aligned16(a.q) && ((a.q_ld | a.q_bs | a.q_bs2) & 7) == 0);
+    if (!q_ok || !aligned16(a.k) || !aligned16(a.v) || !aligned16(a.o) ||
+        ((a.k_ld | a.k_bs | a.k_bs2 | a.v_ld | a.v_bs | a.v_bs2 | a.o_ld | a.o_bs | a.o_bs2) & 7))
+        return fail(CM_EALIGN, "attention: rows, heads and sequences must be 16-byte aligned");
+    a.valid0 = mask & 0xFFFFu;
+    a.period = mask >> 16;
+    a.dlim = smx_dlim(a.cm & 0xFFFFFFu, a.cfg & 63u);
+    APlanes po{};
+    if (planes != nullptr) {
+        // the matmul's A: planes_rows rows of all heads; the outer pairs are rows or, at nq rows, heads
+        const uint64_t rows = (uint64_t)(batch / a.inner) * nq;
+        const bool by_head = planes_rows == nq;
+        if ((!by_head && planes_rows != rows) || (reinterpret_cast<uintptr_t>(planes) & 255))
+            return fail(CM_EINVAL, "attention planes: %u rows, 256-byte aligned", planes_rows);
+        const uint32_t heads = by_head ? batch : a.inner;
+        if (heads > 64) return fail(CM_EINVAL, "attention planes: %u heads above 64", heads);
+        a.p_rows = by_head ? 0 : nq;
+        a.p_heads = by_head ? a.inner : 0;
+        po = a_planes_view(planes, planes_rows, heads * kHd, heads);
+    }
+    const dim3 grid(nq / 16, batch);
+    switch ((a.keys + 255) / 256) {
+#define CM_ATP(NS)                                                                                                \
+    case NS:                                                                                                      \
+        CM_LAUNCH("attention_kernel", attention_pairs_kernel<NS>, grid, dim3(256), 0, s, a, st->smx_tab, po);     \
+        return CM_OK;
+        CM_ATP(1) CM_ATP(2) CM_ATP(3)
+    default:
+        CM_LAUNCH("attention_kernel", attention_pairs_kernel<4>, grid, dim3(256), 0, s, a, st->smx_tab, po);
+        return CM_OK;
+#undef CM_ATP
+    }
+}
+
 }  // namespace
 }  // namespace cm
 
@@ -404,4 +717,15 @@ extern "C" int cm_attention_planes(const int16_t* qkv, int16_t* o, uint32_t batc
     if (planes == nullptr) return cm::fail(CM_EINVAL, "attention planes: no planes buffer");
     return cm::run_attention(qkv, o, batch, seq, heads, head_dim, ld, q_off, k_off, v_off, (uint64_t)heads * 64,
                              smx_cm, smx_cfg, planes, cm::as_stream(stream));
+}
+
+extern "C" int cm_attention_strided(const int16_t* q, const int16_t* k, const int16_t* v, int16_t* o, uint32_t nq,
+                                    uint32_t keys, uint32_t batch, uint32_t inner, uint32_t head_dim, uint64_t q_ld,
+                                    uint64_t q_ds, uint64_t q_bs, uint64_t q_bs2, uint64_t k_ld, uint64_t k_bs,
+                                    uint64_t k_bs2, uint64_t v_ld, uint64_t v_bs, uint64_t v_bs2, uint64_t o_ld,
+                                    uint64_t o_bs, uint64_t o_bs2, uint32_t smx_cm, uint32_t smx_cfg,
+                                    uint32_t smx_mask, void* planes, uint32_t planes_rows, void* stream) {
+    cm::AttnPairs a{q, k, v, o, q_ld, q_ds, q_bs, q_bs2, k_ld, k_bs, k_bs2, v_ld, v_bs, v_bs2, o_ld, o_bs, o_bs2,
+                    keys, inner, 0, 0, smx_cm, smx_cfg, 0, 0, 0};
+    return cm::run_attention_pairs(a, nq, batch, head_dim, smx_mask, planes, planes_rows, cm::as_stream(stream));
 }

@@ -19,7 +19,7 @@ from .dtype import AP_FIXED_16_8, ApFixed16
 from .graph import (AttentionNode, AttnContractNode, AttnMergeNode, AttnSoftmaxNode, ConvNode, DecodeAttentionNode, Graph,
                     KvWriteNode, LlmAttnConvNode, MatmulConvNode, SelectRowNode,
                     MatmulNode, PermuteNode, PoolNode, ReshapeNode, RowOpsNode, ScheduledNode, SchedulerError, SoftmaxVopNode,
-                    TensorInfo, attn_keys)
+                    SMX_MAX_KEYS, TensorInfo, attn_keys)
 from .packing import conv_bias_image, conv_lowered_b_image, conv_weight_image, pack_matmul_b
 from .host_ops import HostNode, LlmEmbedNode
 from .rowops_nodes import DecodePrepNode, RoCallNode, RoJob, RowOpsAdapter
@@ -190,6 +190,12 @@ class Simulator:
                 # a residual add and the LayerNorm of its output: one launch, both outputs kept
                 self._addx_norm(sn, nodes[i], raw)
                 i += 1
+                continue
+            chain = self._attn_chain(i - 1)
+            if chain is not None:
+                # a prompt's attention, group by group: one launch, the merged output alone
+                self._attn_chain_run(chain, raw)
+                i += 3 * chain[0].KV
                 continue
             if i < len(nodes) and self._conv_act_fusable(sn, nodes[i]):
                 # a convolution and the RELU / RELU6 of its output: one launch, the activated output alone
@@ -580,10 +586,13 @@ class Simulator:
             return None
         if isinstance(p, AttentionNode):
             cols = p.heads * p.head_dim
-            ok = (p.head_dim == 64 and p.seq in (64, 128, 256, 384) and cols == k and p.batch * p.seq == n
+            ok = (p.head_dim == 64 and (p.seq in self._ATT_SEQ or self._att_any(p)) and cols == k and p.batch * p.seq == n
                   and int(p.inputs[0].shape[-1]) % 8 == 0 and p.q_off % 8 == 0 and p.k_off % 8 == 0
                   and p.v_off % 8 == 0 and p.heads <= 64)
             return p.heads if ok else None
+        if isinstance(p, AttnMergeNode):
+            # written with the planes where the chain before it runs as one launch (_attn_chain)
+            return p.H if p.HD == 64 and p.H <= 64 and p.T == n and p.H * 64 == k and ot.numel == n * k else None
         if isinstance(p, ScheduledNode) and p.op_code <= 9 and ot.numel == n * k and k <= 32768:
             if p.arity == 1:
                 return (k + 1023) // 1024 if p.inputs[0].numel == n * k else None
@@ -621,6 +630,8 @@ class Simulator:
     def _planes_node(self, sn, raw) -> bool:
         """Run ``sn`` with the byte planes of its output as well (raw[name + '#planes']); False
         if it runs the plain way after all."""
+        if isinstance(sn, AttnMergeNode):            # its planes come from the whole chain's launch alone
+            return False
         n, k, nsum = self._planes_out(sn)
         name = sn.output.onnx_name
         planes = units.a_planes(n, k, nsum, self.device)
@@ -1238,6 +1249,12 @@ class Simulator:
                 return o
             units.attention(x, o, B, T, H, hd, ld, sn.q_off, sn.k_off, sn.v_off, cols, sn.cm, sn.cfg)
             return o
+        if self._att_any(sn) and ld % 8 == 0 and sn.q_off % 8 == 0 and sn.k_off % 8 == 0 and sn.v_off % 8 == 0:
+            view = lambda off: (off, ld, T * ld, hd)                                     # noqa: E731
+            units.attention_strided(x, x, x, o, T, T, B * H, H, view(sn.q_off), view(sn.k_off), view(sn.v_off),
+                                    (0, cols, T * cols, hd), sn.cm, sn.cfg, T, planes=planes, planes_rows=B * T)
+            self._attention_out = o
+            return o
         if planes is not None:
             raise SchedulerError(f"attention '{ot.onnx_name}': no planes for this shape")
         if T % 16:
@@ -1258,6 +1275,88 @@ class Simulator:
         units.matmul(pr, vh, oh, T, T, hd, batch=BH, a_bs=T * kp, b_bs=T * hd, c_bs=T * hd, wrap32=True)
         units.permute16(oh, o, (B, T, H, hd), (H * T * hd, hd, T * hd, 1))
         return o
+
+    _ATT_SEQ = (64, 128, 256, 384)               # sequence lengths cm_attention takes
+
+    @staticmethod
+    def _att_any(sn: AttentionNode) -> bool:
+        """An AttentionNode cm_attention_strided takes (other lengths than _ATT_SEQ)."""
+        return (sn.head_dim == 64 and sn.seq % 16 == 0 and 0 < sn.seq <= 1024 and sn.batch * sn.heads <= 65535
+                and 0 < (sn.cfg >> 8) & 31)
+
+    def _attn_chain(self, i: int):
+        """The attention of a prompt (or an encoder's prep chain) that starts at node ``i``: per KV group,
+        in order, q.K^T (LlmAttnConvNode), the softmax node and P.V, then the merge, where no score, P
+        or group output is kept or read by another node -- (the first q.K^T, the first softmax, the first
+        P.V, the merge), one cm_attention_strided call; else None.  Scores, P and the groups' outputs are
+        then not materialized."""
+        nodes = self._graph.nodes
+        qk = nodes[i]
+        if self._keep is None or not (isinstance(qk, LlmAttnConvNode) and qk.kind == "qk" and qk.group == 0):
+            return None
+        KV, G, T, C = qk.KV, qk.G, qk.T, qk.C
+        if (i + 3 * KV >= len(nodes) or qk.HD != 64 or KV < 1 or G < 1 or qk.H != KV * G or T % 16 or C % 16
+                or C > SMX_MAX_KEYS or qk.H > 65535 or (G * T) % 8):
+            return None
+        merge = nodes[i + 3 * KV]
+        if not (isinstance(merge, AttnMergeNode) and (merge.T, merge.H, merge.KV, merge.HD) == (T, qk.H, KV, 64)
+                and len(merge.inputs) == KV):
+            return None
+        sm0, pv0 = nodes[i + 1], nodes[i + 2]
+        if not (isinstance(sm0, AttnSoftmaxNode) and isinstance(pv0, LlmAttnConvNode)):
+            return None
+        names = lambda ts: [t.onnx_name for t in ts]                                     # noqa: E731
+        fixed = set(self._keep) | {t.onnx_name for t in self._graph.output_tensors + self._graph.state_tensors}
+        counts = self._reader_counts()
+        regs = None
+        for g in range(KV):
+            a, sm, b = nodes[i + 3 * g:i + 3 * g + 3]
+            if not (isinstance(a, LlmAttnConvNode) and isinstance(sm, AttnSoftmaxNode) and isinstance(b, LlmAttnConvNode)
+                    and a.kind == "qk" and b.kind == "pv" and a.group == b.group == g):
+                return None
+            geo = (T, qk.H, KV, 64, C, qk.Q, qk.static, qk.has_n)
+            if any((c.T, c.H, c.KV, c.HD, c.C, c.Q, c.static, c.has_n) != geo for c in (a, b)):
+                return None
+            if (sm.T, sm.G, sm.C, sm.Q, sm.causal, sm.static) != (T, G, C, qk.Q, sm0.causal, qk.static):
+                return None
+            regs = sm.regs()[0] if regs is None else regs
+            if any(r != regs for r in sm.regs()):
+                return None
+            if (names(a.inputs) != names(qk.inputs) or names(b.inputs[1:]) != names(pv0.inputs[1:])
+                    or names(sm.inputs[1:]) != names(qk.inputs[2:]) or names(b.inputs[2:]) != names(qk.inputs[2:])):
+                return None
+            links = (a.output.onnx_name, sm.output.onnx_name, b.output.onnx_name)
+            if links != (sm.inputs[0].onnx_name, b.inputs[0].onnx_name, merge.inputs[g].onnx_name):
+                return None
+            if any(nm in fixed or counts.get(nm, 0) != 1 for nm in links):
+                return None
+        if qk.inputs[0].group_layout != (KV, 64) or pv0.inputs[1].group_layout != (KV, 64) or not 0 < (regs[1] >> 8) & 31:
+            return None
+        return qk, sm0, pv0, merge
+
+    def _attn_chain_run(self, chain, raw) -> None:
+        """_attn_chain's nodes in one launch: the merged output (and the byte planes of the MatMul that
+        takes it as A), q read from its q.K^T image [KV][HD][G T], K / V from the group-major caches."""
+        qk, sm, pv, merge = chain
+        KV, G, T, C, H = qk.KV, qk.G, qk.T, qk.C, qk.H
+        pos, n_in = sm.pos_n(lambda t: self._host_int(t, raw))
+        n, keys = attn_keys(pos, n_in, T, C, qk.Q)
+        if qk.static:
+            keys = C
+        name = merge.output.onnx_name
+        pl = self._planes_out(merge)
+        planes = units.a_planes(*pl, self.device) if pl is not None else None
+        out = None if planes is not None and self._planes_only(name) else self._new(merge.output)
+        cm_r, cfg = sm.regs()[0]
+        cache = (0, 64, C * 64, 0)
+        units.attention_strided(self._get(qk.inputs[1], raw).reshape(-1), self._get(qk.inputs[0], raw).reshape(-1),
+                                self._get(pv.inputs[1], raw).reshape(-1), out, T, keys, H, G,
+                                (0, 1, 64 * G * T, T), cache, cache, (0, H * 64, G * 64, 64), cm_r, cfg,
+                                sm.mask_reg(pos, n, keys), q_ds=G * T, planes=planes, planes_rows=T)
+        if out is not None:
+            raw[name] = out
+        if planes is not None:
+            raw[name + "#planes"] = planes
 
     def _decode_attention(self, sn: DecodeAttentionNode, raw) -> torch.Tensor:
         """q.K^T, the row-mode softmax and P.V of every KV group in one launch."""

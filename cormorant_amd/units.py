@@ -165,6 +165,40 @@ def attention(qkv: torch.Tensor, o: torch.Tensor, batch: int, seq: int, heads: i
     return o
 
 
+def attention_strided(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: Optional[torch.Tensor], nq: int, keys: int,
+                      batch: int, inner: int, q_view, k_view, v_view, o_view, smx_cm: int, smx_cfg: int, smx_mask: int,
+                      q_ds: int = 1, planes: Optional[torch.Tensor] = None, planes_rows: int = 0,
+                      head_dim: int = 64) -> Optional[torch.Tensor]:
+    """cm_attention_strided: the attention of ``batch`` (sequence, head) pairs.  Each view is (offset,
+    ld, bs, bs2) in elements of its tensor: pair p at offset + (p // inner) bs + (p % inner) bs2, rows ld
+    apart (q's d elements q_ds apart); with ``planes`` (a_planes) o's byte planes too, and o may be None."""
+    if inner < 1 or batch % inner:
+        raise ValueError(f"attention_strided: {batch} pairs by {inner}")
+
+    def extent(view, rows, last):
+        off, ld, bs, bs2 = view
+        return off + (batch // inner - 1) * bs + (inner - 1) * bs2 + (rows - 1) * ld + last
+    if batch and nq and keys:
+        if min(min(view) for view in (q_view, k_view, v_view, o_view)) < 0 or q_ds < 1:
+            raise ValueError("attention_strided: negative strides or offsets")
+        _require(q, "q", torch.int16, extent(q_view, nq, (head_dim - 1) * q_ds + 1))
+        _require(k, "k", torch.int16, extent(k_view, keys, head_dim))
+        _require(v, "v", torch.int16, extent(v_view, keys, head_dim))
+        if o is not None:
+            _require(o, "o", torch.int16, extent(o_view, nq, head_dim))
+        if planes is not None:
+            heads = batch if planes_rows == nq else inner
+            _require_planes(planes, planes_rows, heads * head_dim, heads)
+    (qo, qld, qb, qb2), (ko, kld, kb, kb2), (vo, vld, vb, vb2), (oo, old, ob, ob2) = q_view, k_view, v_view, o_view
+    rc = _lib.lib().cm_attention_strided(_ptr(q) + 2 * qo, _ptr(k) + 2 * ko, _ptr(v) + 2 * vo,
+                                         _ptr(o) + 2 * oo if o is not None else None, nq, keys, batch, inner, head_dim,
+                                         qld, q_ds, qb, qb2, kld, kb, kb2, vld, vb, vb2, old, ob, ob2,
+                                         smx_cm & 0xFFFFFFFF, smx_cfg & 0xFFFFFFFF, smx_mask & 0xFFFFFFFF, _ptr(planes),
+                                         planes_rows, _stream())
+    _lib.check(rc, "cm_attention_strided")
+    return o
+
+
 def matmul_b_extent(k: int, m: int, b_packed: int, gemv_kw: int) -> int:
     if gemv_kw or b_packed == 2:
         return k * m
