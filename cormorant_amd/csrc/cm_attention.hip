@@ -340,6 +340,17 @@ void* attention_fn() {
     return reinterpret_cast<void*>(&attention_kernel<T, PL>);
 }
 
+// The operands of attention_pairs_kernel (below), with their strides.
+struct AttnPairs {
+    const int16_t *q, *k, *v;
+    int16_t* o;
+    uint64_t q_ld, q_ds, q_bs, q_bs2, k_ld, k_bs, k_bs2, v_ld, v_bs, v_bs2, o_ld, o_bs, o_bs2;
+    uint32_t keys, inner, valid0, period, cm, cfg, dlim;
+    uint32_t p_rows, p_heads;                // plane row / head of an outer step (pair / inner)
+};
+int run_attention_pairs(AttnPairs a, uint32_t nq, uint32_t batch, uint32_t head_dim, uint32_t mask, void* planes,
+                        uint32_t planes_rows, hipStream_t s);
+
 int run_attention(const int16_t* qkv, int16_t* o, uint32_t batch, uint32_t seq, uint32_t heads, uint32_t head_dim,
                   uint64_t ld, uint32_t q_off, uint32_t k_off, uint32_t v_off, uint64_t o_ld, uint32_t smx_cm,
                   uint32_t smx_cfg, void* planes, hipStream_t s) {
@@ -360,6 +371,14 @@ int run_attention(const int16_t* qkv, int16_t* o, uint32_t batch, uint32_t seq, 
     if (planes != nullptr && (o_ld != (uint64_t)heads * kHd || heads > 64 || (reinterpret_cast<uintptr_t>(planes) & 255)))
         return fail(CM_EINVAL, "attention planes: o rows of exactly heads x 64 (at most 64 heads), 256-byte aligned "
                                "planes");
+    // few (sequence, head) pairs: 16 queries a workgroup, the keys over its wavefronts (12 heads, us: 128
+    // tokens 8.0 -> 5.8 at batch 1, 8.2 -> 7.7 at 4, 8.5 against 9.7 at 8; 256 tokens 11.2 -> 8.9 at 2,
+    // 11.6 either way at 4; 384 tokens 14.5 -> 12.3 at 1, 15.0 against 16.0 at 2; 64 tokens 6.7 -> 5.9 at 4)
+    if (seq / 16 * batch * heads <= (uint32_t)st->cus * (seq > 64 ? 3 : 2) / 2) {
+        const AttnPairs a{qkv + q_off, qkv + k_off, qkv + v_off, o, ld, 1, seq * ld, kHd, ld, seq * ld, kHd, ld,
+                          seq * ld, kHd, o_ld, seq * o_ld, kHd, seq, heads, 0, 0, smx_cm, smx_cfg, 0, 0, 0};
+        return run_attention_pairs(a, seq, batch * heads, head_dim, seq, planes, batch * seq, s);
+    }
     const size_t lds = 16384 + 2 * (size_t)(kHd / 2) * (seq + 16) + 4 * 64 * sizeof(int32_t);
     if (lds > st->lds_per_block) return fail(CM_EINVAL, "attention: %zu bytes of LDS per workgroup", lds);
     const uint32_t dlim = smx_dlim(smx_cm & 0xFFFFFFu, smx_cfg & 63u);
@@ -394,8 +413,10 @@ int run_attention(const int16_t* qkv, int16_t* o, uint32_t batch, uint32_t seq, 
 // own strides: an encoder's sequences that the kernel above has no instance for, and a prompt's
 // queries over a KV cache (q in the q.K^T image, d apart q_ds).  Node by node such a layer runs
 // head transposes, two operand splits a contraction, two GEMMs and the softmax, each a launch over
-// a few workgroups: 95 us at 5 sequences of 208 tokens and 12 heads, 75 us a KV group for 256
-// queries over 560 keys.
+// a few workgroups: 95 us at 5 sequences of 208 tokens and 12 heads (14.8 here), 75 us a KV group
+// for 256 queries over 560 keys (14.2 here for 15 heads of 5 groups).  Bound by each workgroup's chain
+// of loads, barriers and dependent MFMA / VALU steps, so the LDS is kept to 37 KiB (four workgroups a
+// unit) and the K rows and the first V rows are loaded ahead of their use (18.6 and 16.3 us without).
 //
 // A workgroup takes 16 queries of one (sequence, head) pair and its 4 wavefronts the keys: wave w
 // the 64-key steps w, w + 4, .. (at most NS), so that few queries still fill the chip and a lane's
@@ -405,21 +426,14 @@ int run_attention(const int16_t* qkv, int16_t* o, uint32_t batch, uint32_t seq, 
 // sums of o are added in LDS (the wrapped sum is one mod 2^32, so the order is free).  All offset
 // terms come from MFMAs against ones: sum_j P V = 2^16 HH + 2^8 MID + LL + 2^15 sum h_V + 2^7 sum l_V
 // + 128 sum P over every 64-key step, keys past the end taken as V = P = 0.
-struct AttnPairs {
-    const int16_t *q, *k, *v;
-    int16_t* o;
-    uint64_t q_ld, q_ds, q_bs, q_bs2, k_ld, k_bs, k_bs2, v_ld, v_bs, v_bs2, o_ld, o_bs, o_bs2;
-    uint32_t keys, inner, valid0, period, cm, cfg, dlim;
-    uint32_t p_rows, p_heads;                // plane row / head of an outer step (pair / inner)
-};
 constexpr uint32_t kVs = 80;                 // V^T plane row stride in bytes (64 keys, rows 20 banks apart)
 constexpr uint32_t kOs = 68;                 // partial o row stride in dwords
 
 template <uint32_t NS>
-__global__ __launch_bounds__(256, 2) void attention_pairs_kernel(AttnPairs a, const int32_t* __restrict__ tab,
+__global__ __launch_bounds__(256, NS == 1 ? 4 : 2) void attention_pairs_kernel(AttnPairs a, const int32_t* __restrict__ tab,
                                                                  APlanes po) {
     __shared__ __attribute__((aligned(16))) int32_t stab[4096];
-    __shared__ __attribute__((aligned(16))) uint8_t vt[4][2 * kHd * kVs];          // [wave][hi, lo][64 d][kVs]
+    __shared__ __attribute__((aligned(16))) uint8_t vt[4][kHd * kVs];              // [wave][hi, lo][32 d][kVs]
     __shared__ int32_t redm[4][16], reds[4][16];
     const uint32_t t = threadIdx.x, lane = t & 63, c16 = lane & 15, g = lane >> 4;
     const uint32_t w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -457,24 +471,29 @@ __global__ __launch_bounds__(256, 2) void attention_pairs_kernel(AttnPairs a, co
     const v4i c20 = {1 << 20, 1 << 20, 1 << 20, 1 << 20};
     const v4i qh1 = mfma(ones, qh, zero), ql1 = mfma(ones, ql, zero);
 
-    // ---- phase 1: the scores of the wave's steps; the unread ones stay below every score
+    // ---- phase 1: the scores of the wave's steps, every step's K rows loaded before the first is used
     int32_t sv[16 * NS];
+    int4 kx[NS][4][2];
 #pragma unroll
     for (uint32_t s = 0; s < NS; s++) {
         const uint32_t k0 = 64 * (w + 4 * s);
         if (k0 < kend) {
-            int4 x[4][2];
 #pragma unroll
             for (uint32_t kb = 0; kb < 4; kb++) {
                 const int16_t* kr = kp + (uint64_t)min(k0 + 16 * kb + c16, a.keys - 1) * a.k_ld;
-                x[kb][0] = *reinterpret_cast<const int4*>(kr);
-                x[kb][1] = *reinterpret_cast<const int4*>(kr + 8);
+                kx[s][kb][0] = *reinterpret_cast<const int4*>(kr);
+                kx[s][kb][1] = *reinterpret_cast<const int4*>(kr + 8);
             }
+        }
+    }
+#pragma unroll
+    for (uint32_t s = 0; s < NS; s++) {
+        if (64 * (w + 4 * s) < kend) {
 #pragma unroll
             for (uint32_t kb = 0; kb < 4; kb++) {
                 uint32_t h0, h1, h2, h3, l0, l1, l2, l3;
-                limbs8(x[kb][0], h0, h1, l0, l1);
-                limbs8(x[kb][1], h2, h3, l2, l3);
+                limbs8(kx[s][kb][0], h0, h1, l0, l1);
+                limbs8(kx[s][kb][1], h2, h3, l2, l3);
                 const v4i kh = {(int)h0, (int)h1, (int)h2, (int)h3}, kl = {(int)l0, (int)l1, (int)l2, (int)l3};
                 const v4i hh = mfma(kh, qh, zero);
                 v4i mid = mfma(kh, ql, zero);
@@ -493,6 +512,21 @@ __global__ __launch_bounds__(256, 2) void attention_pairs_kernel(AttnPairs a, co
             for (uint32_t n = 0; n < 16; n++) sv[16 * s + n] = 0;
         }
     }
+    // V^T goes through the wave's tile 32 d at a time: half u % 2 of step u / 2.  A lane's task is 4 keys
+    // (4 qd ..) x 8 d (8 c ..); the next half's rows are loaded while this one's are used, the first
+    // half's here, under the softmax.
+    const uint32_t c = lane & 3, qd = lane >> 2;
+    int4 vx[4];
+    auto load_v = [&](uint32_t u) {
+        const uint32_t key = 64 * (w + 4 * (u >> 1)) + 4 * qd;             // keys is a multiple of 16
+        const int16_t* vr = vp + (uint64_t)(key < a.keys ? key : 0) * a.v_ld + 32 * (u & 1) + 8 * c;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) {
+            vx[r] = *reinterpret_cast<const int4*>(vr + r * a.v_ld);
+            if (key >= a.keys) vx[r] = make_int4(0, 0, 0, 0);
+        }
+    };
+    if (64 * w < kend) load_v(0);
 
     // ---- phase 2: the softmax over the valid keys of the lane's query
     auto key_of = [&](uint32_t s, uint32_t n) { return 64 * (w + 4 * s) + 16 * (n >> 2) + 4 * g + (n & 3); };
@@ -539,49 +573,13 @@ __global__ __launch_bounds__(256, 2) void attention_pairs_kernel(AttnPairs a, co
 
     // ---- phase 3: the wave's part of o^T[d][qi], 4 blocks of 16 d
     uint8_t* vth = vt[w];
-    uint8_t* vtl = vth + kHd * kVs;
+    uint8_t* vtl = vth + 32 * kVs;
     v4i ohh[4], omid[4], oll[4], oha[4], ola[4];
 #pragma unroll
     for (uint32_t m = 0; m < 4; m++) ohh[m] = omid[m] = oll[m] = oha[m] = ola[m] = zero;
 #pragma unroll
     for (uint32_t s = 0; s < NS; s++) {
-        const uint32_t k0 = 64 * (w + 4 * s);
-        if (k0 >= kend) break;
-        // V^T of the step: a task is 4 keys (4 qd ..) x 8 d (8 c ..)
-        const uint32_t c = lane & 7;
-        int4 x[2][4];
-#pragma unroll
-        for (uint32_t it = 0; it < 2; it++) {
-            const uint32_t key = k0 + 4 * ((lane >> 3) + 8 * it);          // keys is a multiple of 16
-            const int16_t* vr = vp + (uint64_t)(key < a.keys ? key : 0) * a.v_ld + 8 * c;
-#pragma unroll
-            for (uint32_t r = 0; r < 4; r++) {
-                x[it][r] = *reinterpret_cast<const int4*>(vr + r * a.v_ld);
-                if (key >= a.keys) x[it][r] = make_int4(0, 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (uint32_t it = 0; it < 2; it++) {
-            const uint32_t qd = (lane >> 3) + 8 * it, p0 = 16 * (qd & 3) + 4 * (qd >> 2);
-#pragma unroll
-            for (uint32_t q = 0; q < 4; q++) {
-                const uint32_t a0 = dword(x[it][0], q), a1 = dword(x[it][1], q), a2 = dword(x[it][2], q), a3 = dword(x[it][3], q);
-                const uint32_t th01 = __builtin_amdgcn_perm(a1, a0, 0x07030501u);
-                const uint32_t th23 = __builtin_amdgcn_perm(a3, a2, 0x07030501u);
-                const uint32_t tl01 = __builtin_amdgcn_perm(a1, a0, 0x06020400u);
-                const uint32_t tl23 = __builtin_amdgcn_perm(a3, a2, 0x06020400u);
-                const uint32_t d0 = 8 * c + 2 * q;
-                *reinterpret_cast<uint32_t*>(vth + d0 * kVs + p0) = __builtin_amdgcn_perm(th23, th01, 0x05040100u);
-                *reinterpret_cast<uint32_t*>(vth + (d0 + 1) * kVs + p0) = __builtin_amdgcn_perm(th23, th01, 0x07060302u);
-                *reinterpret_cast<uint32_t*>(vtl + d0 * kVs + p0) = __builtin_amdgcn_perm(tl23, tl01, 0x05040100u) ^ 0x80808080u;
-                *reinterpret_cast<uint32_t*>(vtl + (d0 + 1) * kVs + p0) =
-                    __builtin_amdgcn_perm(tl23, tl01, 0x07060302u) ^ 0x80808080u;
-            }
-        }
-        // the tile is the wave's own: LDS operations of a wave complete in order
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        if (64 * (w + 4 * s) >= kend) break;
         uint32_t ph[4], pl[4];
 #pragma unroll
         for (uint32_t q = 0; q < 4; q++) {
@@ -594,20 +592,44 @@ __global__ __launch_bounds__(256, 2) void attention_pairs_kernel(AttnPairs a, co
         const v4i bh4 = {(int)ph[0], (int)ph[1], (int)ph[2], (int)ph[3]};
         const v4i bl4 = {(int)pl[0], (int)pl[1], (int)pl[2], (int)pl[3]};
 #pragma unroll
-        for (uint32_t m = 0; m < 4; m++) {
-            const uint32_t off = (16 * m + c16) * kVs + 16 * g;
-            const v4i vh = *reinterpret_cast<const v4i*>(vth + off);
-            const v4i vl = *reinterpret_cast<const v4i*>(vtl + off);
-            ohh[m] = mfma(vh, bh4, ohh[m]);
-            omid[m] = mfma(vh, bl4, omid[m]);
-            oha[m] = mfma(vh, ones, oha[m]);
-            omid[m] = mfma(vl, bh4, omid[m]);
-            oll[m] = mfma(vl, bl4, oll[m]);
-            ola[m] = mfma(vl, ones, ola[m]);
+        for (uint32_t half = 0; half < 2; half++) {
+            const uint32_t p0 = 16 * (qd & 3) + 4 * (qd >> 2);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++) {
+                const uint32_t a0 = dword(vx[0], q), a1 = dword(vx[1], q), a2 = dword(vx[2], q), a3 = dword(vx[3], q);
+                const uint32_t th01 = __builtin_amdgcn_perm(a1, a0, 0x07030501u);
+                const uint32_t th23 = __builtin_amdgcn_perm(a3, a2, 0x07030501u);
+                const uint32_t tl01 = __builtin_amdgcn_perm(a1, a0, 0x06020400u);
+                const uint32_t tl23 = __builtin_amdgcn_perm(a3, a2, 0x06020400u);
+                const uint32_t d0 = 8 * c + 2 * q;
+                *reinterpret_cast<uint32_t*>(vth + d0 * kVs + p0) = __builtin_amdgcn_perm(th23, th01, 0x05040100u);
+                *reinterpret_cast<uint32_t*>(vth + (d0 + 1) * kVs + p0) = __builtin_amdgcn_perm(th23, th01, 0x07060302u);
+                *reinterpret_cast<uint32_t*>(vtl + d0 * kVs + p0) = __builtin_amdgcn_perm(tl23, tl01, 0x05040100u) ^ 0x80808080u;
+                *reinterpret_cast<uint32_t*>(vtl + (d0 + 1) * kVs + p0) =
+                    __builtin_amdgcn_perm(tl23, tl01, 0x07060302u) ^ 0x80808080u;
+            }
+            const uint32_t next = 2 * s + half + 1;
+            if (next < 2 * NS && 64 * (w + 4 * (next >> 1)) < kend) load_v(next);
+            // the tile is the wave's own: LDS operations of a wave complete in order
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+#pragma unroll
+            for (uint32_t mh = 0; mh < 2; mh++) {
+                const uint32_t off = (16 * mh + c16) * kVs + 16 * g, m = 2 * half + mh;
+                const v4i vh = *reinterpret_cast<const v4i*>(vth + off);
+                const v4i vl = *reinterpret_cast<const v4i*>(vtl + off);
+                ohh[m] = mfma(vh, bh4, ohh[m]);
+                omid[m] = mfma(vh, bl4, omid[m]);
+                oha[m] = mfma(vh, ones, oha[m]);
+                omid[m] = mfma(vl, bh4, omid[m]);
+                oll[m] = mfma(vl, bl4, oll[m]);
+                ola[m] = mfma(vl, ones, ola[m]);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
     }
     // the wave's partials [query][d] over its own V^T tile (every read of it done)
     int32_t* pw = reinterpret_cast<int32_t*>(vt[w]);
