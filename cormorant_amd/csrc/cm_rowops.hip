@@ -180,8 +180,9 @@ __device__ __forceinline__ void stage_params(uint4* lds, const uint8_t* params, 
 }
 
 // COPY / ADDX parameters as the element loop uses them, one 16-byte entry per column: the
-// three shifts and two fast-path flags in one word (sa | sb << 8 | sc << 16; bit 24: every
-// term within the 64-bit bounds with a 32-bit B, bit 25: with a 16-bit B), G, and
+// three shifts and the fast-path flags in one word (sa | sb << 8 | sc << 16; bit 24: every
+// term within the 64-bit bounds with a 32-bit B, bit 25: with a 16-bit B, bit 26: x + (y << sb) + bias
+// with (y << sb) + bias exact in int32 for a 16-bit B), G, and
 // Bq 2^bq_sh + 2^(sc - 1) (the bias with the rounding half folded in; 0 when bq_sh > 40, a
 // job the 128-bit path takes whole).
 template <uint32_t BATCH = 1>
@@ -193,7 +194,8 @@ __device__ __forceinline__ void stage_addx_params(uint4* lds, const uint8_t* par
         const uint32_t w = (uint32_t)q.sa | ((uint32_t)q.sb << 8) | ((uint32_t)q.sc << 16) |
                            ((base && q.sb <= 30) ? 1u << 24 : 0u) | ((base && q.sb <= 46) ? 1u << 25 : 0u);
         const u64 bs = bq_sh <= 40 ? (u64)(q.bq * ((i64)1 << bq_sh) + norm_half((uint32_t)q.sc)) : 0;
-        lds[pslot(i, units)] = make_uint4(w, (uint32_t)q.g, (uint32_t)bs, (uint32_t)(bs >> 32));
+        const bool plain = bq_sh <= 40 && q.sa == 0 && q.sc == 0 && q.sb <= 15 && bs + (1u << 30) < (1ull << 31);
+        lds[pslot(i, units)] = make_uint4(w | (plain ? 1u << 26 : 0u), (uint32_t)q.g, (uint32_t)bs, (uint32_t)(bs >> 32));
     });
 }
 
@@ -212,11 +214,30 @@ __device__ __forceinline__ void addx_unit_wide(const int (&x)[8], const int (&y)
 // One COPY / ADDX unit from the staged entries (stage_addx_params): 64-bit arithmetic where
 // every term stays below 2^61 (x << sa <= 2^61, y << sb, Bq << bq_sh <= 2^61), round half to even
 // as one shift and an exact-tie test; else the 128-bit form (a branch taken by the lanes that
-// need it).
+// need it).  The residual add itself (int32 out, no shift of x or of the sum: `plain` entries, a
+// uniform branch) is one shift, one add and one saturating add.
 template <int BK, int CK, bool BEN>
 __device__ __forceinline__ void addx_unit(const int (&x)[8], const int (&y)[8], uint32_t u, uint32_t units,
                                           const Job& j, const uint4* ro_lds, const uint8_t* praw, bool bcast,
                                           bool scale, bool relu, int (&r)[8]) {
+    if constexpr (BK == 0 && CK == 1) {
+        uint32_t all = 1u << 26;
+        uint4 e[8];
+#pragma unroll
+        for (int l = 0; l < 8; l++) {
+            e[l] = ro_lds[bcast ? 0u : l * units + u];
+            all &= e[l].x;
+        }
+        if (__all(all != 0) && !scale) {
+#pragma unroll
+            for (int l = 0; l < 8; l++) {
+                const int t = (BEN ? (int)((uint32_t)y[l] << ((e[l].x >> 8) & 15)) : 0) + (int)e[l].z;
+                r[l] = __builtin_elementwise_add_sat(x[l], t);
+                if (relu) r[l] = max(r[l], 0);
+            }
+            return;
+        }
+    }
     bool wide = scale || j.bq_sh > 40;
 #pragma unroll
     for (int l = 0; l < 8; l++) {
@@ -247,9 +268,9 @@ __device__ __forceinline__ void addx_unit(const int (&x)[8], const int (&y)[8], 
 template <int UPL, bool PL>
 __device__ __forceinline__ void norm_row(const Job& j, const int (&x)[UPL][8], uint8_t* rc, const uint4* ro_lds,
                                          bool bcast, const uint8_t* tab, uint32_t lane, uint32_t units, bool ln,
-                                         const APlanes& po, u64 prow) {
+                                         bool high, const APlanes& po, u64 prow) {
     int4 o[UPL];
-    norm_row_vals<UPL>(j.n, j.eps, x, ro_lds, bcast, tab, lane, units, ln, o);
+    norm_row_vals<UPL>(j.n, j.eps, x, ro_lds, bcast, tab, lane, units, ln, high, o);
     int32_t ps[UPL];
 #pragma unroll
     for (int k = 0; k < UPL; k++) {
@@ -322,6 +343,7 @@ __global__ __launch_bounds__(64 * NW) void ro_norm_fast_kernel(Job j, const uint
     }
     stage_norm_params(ro_lds, params, nsl, units, j.bq_sh);
     __syncthreads();
+    const bool high = norm_shift_high<UPL>(ro_lds, bcast, lane, 64, units);
     const bool scale = (ja.op & F_SCALE) != 0, relu = (ja.op & F_RELU) != 0;
     for (; row < rows; row += stride) {
         const uint32_t i1 = (uint32_t)(row % j.c1), i2 = (uint32_t)(row / j.c1);
@@ -344,8 +366,7 @@ __global__ __launch_bounds__(64 * NW) void ro_norm_fast_kernel(Job j, const uint
             }
         }
         norm_row<UPL, PL>(j, x, j.c != nullptr ? j.c + (u64)i2 * j.c_s2 + (u64)i1 * j.c_s1 : nullptr, ro_lds, bcast, tab,
-                          lane, units, ln, po,
-                          row);
+                          lane, units, ln, high, po, row);
         if (row + stride < rows) load_row(row + stride);
     }
 }
@@ -417,6 +438,7 @@ __global__ __launch_bounds__(TPR) void ro_norm_wg_kernel(Job j, const uint8_t* _
     }
     const bool scale = (ja.op & F_SCALE) != 0, relu = (ja.op & F_RELU) != 0;
     const uint32_t nslab = min(po.nsum, (units + 127) / 128);
+    bool high = false;                                   // norm_shift_high, once the entries are staged
     for (uint32_t it = 0; row < rows; row += gridDim.x, it++) {
         const uint32_t i1 = (uint32_t)(row % j.c1), i2 = (uint32_t)(row / j.c1);
         if constexpr (ADDX) {
@@ -434,8 +456,7 @@ __global__ __launch_bounds__(TPR) void ro_norm_wg_kernel(Job j, const uint8_t* _
                 for (int l = 0; l < 8; l++) x[k][l] = r[l];
             }
         }
-        NormSums ts = norm_sums<UPL>(x);
-        norm_sums_wave(ts);
+        NormSums ts = norm_sums_of_wave<UPL>(x);
         if constexpr (SELF) {
             if (it == 0) {
 #pragma unroll
@@ -451,6 +472,7 @@ __global__ __launch_bounds__(TPR) void ro_norm_wg_kernel(Job j, const uint8_t* _
                 }
             }
         }
+        if (it == 0) high = norm_shift_high<UPL>(ro_lds, bcast, t, TPR, units);
         NormSums* ws = wsum[it & 1];                     // alternate: a row's reads end before the next's writes
         if (lane == 0) ws[wave] = ts;
         __syncthreads();
@@ -458,7 +480,7 @@ __global__ __launch_bounds__(TPR) void ro_norm_wg_kernel(Job j, const uint8_t* _
 #pragma unroll
         for (int w = 1; w < NWV; w++) norm_sums_add(ts, ws[w]);
         int4 o[UPL];
-        norm_row_finish<UPL>(j.n, j.eps, ts, x, ro_lds, bcast, tab, t, TPR, units, ln, o);
+        norm_row_finish<UPL>(j.n, j.eps, ts, x, ro_lds, bcast, tab, t, TPR, units, ln, high, o);
         uint8_t* rc = j.c != nullptr ? j.c + (u64)i2 * j.c_s2 + (u64)i1 * j.c_s1 : nullptr;   // null: planes alone
 #pragma unroll
         for (int k = 0; k < UPL; k++) {

@@ -304,18 +304,113 @@ __device__ __forceinline__ void norm_sums_wave(NormSums& t) {
     }
 }
 
+// x of the lane's neighbour in step `i` of a sum over the 16 lanes of a DPP row (quad_perm [1,0,3,2],
+// quad_perm [2,3,0,1], row_half_mirror, row_mirror).
+template <int I>
+__device__ __forceinline__ uint32_t row16_step(uint32_t x) {
+    constexpr int ctrl = I == 0 ? 0xB1 : I == 1 ? 0x4E : I == 2 ? 0x141 : 0x140;
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, 0xF, 0xF, false);
+}
+
+// A value of |x| for which the short sums hold: a lane's 8 UPL elements over 16 lanes in int32, the
+// squares in 64 bits, and 24-bit products n x (n <= 4096).
+template <int UPL>
+constexpr uint32_t kNormShort = 1u << (UPL == 1 ? 23 : UPL == 2 ? 23 : 21);
+
+// The wavefront's sums (norm_sums, then norm_sums_wave).  Where every |x| is below kNormShort (the
+// residual stream at 2^-15: |value| < 256) a lane adds its elements in int32 and their squares in one
+// 64-bit multiply-add each, the 16 lanes of a row meet over DPP and the four rows in scalar registers,
+// instead of 128-bit carries and seven LDS shuffles a step.
+template <int UPL>
+__device__ __forceinline__ NormSums norm_sums_of_wave(const int (&x)[UPL][8]) {
+    static_assert(UPL <= 8, "kNormShort");
+    int mx = 0, mn = 0;
+#pragma unroll
+    for (int k = 0; k < UPL; k++)
+#pragma unroll
+        for (int l = 0; l < 8; l++) {
+            mx = max(mx, x[k][l]);
+            mn = min(mn, x[k][l]);
+        }
+    uint32_t am = max((uint32_t)mx, 0u - (uint32_t)mn);
+    am = max(am, row16_step<0>(am));
+    am = max(am, row16_step<1>(am));
+    am = max(am, row16_step<2>(am));
+    am = max(am, row16_step<3>(am));
+    auto row = [](uint32_t v, int r) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 16 * r); };
+    const uint32_t amax = max(max(row(am, 0), row(am, 1)), max(row(am, 2), row(am, 3)));
+    if (amax >= kNormShort<UPL>) {
+        NormSums t = norm_sums<UPL>(x);
+        norm_sums_wave(t);
+        return t;
+    }
+    int s1 = 0;
+    u64 s2 = 0;
+#pragma unroll
+    for (int k = 0; k < UPL; k++)
+#pragma unroll
+        for (int l = 0; l < 8; l++) {
+            s1 += x[k][l];
+            s2 += (u64)((i64)x[k][l] * x[k][l]);
+        }
+    auto add = [&](uint32_t d1, uint32_t lo, uint32_t hi) {
+        s1 += (int)d1;
+        s2 += ((u64)hi << 32) | lo;
+    };
+    add(row16_step<0>(s1), row16_step<0>((uint32_t)s2), row16_step<0>((uint32_t)(s2 >> 32)));
+    add(row16_step<1>(s1), row16_step<1>((uint32_t)s2), row16_step<1>((uint32_t)(s2 >> 32)));
+    add(row16_step<2>(s1), row16_step<2>((uint32_t)s2), row16_step<2>((uint32_t)(s2 >> 32)));
+    add(row16_step<3>(s1), row16_step<3>((uint32_t)s2), row16_step<3>((uint32_t)(s2 >> 32)));
+    NormSums t{0, 0, 0, amax};
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        t.s1 += (int)row((uint32_t)s1, r);
+        t.lo += ((u64)row((uint32_t)(s2 >> 32), r) << 32) | row((uint32_t)s2, r);
+    }
+    return t;
+}
+
+// Whether every column of the lanes' units u0 + ustride k has its shift in 33 .. 61, wavefront-uniform:
+// norm_row_finish then takes the result from the high word of the 64-bit value.
+template <int UPL>
+__device__ __forceinline__ bool norm_shift_high(const uint4* lds, bool bcast, uint32_t u0, uint32_t ustride,
+                                                uint32_t units) {
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < UPL; k++) {
+        const uint32_t u = u0 + ustride * k;
+        if (u >= units) continue;
+#pragma unroll
+        for (int l = 0; l < 8; l++) {
+            const uint32_t sc = lds[bcast ? 0u : l * units + u].y;
+            ok = ok && sc >= 33 && sc <= 61;
+        }
+    }
+    return __all(ok);
+}
+
+__device__ __forceinline__ u64 uniform64(u64 v) {
+    return ((u64)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
 // The int16 results of a NORM row (n elements, eps, LN or RMS) of the fast path from the row's
 // sums t: x[k] = unit u0 + ustride k of the row (int32, zero past the row), the parameters
 // staged by stage_norm_params at lds; 64-bit arithmetic where every element's bounds allow, the
 // lanes' units in 128 bits otherwise (a branch uniform over the wavefront; both give the exact
-// values).
+// values).  `t` is the same in every lane: the row's scale is computed in scalar registers.  With `high`
+// (norm_shift_high) an element is about 12 instructions: P1 = (A Rm) >> shp from the product's high
+// word, one 64-bit multiply-add by G and the bias, the shift and the clamp in 32 bits; at 24576 x 768
+// with the residual add the launch goes from 73 us (bound by its 64-bit shifts, compares and shuffles)
+// to 54 (226 MB, 4.2 TB/s).
 template <int UPL>
 __device__ __forceinline__ void norm_row_finish(uint32_t n, i64 eps, const NormSums& t, const int (&x)[UPL][8],
                                                 const uint4* ro_lds, bool bcast, const uint8_t* tab, uint32_t u0,
-                                                uint32_t ustride, uint32_t units, bool ln, int4 (&o)[UPL]) {
-    const i64 s1 = t.s1;
-    const uint32_t amax = t.amax;
-    const i128 S1 = s1, S2 = (i128)(((unsigned __int128)t.hi << 64) | t.lo);
+                                                uint32_t ustride, uint32_t units, bool ln, bool high,
+                                                int4 (&o)[UPL]) {
+    const i64 s1 = (i64)uniform64((u64)t.s1);
+    const uint32_t amax = (uint32_t)__builtin_amdgcn_readfirstlane((int)t.amax);
+    const i128 S1 = s1, S2 = (i128)(((unsigned __int128)uniform64(t.hi) << 64) | uniform64(t.lo));
     i128 D = ln ? ((i128)n * S2 - S1 * S1 + (i128)eps) : (S2 + (i128)eps);
     if (D <= 0) D = 1;
     u64 Rm;
@@ -328,6 +423,35 @@ __device__ __forceinline__ void norm_row_finish(uint32_t n, i64 eps, const NormS
     const bool a32 = abound < ((u64)1 << 31) && ((abound * Rm) >> shp) < ((u64)1 << 31) - 2;
     bool wide = !a32;
     const int32_t rm_lo = (int32_t)(uint32_t)Rm;     // Rm - 2^32: Rm lies in [2^31, 2^32)
+    if (a32 && high) {
+        const bool small = amax < kNormShort<1>;     // n x in 24-bit factors (n <= 4096)
+#pragma unroll
+        for (int k = 0; k < UPL; k++) {
+            const uint32_t u = u0 + ustride * k;
+            o[k] = make_int4(0, 0, 0, 0);
+            if (u >= units) continue;
+            int r[8];
+#pragma unroll
+            for (int l = 0; l < 8; l++) {
+                const uint4 e = ro_lds[bcast ? 0u : l * units + u];
+                const int32_t nx = small ? __mul24((int)n, x[k][l]) : (int32_t)(n * (uint32_t)x[k][l]);
+                const int32_t A = ln ? (int32_t)((uint32_t)nx - (uint32_t)s1) : x[k][l];
+                // A Rm in two words, its high word floor(A Rm / 2^32)
+                const int32_t ph = __mulhi(A, rm_lo) + A;
+                const int32_t P1 = shp >= 32 ? ph >> min(shp - 32, 31)
+                                             : (int32_t)__builtin_amdgcn_alignbit((uint32_t)ph, (uint32_t)A * (uint32_t)rm_lo,
+                                                                                  (uint32_t)shp);
+                const u64 w = (u64)((i64)P1 * (int32_t)e.x) + (((u64)e.w << 32) | e.z);
+                const uint32_t sc = e.y, wh = (uint32_t)(w >> 32);
+                // round half to even as below: the low sc bits all zero is a tie
+                const bool tie = ((wh << (64 - sc)) | (uint32_t)w) == 0;
+                const int32_t v = ((int32_t)wh >> (sc - 32)) & (tie ? ~1 : ~0);
+                r[l] = min(max(v, -32768), 32767);
+            }
+            o[k] = pack16(r);
+        }
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < UPL; k++) {
         const uint32_t u = u0 + ustride * k;
@@ -369,10 +493,9 @@ __device__ __forceinline__ void norm_row_finish(uint32_t n, i64 eps, const NormS
 template <int UPL>
 __device__ __forceinline__ void norm_row_vals(uint32_t n, i64 eps, const int (&x)[UPL][8], const uint4* ro_lds,
                                               bool bcast, const uint8_t* tab, uint32_t lane, uint32_t units, bool ln,
-                                              int4 (&o)[UPL]) {
-    NormSums t = norm_sums<UPL>(x);
-    norm_sums_wave(t);
-    norm_row_finish<UPL>(n, eps, t, x, ro_lds, bcast, tab, lane, 64, units, ln, o);
+                                              bool high, int4 (&o)[UPL]) {
+    const NormSums t = norm_sums_of_wave<UPL>(x);
+    norm_row_finish<UPL>(n, eps, t, x, ro_lds, bcast, tab, lane, 64, units, ln, high, o);
 }
 
 }  // namespace ro
