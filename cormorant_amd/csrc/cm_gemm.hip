@@ -1347,6 +1347,154 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_ring_kernel(
 #undef CM_STORE
 }
 
+// ---------------------------------------------------------------- 1x1 convolutions, input split in the GEMM
+// A 1x1 stride-1 convolution is the product of the weights' planes and each image's [channels][pixels]
+// matrix.  Folding the images into byte planes first (split_fold*) writes and reads the whole input
+// again and costs a launch of 5 - 15 us; here a workgroup of 4 waves (64 x 64 outputs, 32 x 32 a wave)
+// splits its own 64 channels x 64 pixels a step: a thread loads 4 channels x 4 pixels (8-byte loads at
+// any alignment), transposes them with byte permutes into one dword of 4 channels a pixel and plane,
+// and adds the pixel's byte sums (v_dot4) on the way.  Every operand comes through registers, D steps
+// ahead (the pixels of a step are 64 rows a plane apart in HBM: a load at its use costs 2 - 3 us a
+// step), into two LDS buffers with one LDS-only barrier a step.  Pixel rows are 80 bytes (20 banks)
+// apart, so the fragment reads of 16 rows meet no conflict.  The input is split again for every row
+// tile, so it pays while the output rows are few tiles or the steps few (conv_direct).
+constexpr uint32_t kDbp = 80;                    // bytes of a pixel row of a staged B plane
+constexpr int DT = 64;                           // tile rows and columns
+
+template <class Epi>
+__global__ __launch_bounds__(256, 3) void conv_direct_kernel(
+    const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
+    uint32_t a_lines, uint32_t nsum_a, const int16_t* __restrict__ x, uint64_t x_img, uint32_t K,
+    uint32_t plane, uint32_t tiles_r, uint32_t tiles_c, uint32_t batch, uint32_t kp, int32_t k64, uint32_t mode, Epi epi) {
+    constexpr int A_T = DT * BK, B_T = DT * kDbp, BUF = 2 * A_T + 2 * B_T;
+    constexpr int D = 2;                               // steps ahead (3 and 4 measured the same)
+    __shared__ __attribute__((aligned(16))) int8_t buf[2][BUF];        // Ah, Al [64][64], Bh, Bl [64][kDbp]
+    __shared__ int2 rterm[DT], cterm[DT];              // (h, l) halves
+    __shared__ int32_t csum[DT];
+
+    // the row tiles of one pixel tile run on one XCD, one after the other (its L2 holds the pixels)
+    const TilePos tp = tile_pos(blockIdx.x, tiles_r, tiles_c * batch, 1);
+    const uint32_t tr = tp.tr, img = tp.tc / tiles_c, tc = tp.tc - img * tiles_c;
+    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const uint32_t wr = wave >> 1, wc = wave & 1, l32 = lane & 31, lh = lane >> 5;
+    const uint32_t nk = kp / BK, col0 = tc * DT;
+
+    // A: thread (row t / 4, 16-byte chunk t % 4) of each plane; B: channels 4 kg .., pixels 4 pg ..
+    const uint32_t arow = t >> 2, achunk = t & 3, adst = arow * BK + (achunk ^ ((arow >> 2) & 3)) * 16;
+    const uint64_t aoff = ((uint64_t)tr * DT + arow) * kp + achunk * 16;
+    const uint32_t pg = lane & 15, kg = 4 * wave + (lane >> 4);
+    // a group past the plane's end reads the plane's last 4 pixels, shifted to their places (plane >= 4)
+    const uint32_t px = min(col0 + 4 * pg, plane - 4), over = min(col0 + 4 * pg - px, 3u) * 16;
+    const bool ragged = (plane & 3) != 0 && col0 + DT > plane;         // uniform: some group needs the shift
+    const int16_t* xp = x + img * x_img + px;
+    struct Step { int4 ah, al; uint64_t b[4]; };
+    auto load = [&](Step& v, uint32_t step) {
+        v.ah = *reinterpret_cast<const int4*>(Ahi + aoff + step * BK);
+        v.al = *reinterpret_cast<const int4*>(Alo + aoff + step * BK);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            __builtin_memcpy(&v.b[r], xp + (uint64_t)min(step * BK + 4 * kg + r, K - 1) * plane, 8);
+    };
+    int32_t sh[4] = {0, 0, 0, 0}, sl[4] = {0, 0, 0, 0};
+    auto store = [&](int8_t* sm, Step& v, uint32_t step) {
+        *reinterpret_cast<int4*>(sm + adst) = v.ah;
+        *reinterpret_cast<int4*>(sm + A_T + adst) = v.al;
+        if (ragged) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) v.b[r] >>= over;
+        }
+        if ((step + 1) * BK > K) {                     // uniform: channels past K are padding (bytes 0, 0)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (step * BK + 4 * kg + r >= K) v.b[r] = 0x0080008000800080ull;
+        }
+        int8_t* p = sm + 2 * A_T + 4 * pg * kDbp + 4 * kg;
+#pragma unroll
+        for (int c2 = 0; c2 < 2; c2++) {
+            const uint32_t d0 = (uint32_t)(v.b[0] >> (32 * c2)), d1 = (uint32_t)(v.b[1] >> (32 * c2)),
+                           d2 = (uint32_t)(v.b[2] >> (32 * c2)), d3 = (uint32_t)(v.b[3] >> (32 * c2));
+            const uint32_t xh = __builtin_amdgcn_perm(d1, d0, 0x07030501u), yh = __builtin_amdgcn_perm(d3, d2, 0x07030501u);
+            const uint32_t xl = __builtin_amdgcn_perm(d1, d0, 0x06020400u), yl = __builtin_amdgcn_perm(d3, d2, 0x06020400u);
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const uint32_t sel = e ? 0x07060302u : 0x05040100u;
+                const int h = (int)__builtin_amdgcn_perm(yh, xh, sel), l = (int)(__builtin_amdgcn_perm(yl, xl, sel) ^ 0x80808080u);
+                sh[2 * c2 + e] = __builtin_amdgcn_sdot4(h, 0x01010101, sh[2 * c2 + e], false);
+                sl[2 * c2 + e] = __builtin_amdgcn_sdot4(l, 0x01010101, sl[2 * c2 + e], false);
+                *reinterpret_cast<int*>(p + (2 * c2 + e) * kDbp) = h;
+                *reinterpret_cast<int*>(p + (2 * c2 + e) * kDbp + B_T) = l;
+            }
+        }
+    };
+    Step v[D];
+#pragma unroll
+    for (int i = 0; i < D; i++)
+        if (i == 0 || (uint32_t)i < nk) load(v[i], i);
+    if (t < (uint32_t)DT) {                            // the rows' terms (the weights' sums and the bias)
+        const uint32_t line = tr * DT + t;
+        int32_t sum = 0;
+        for (uint32_t s = 0; s < nsum_a; s++) sum += rpart[(uint64_t)s * a_lines + line];
+        rterm[t] = make_int2(epi.row_bias(line) - k64 + (sum >> 1), (sum & 1) << 7);
+        csum[t] = (int32_t)(128 * K);                  // x = 256 h + l + 128
+    }
+
+    const uint32_t sw = (l32 >> 2) & 3;
+    const uint32_t fa = (wr * 32 + l32) * BK, fb = 2 * A_T + (wc * 32 + l32) * kDbp + lh * 16;
+    const uint32_t ch[2] = {((0 + lh) ^ sw) * 16, ((2 + lh) ^ sw) * 16};
+    v16i hh[1][1] = {{v16i{}}}, mid[1][1] = {{v16i{}}}, ll[1][1] = {{v16i{}}};
+    for (uint32_t kt = 0; kt < nk;) {
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            int8_t* sm = buf[i];
+            store(sm, v[i], kt);
+            if (kt + D < nk) load(v[i], kt + D);
+            lds_barrier();                             // this buffer's readers of two steps ago passed the last one
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const v4i ah = *reinterpret_cast<const v4i*>(sm + fa + ch[s]);
+                const v4i al = *reinterpret_cast<const v4i*>(sm + A_T + fa + ch[s]);
+                const v4i bh = *reinterpret_cast<const v4i*>(sm + fb + s * 32);
+                const v4i bl = *reinterpret_cast<const v4i*>(sm + fb + B_T + s * 32);
+                hh[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah, bh, hh[0][0], 0, 0, 0);
+                mid[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah, bl, mid[0][0], 0, 0, 0);
+                ll[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al, bl, ll[0][0], 0, 0, 0);
+                mid[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al, bh, mid[0][0], 0, 0, 0);
+            }
+            if (++kt >= nk) break;
+        }
+    }
+    // the pixels' sums: over the four lanes kg of a wave, then the waves
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        int32_t s = (sh[q] << 8) + sl[q];
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        if (lane < 16) atomicAdd(&csum[4 * pg + q], s);
+    }
+    __syncthreads();
+    if (t < (uint32_t)DT) cterm[t] = make_int2(csum[t] >> 1, (csum[t] & 1) << 7);
+    __syncthreads();
+
+    const uint32_t row0 = tr * DT;
+#define CM_STORE(M, P) store_wave_tile<M, P, 1, 1>(hh, mid, ll, rterm, cterm, img, row0, col0, wr, wc, l32, lh, epi)
+#define CM_STORE_FAST(M) \
+    store_wave_fast<M, 1, 1>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi)
+    const TileBase tb = epi.tile_base(img, row0, col0, DT, DT);
+    if (tb.base != nullptr) {
+        if (mode == kWrap) CM_STORE_FAST(kWrap);
+        else if (mode == kSatNarrow) CM_STORE_FAST(kSatNarrow);
+        else CM_STORE_FAST(kSatWide);
+    } else if (mode == kSatNarrow) {
+        if (epi.pairs) CM_STORE(kSatNarrow, true); else CM_STORE(kSatNarrow, false);
+    } else if (mode == kWrap) {
+        if (epi.pairs) CM_STORE(kWrap, true); else CM_STORE(kWrap, false);
+    } else {
+        if (epi.pairs) CM_STORE(kSatWide, true); else CM_STORE(kSatWide, false);
+    }
+#undef CM_STORE_FAST
+#undef CM_STORE
+}
+
 // ---------------------------------------------------------------- standard conv, few taps
 // A standard convolution whose taps per output (in_ch kh kw <= 80) are few -- a network's stem
 // over its 1 .. 4 input channels, the 1x1 convolutions of up to 80 channels -- straight on the
@@ -2690,6 +2838,14 @@ struct ConvGeom {
     }
 };
 
+// A folded 1x1 convolution whose workgroups split their own input (conv_direct_kernel) instead of the
+// fold split and the plane GEMM: at most 8 row tiles, each of which splits the input again.  Measured
+// at batch 32, us (both launches of the other form): 96 -> 24 at 56 x 56 15.7 (32.1), 144 -> 32 at 28 x 28
+// 9.3 (16.6), 64 -> 384 at 14 x 14 8.5 (11.5), 576 -> 96 at 14 x 14 11.6 (17.6), 960 -> 320 at 7 x 7 16.6
+// (18.0), 512 -> 512 at 28 x 28 61.7 (69.8); 96 -> 576 at 14 x 14 14.1 (13.7), 320 -> 1280 at 7 x 7 16.0
+// (13.6), 1024 -> 2048 at 14 x 14, batch 8, 41.7 (31.0).
+bool conv_direct(const ConvGeom& g) { return g.out_ch <= 8 * DT && g.plane() >= 4; }
+
 // k of the GEMM: 16-channel tiles x kernel positions (the packed weight order), in BK steps.
 uint32_t conv_kp(uint32_t in_ch, uint32_t kh, uint32_t kw) {
     return (uint32_t)round_up((uint64_t)((in_ch + 15) / 16) * kh * kw * 16, BK);
@@ -2717,6 +2873,16 @@ int conv_gemm(const int16_t* x, const Planes& A, Planes& B, const int16_t* bptr,
               const DeviceState* st, hipStream_t s, int32_t lo, int32_t hi) {
     const uint32_t plane = g.plane();
     const uint64_t img = (uint64_t)g.out_ch * plane;
+    if (g.fold() && conv_direct(g)) {
+        const bool pairs = (reinterpret_cast<uintptr_t>(y) & 3) == 0 && (plane & 1) == 0;
+        const EpiConv epi{y, bptr, img, g.out_ch, plane, plane, 0, 0, g.wrap, pairs ? 1u : 0u, 0, lo, hi};
+        const uint32_t k = g.in_ch, mode = g.wrap ? kWrap : (k <= 8192 ? kSatNarrow : kSatWide);
+        const uint32_t tiles_r = ceil_div(g.out_ch, DT), tiles_c = ceil_div(plane, DT);
+        CM_LAUNCH("gemm_planes_kernel", (conv_direct_kernel<EpiConv>), dim3(tiles_r * tiles_c * g.batch), dim3(256), 0, s,
+                  A.hi, A.lo, A.part, A.lines_p, A.nsum(), x, (uint64_t)k * plane, k, plane,
+                  tiles_r, tiles_c, g.batch, A.kp, (int32_t)(64 * k), mode, epi);
+        return CM_OK;
+    }
     if (g.fold()) {
         const uint32_t cols = g.batch * plane;
         if (B.lines_p / 64 >= 4 * st->cus) {
