@@ -21,6 +21,8 @@
 #include "cm_common.h"
 #include "cm_rowops_math.h"
 
+#include <type_traits>
+
 namespace cm {
 namespace {
 
@@ -1347,152 +1349,325 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_ring_kernel(
 #undef CM_STORE
 }
 
-// ---------------------------------------------------------------- 1x1 convolutions, input split in the GEMM
+// ---------------------------------------------------------------- 1x1 convolutions, pixels in registers
 // A 1x1 stride-1 convolution is the product of the weights' planes and each image's [channels][pixels]
 // matrix.  Folding the images into byte planes first (split_fold*) writes and reads the whole input
-// again and costs a launch of 5 - 15 us; here a workgroup of 4 waves (64 x 64 outputs, 32 x 32 a wave)
-// splits its own 64 channels x 64 pixels a step: a thread loads 4 channels x 4 pixels (8-byte loads at
-// any alignment), transposes them with byte permutes into one dword of 4 channels a pixel and plane,
-// and adds the pixel's byte sums (v_dot4) on the way.  Every operand comes through registers, D steps
-// ahead (the pixels of a step are 64 rows a plane apart in HBM: a load at its use costs 2 - 3 us a
-// step), into two LDS buffers with one LDS-only barrier a step.  Pixel rows are 80 bytes (20 banks)
-// apart, so the fragment reads of 16 rows meet no conflict.  The input is split again for every row
-// tile, so it pays while the output rows are few tiles or the steps few (conv_direct).
-constexpr uint32_t kDbp = 80;                    // bytes of a pixel row of a staged B plane
-constexpr int DT = 64;                           // tile rows and columns
-
-template <class Epi>
-__global__ __launch_bounds__(256, 3) void conv_direct_kernel(
-    const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
-    uint32_t a_lines, uint32_t nsum_a, const int16_t* __restrict__ x, uint64_t x_img, uint32_t K,
-    uint32_t plane, uint32_t tiles_r, uint32_t tiles_c, uint32_t batch, uint32_t kp, int32_t k64, uint32_t mode, Epi epi) {
-    constexpr int A_T = DT * BK, B_T = DT * kDbp, BUF = 2 * A_T + 2 * B_T;
-    constexpr int D = 2;                               // steps ahead (3 and 4 measured the same)
-    __shared__ __attribute__((aligned(16))) int8_t buf[2][BUF];        // Ah, Al [64][64], Bh, Bl [64][kDbp]
-    __shared__ int2 rterm[DT], cterm[DT];              // (h, l) halves
-    __shared__ int32_t csum[DT];
-
-    // the row tiles of one pixel tile run on one XCD, one after the other (its L2 holds the pixels)
-    const TilePos tp = tile_pos(blockIdx.x, tiles_r, tiles_c * batch, 1);
-    const uint32_t tr = tp.tr, img = tp.tc / tiles_c, tc = tp.tc - img * tiles_c;
-    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const uint32_t wr = wave >> 1, wc = wave & 1, l32 = lane & 31, lh = lane >> 5;
-    const uint32_t nk = kp / BK, col0 = tc * DT;
-
-    // A: thread (row t / 4, 16-byte chunk t % 4) of each plane; B: channels 4 kg .., pixels 4 pg ..
-    const uint32_t arow = t >> 2, achunk = t & 3, adst = arow * BK + (achunk ^ ((arow >> 2) & 3)) * 16;
-    const uint64_t aoff = ((uint64_t)tr * DT + arow) * kp + achunk * 16;
-    const uint32_t pg = lane & 15, kg = 4 * wave + (lane >> 4);
-    // a group past the plane's end reads the plane's last 4 pixels, shifted to their places (plane >= 4)
-    const uint32_t px = min(col0 + 4 * pg, plane - 4), over = min(col0 + 4 * pg - px, 3u) * 16;
-    const bool ragged = (plane & 3) != 0 && col0 + DT > plane;         // uniform: some group needs the shift
-    const int16_t* xp = x + img * x_img + px;
-    struct Step { int4 ah, al; uint64_t b[4]; };
-    auto load = [&](Step& v, uint32_t step) {
-        v.ah = *reinterpret_cast<const int4*>(Ahi + aoff + step * BK);
-        v.al = *reinterpret_cast<const int4*>(Alo + aoff + step * BK);
+// again and costs a launch; here a wave of 32 output channels x 32 PX pixels reads its pixels straight
+// into the MFMA operand's layout: a lane's operand is 16 channels of one pixel, so it loads its PX
+// pixels in 16 channels (32 lanes side by side), transposes them with byte permutes and adds the
+// pixel's byte sums (v_dot4).  The weights' operand is 16 bytes of each plane.  Nothing is staged and
+// no barrier stands in the loop; D steps of 32 channels are in flight (a step's rows lie a plane
+// apart in HBM).  KW waves share one output tile's channels where the tiles alone leave the chip idle:
+// they exchange their accumulators through LDS and each stores 16 / KW of a lane's rows.  The launch
+// bounds keep a wave within 256 registers, so that the accumulators stay where the epilogue's vector
+// instructions read them (in AGPRs, 3 moves an element: 16 -> 96 at 32 x 112 x 112 37 us, 28 without).
+// Measured at batch 32, us, against a workgroup that split its 64 x 64 tile's pixels through LDS: 96 ->
+// 24 at 56 x 56 7.9 (15.9; its 24 MB 4.0 at 6 TB/s), 576 -> 96 at 14 x 14 9.7 (11.8), 960 -> 320 at 7 x 7
+// 11.4 (16.6), 512 -> 512 at 28 x 28 55.8 (65.5).
+// A wave's pixels of 16 channels from c0 on, PX a lane: one 32-bit offset a lane (the lane's pixel and
+// channel; below 2^32 bytes, the dispatch's rule) on scalar row addresses.  Channels at and past K read
+// some channel below it (their weights' planes are 0 there).
+template <int PX, bool RAG>
+struct PointPx {
+    typedef typename std::conditional<PX == 1, uint16_t, uint32_t>::type Px;
+    Px b[16];
+    __device__ __forceinline__ void load(const int16_t* x, uint32_t pix, uint32_t row, uint32_t c0, uint32_t K) {
+        const uint32_t off = pix + (RAG ? 0u : min(c0, K - 16) * row);
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            __builtin_memcpy(&v.b[r], xp + (uint64_t)min(step * BK + 4 * kg + r, K - 1) * plane, 8);
-    };
-    int32_t sh[4] = {0, 0, 0, 0}, sl[4] = {0, 0, 0, 0};
-    auto store = [&](int8_t* sm, Step& v, uint32_t step) {
-        *reinterpret_cast<int4*>(sm + adst) = v.ah;
-        *reinterpret_cast<int4*>(sm + A_T + adst) = v.al;
-        if (ragged) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) v.b[r] >>= over;
+        for (uint32_t r = 0; r < 16; r++) {
+            const char* xr = reinterpret_cast<const char*>(x) + (RAG ? 0u : (uint64_t)(r * row));
+            __builtin_memcpy(&b[r], xr + (RAG ? off + min(c0 + r, K - 1) * row : off), sizeof(Px));
         }
-        if ((step + 1) * BK > K) {                     // uniform: channels past K are padding (bytes 0, 0)
+    }
+    // the byte planes of pixel j in channels c0 + 4 g .. + 3 (plane bytes as the splits write them), and
+    // their sums over the channels below K
+    __device__ __forceinline__ void planes(v4i (&bh)[PX], v4i (&bl)[PX], int32_t (&sh)[PX], int32_t (&sl)[PX],
+                                           uint32_t c0, uint32_t K) const {
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                if (step * BK + 4 * kg + r >= K) v.b[r] = 0x0080008000800080ull;
-        }
-        int8_t* p = sm + 2 * A_T + 4 * pg * kDbp + 4 * kg;
+        for (int g = 0; g < 4; g++) {
+            uint32_t one = 0x01010101u;
+            if constexpr (RAG) one = c0 + 4 * g >= K ? 0u : one >> (8 * (4 - min(K - c0 - 4 * g, 4u)));
+            else one = c0 >= K ? 0u : one;
+            if constexpr (PX == 1) {
+                const uint32_t a = (uint32_t)b[4 * g] | (uint32_t)b[4 * g + 1] << 16,
+                               c = (uint32_t)b[4 * g + 2] | (uint32_t)b[4 * g + 3] << 16;
+                bh[0][g] = (int)__builtin_amdgcn_perm(c, a, 0x07050301u);
+                bl[0][g] = (int)(__builtin_amdgcn_perm(c, a, 0x06040200u) ^ 0x80808080u);
+            } else {
+                const uint32_t xh = __builtin_amdgcn_perm(b[4 * g + 1], b[4 * g], 0x07030501u),
+                               yh = __builtin_amdgcn_perm(b[4 * g + 3], b[4 * g + 2], 0x07030501u),
+                               xl = __builtin_amdgcn_perm(b[4 * g + 1], b[4 * g], 0x06020400u),
+                               yl = __builtin_amdgcn_perm(b[4 * g + 3], b[4 * g + 2], 0x06020400u);
 #pragma unroll
-        for (int c2 = 0; c2 < 2; c2++) {
-            const uint32_t d0 = (uint32_t)(v.b[0] >> (32 * c2)), d1 = (uint32_t)(v.b[1] >> (32 * c2)),
-                           d2 = (uint32_t)(v.b[2] >> (32 * c2)), d3 = (uint32_t)(v.b[3] >> (32 * c2));
-            const uint32_t xh = __builtin_amdgcn_perm(d1, d0, 0x07030501u), yh = __builtin_amdgcn_perm(d3, d2, 0x07030501u);
-            const uint32_t xl = __builtin_amdgcn_perm(d1, d0, 0x06020400u), yl = __builtin_amdgcn_perm(d3, d2, 0x06020400u);
+                for (int j = 0; j < 2; j++) {
+                    const uint32_t sel = j ? 0x07060302u : 0x05040100u;
+                    bh[j][g] = (int)__builtin_amdgcn_perm(yh, xh, sel);
+                    bl[j][g] = (int)(__builtin_amdgcn_perm(yl, xl, sel) ^ 0x80808080u);
+                }
+            }
 #pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const uint32_t sel = e ? 0x07060302u : 0x05040100u;
-                const int h = (int)__builtin_amdgcn_perm(yh, xh, sel), l = (int)(__builtin_amdgcn_perm(yl, xl, sel) ^ 0x80808080u);
-                sh[2 * c2 + e] = __builtin_amdgcn_sdot4(h, 0x01010101, sh[2 * c2 + e], false);
-                sl[2 * c2 + e] = __builtin_amdgcn_sdot4(l, 0x01010101, sl[2 * c2 + e], false);
-                *reinterpret_cast<int*>(p + (2 * c2 + e) * kDbp) = h;
-                *reinterpret_cast<int*>(p + (2 * c2 + e) * kDbp + B_T) = l;
+            for (int j = 0; j < PX; j++) {
+                sh[j] = __builtin_amdgcn_sdot4(bh[j][g], (int)one, sh[j], false);
+                sl[j] = __builtin_amdgcn_sdot4(bl[j][g], (int)one, sl[j], false);
             }
         }
+    }
+};
+
+// The results of a lane's PX pixels in one row: rows of terms (rh, rl), columns (ch, cl), as recombine; two
+// pixels are saturated, packed and clamped in pairs.  kSatTiny: K <= 256, where 2^8 HH needs no clamp.
+constexpr uint32_t kSatTiny = 4;
+typedef short v2s __attribute__((ext_vector_type(2)));
+template <uint32_t MODE, int PX>
+__device__ __forceinline__ void point_out(int16_t* dst, const int32_t (&hh)[PX], const int32_t (&mid)[PX], const int32_t (&ll)[PX],
+                                          int2 rt, const int32_t (&ch)[PX], const int32_t (&cl)[PX], int32_t lo, int32_t hi) {
+    int32_t q[PX];
+#pragma unroll
+    for (int j = 0; j < PX; j++) {
+        if constexpr (MODE == kSatTiny) q[j] = (int32_t)((uint32_t)hh[j] << 8) + (mid[j] + rt.x + ch[j]) + ((ll[j] + rt.y + cl[j]) >> 8);
+        else q[j] = recombine<MODE>(hh[j], mid[j], ll[j], rt.x + ch[j], rt.y + cl[j], -32768, 32767);
+    }
+    if constexpr (PX == 1) {
+        *dst = (int16_t)clamp_i32(q[0], lo, hi);
+    } else {
+        v2s o = __builtin_amdgcn_cvt_pk_i16(q[0], q[1]);
+        o = __builtin_elementwise_min(__builtin_elementwise_max(o, v2s{(short)lo, (short)lo}), v2s{(short)hi, (short)hi});
+        __builtin_memcpy(dst, &o, 4);
+    }
+}
+
+template <int PX, int KW, bool RAG>
+__global__ __launch_bounds__(64 * KW, PX == 2 ? 2 : 3) void conv_point_kernel(
+    const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
+    uint32_t a_lines, uint32_t nsum_a, const int16_t* __restrict__ x, uint32_t K, uint32_t plane, uint32_t cols,
+    uint32_t tiles_r, uint32_t tiles_c, uint32_t kp, uint32_t mode, EpiConv epi) {
+    constexpr int RW = 16 / KW, D = PX == 1 ? 3 : 2;
+    const uint32_t kpart = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63, l32 = lane & 31, lh = lane >> 5;
+    // the row tiles of one pixel tile run on one XCD, one after the other (its L2 holds the pixels)
+    const TilePos tp = tile_pos(blockIdx.x, tiles_r, tiles_c, 1);
+    const uint32_t tr = tp.tr;
+    const uint32_t col = (tp.tc * 32 + l32) * PX;                            // pixels over all images
+    const bool live = col < cols;
+    const uint32_t c = min(col, cols - PX), img = c / plane, p = c - img * plane;
+    const uint32_t nk = (K + 31) / 32, k0 = nk * kpart / KW, k1 = nk * (kpart + 1) / KW;   // this wave's steps
+    const uint32_t pix = 2 * (img * K * plane + p), row = 2 * plane;
+    const int8_t* const ah = Ahi + (uint64_t)(tr * 32 + l32) * kp + 16 * lh;
+    const int8_t* const al = Alo + (uint64_t)(tr * 32 + l32) * kp + 16 * lh;
+    struct Step { v4i ah, al; PointPx<PX, RAG> x; };
+    auto load = [&](Step& v, uint32_t k) {
+        v.ah = *reinterpret_cast<const v4i*>(ah + k * 32);
+        v.al = *reinterpret_cast<const v4i*>(al + k * 32);
+        v.x.load(x, pix, row, 32 * k + 16 * lh, K);
+    };
+    v16i hh[PX], mid[PX], ll[PX];
+    int32_t sh[PX], sl[PX];
+#pragma unroll
+    for (int j = 0; j < PX; j++) {
+        hh[j] = mid[j] = ll[j] = v16i{};
+        sh[j] = sl[j] = 0;
+    }
+    auto step = [&](const Step& v, uint32_t k) {
+        v4i bh[PX], bl[PX];
+        v.x.planes(bh, bl, sh, sl, 32 * k + 16 * lh, K);
+#pragma unroll
+        for (int j = 0; j < PX; j++) {
+            hh[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(v.ah, bh[j], hh[j], 0, 0, 0);
+            mid[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(v.ah, bl[j], mid[j], 0, 0, 0);
+            ll[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(v.al, bl[j], ll[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < PX; j++) mid[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(v.al, bh[j], mid[j], 0, 0, 0);
     };
     Step v[D];
 #pragma unroll
     for (int i = 0; i < D; i++)
-        if (i == 0 || (uint32_t)i < nk) load(v[i], i);
-    if (t < (uint32_t)DT) {                            // the rows' terms (the weights' sums and the bias)
-        const uint32_t line = tr * DT + t;
-        int32_t sum = 0;
-        for (uint32_t s = 0; s < nsum_a; s++) sum += rpart[(uint64_t)s * a_lines + line];
-        rterm[t] = make_int2(epi.row_bias(line) - k64 + (sum >> 1), (sum & 1) << 7);
-        csum[t] = (int32_t)(128 * K);                  // x = 256 h + l + 128
-    }
-
-    const uint32_t sw = (l32 >> 2) & 3;
-    const uint32_t fa = (wr * 32 + l32) * BK, fb = 2 * A_T + (wc * 32 + l32) * kDbp + lh * 16;
-    const uint32_t ch[2] = {((0 + lh) ^ sw) * 16, ((2 + lh) ^ sw) * 16};
-    v16i hh[1][1] = {{v16i{}}}, mid[1][1] = {{v16i{}}}, ll[1][1] = {{v16i{}}};
-    for (uint32_t kt = 0; kt < nk;) {
+        if (k0 + i < k1) load(v[i], k0 + i);
+    int32_t rsum = 0;                                                        // the lane's row's terms
+    for (uint32_t s = 0; s < nsum_a; s++) rsum += rpart[(uint64_t)s * a_lines + tr * 32 + l32];
+    const int32_t rb = epi.row_bias(tr * 32 + l32);
+    for (uint32_t k = k0; k < k1;) {
 #pragma unroll
         for (int i = 0; i < D; i++) {
-            int8_t* sm = buf[i];
-            store(sm, v[i], kt);
-            if (kt + D < nk) load(v[i], kt + D);
-            lds_barrier();                             // this buffer's readers of two steps ago passed the last one
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-                const v4i ah = *reinterpret_cast<const v4i*>(sm + fa + ch[s]);
-                const v4i al = *reinterpret_cast<const v4i*>(sm + A_T + fa + ch[s]);
-                const v4i bh = *reinterpret_cast<const v4i*>(sm + fb + s * 32);
-                const v4i bl = *reinterpret_cast<const v4i*>(sm + fb + B_T + s * 32);
-                hh[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah, bh, hh[0][0], 0, 0, 0);
-                mid[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah, bl, mid[0][0], 0, 0, 0);
-                ll[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al, bl, ll[0][0], 0, 0, 0);
-                mid[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al, bh, mid[0][0], 0, 0, 0);
-            }
-            if (++kt >= nk) break;
+            step(v[i], k);
+            if (k + D < k1) load(v[i], k + D);
+            if (++k >= k1) break;
         }
     }
-    // the pixels' sums: over the four lanes kg of a wave, then the waves
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        int32_t s = (sh[q] << 8) + sl[q];
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
-        if (lane < 16) atomicAdd(&csum[4 * pg + q], s);
-    }
-    __syncthreads();
-    if (t < (uint32_t)DT) cterm[t] = make_int2(csum[t] >> 1, (csum[t] & 1) << 7);
-    __syncthreads();
 
-    const uint32_t row0 = tr * DT;
-#define CM_STORE(M, P) store_wave_tile<M, P, 1, 1>(hh, mid, ll, rterm, cterm, img, row0, col0, wr, wc, l32, lh, epi)
-#define CM_STORE_FAST(M) \
-    store_wave_fast<M, 1, 1>(hh, mid, ll, rterm, cterm, tb.base, tb.ld, wr, wc, l32, lh, epi.lo, epi.hi)
-    const TileBase tb = epi.tile_base(img, row0, col0, DT, DT);
-    if (tb.base != nullptr) {
-        if (mode == kWrap) CM_STORE_FAST(kWrap);
-        else if (mode == kSatNarrow) CM_STORE_FAST(kSatNarrow);
-        else CM_STORE_FAST(kSatWide);
-    } else if (mode == kSatNarrow) {
-        if (epi.pairs) CM_STORE(kSatNarrow, true); else CM_STORE(kSatNarrow, false);
-    } else if (mode == kWrap) {
-        if (epi.pairs) CM_STORE(kWrap, true); else CM_STORE(kWrap, false);
-    } else {
-        if (epi.pairs) CM_STORE(kSatWide, true); else CM_STORE(kSatWide, false);
+    // terms of the columns and the rows: x = 256 h + l + 128 (recombine)
+    __shared__ int2 rterm[32];
+    __shared__ int32_t xch[KW > 1 ? KW * PX * 49 * 64 : 1];                  // [wave][pixel][3 accumulators x 16, sum][lane]
+    if (kpart == 0 && lh == 0) rterm[l32] = make_int2(rb - (int32_t)(64 * K) + (rsum >> 1), (rsum & 1) << 7);
+    int32_t cs[PX];
+#pragma unroll
+    for (int j = 0; j < PX; j++) {
+        cs[j] = (sh[j] << 8) + sl[j];
+        cs[j] += __shfl_xor(cs[j], 32, 64);
     }
-#undef CM_STORE_FAST
-#undef CM_STORE
+    if constexpr (KW > 1) {
+        // wave kpart keeps rows RW kpart .. of every lane and hands the others theirs
+#pragma unroll
+        for (int j = 0; j < PX; j++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                xch[((kpart * PX + j) * 49 + 3 * r) * 64 + lane] = hh[j][r];
+                xch[((kpart * PX + j) * 49 + 3 * r + 1) * 64 + lane] = mid[j][r];
+                xch[((kpart * PX + j) * 49 + 3 * r + 2) * 64 + lane] = ll[j][r];
+            }
+            xch[((kpart * PX + j) * 49 + 48) * 64 + lane] = cs[j];
+        }
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_wave_barrier();
+    }
+    int32_t ch[PX], cl[PX];
+    int32_t fh[RW][PX], fm[RW][PX], fl[RW][PX];
+#pragma unroll
+    for (int j = 0; j < PX; j++) {
+        int32_t s = cs[j];
+        if constexpr (KW > 1) {
+            s = 0;
+#pragma unroll
+            for (int w = 0; w < KW; w++) s += xch[((w * PX + j) * 49 + 48) * 64 + lane];
+        }
+        s += (int32_t)(128 * K);
+        ch[j] = s >> 1;
+        cl[j] = (s & 1) << 7;
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            if constexpr (KW == 1) {
+                fh[r][j] = hh[j][r];
+                fm[r][j] = mid[j][r];
+                fl[r][j] = ll[j][r];
+            } else {
+                const uint32_t q = kpart * RW + r;
+                fh[r][j] = fm[r][j] = fl[r][j] = 0;
+#pragma unroll
+                for (int w = 0; w < KW; w++) {
+                    fh[r][j] += xch[((w * PX + j) * 49 + 3 * q) * 64 + lane];
+                    fm[r][j] += xch[((w * PX + j) * 49 + 3 * q + 1) * 64 + lane];
+                    fl[r][j] += xch[((w * PX + j) * 49 + 3 * q + 2) * 64 + lane];
+                }
+            }
+        }
+    }
+    if (!live) return;                                                       // no barrier follows
+    const bool flat = epi.cn == 0 && tr * 32 + 32 <= epi.rows;               // uniform: rows cs apart, all inside
+    int16_t* const yl = epi.y + img * epi.img + (uint64_t)(tr * 32 + 4 * lh) * epi.cs + p;
+    auto store = [&](auto m) {
+        constexpr uint32_t MODE = decltype(m)::value;
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            const uint32_t q = kpart * RW + r, rl = 8 * (q / 4) + q % 4;
+            int16_t* dst = yl + (uint64_t)rl * epi.cs;
+            if (!flat) {
+                dst = epi.row_ptr(img, tr * 32 + 4 * lh + rl);
+                if (dst == nullptr) continue;
+                dst += p;
+            }
+            point_out<MODE, PX>(dst, fh[r], fm[r], fl[r], rterm[4 * lh + rl], ch, cl, epi.lo, epi.hi);
+        }
+    };
+    if (mode == kWrap) store(std::integral_constant<uint32_t, kWrap>{});
+    else if (mode == kSatNarrow) store(std::integral_constant<uint32_t, kSatNarrow>{});
+    else if (mode == kSatTiny) store(std::integral_constant<uint32_t, kSatTiny>{});
+    else store(std::integral_constant<uint32_t, kSatWide>{});
+}
+
+constexpr uint32_t kPointTiles = 3;              // row tiles of a wave, at most
+
+// The same product of at most 32 NK channels (a network's expansions, whose outputs outweigh everything
+// else): a wave keeps its 32 pixels' operands in registers and takes gt row tiles one after the
+// other, the next tile's weights in flight, so that the pixels' latency and transposition are paid
+// once for all of them.
+template <int NK, bool RAG>
+__global__ __launch_bounds__(256, NK > 1 ? 3 : 4) void conv_point_wide_kernel(
+    const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
+    const int16_t* __restrict__ x, uint32_t K, uint32_t plane, uint32_t cols, uint32_t blocks_r, uint32_t blocks_c,
+    uint32_t tiles_r, uint32_t gt, uint32_t kp, uint32_t mode, EpiConv epi) {
+    constexpr int PX = 1;                                                    // two pixels a lane measured the same
+    __shared__ int2 rterm[kPointTiles * 32];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, lh = lane >> 5;
+    const TilePos tp = tile_pos(blockIdx.x, blocks_r, blocks_c, 1);
+    const uint32_t t0 = tp.tr * gt, t1 = min(t0 + gt, tiles_r);
+    const uint32_t col = ((tp.tc * 4 + wave) * 32 + l32) * PX;               // pixels over all images
+    const bool live = col < cols;
+    const uint32_t c = min(col, cols - PX), img = c / plane, p = c - img * plane;
+    const uint32_t pix = 2 * (img * K * plane + p), row = 2 * plane;
+    const uint64_t aoff = (uint64_t)(t0 * 32 + l32) * kp + 16 * lh;
+    PointPx<PX, RAG> px[NK];
+#pragma unroll
+    for (int k = 0; k < NK; k++) px[k].load(x, pix, row, 32 * k + 16 * lh, K);
+    v4i ah[NK], al[NK];
+    auto load_a = [&](uint32_t t) {
+#pragma unroll
+        for (int k = 0; k < NK; k++) {
+            ah[k] = *reinterpret_cast<const v4i*>(Ahi + aoff + (uint64_t)(t - t0) * 32 * kp + 32 * k);
+            al[k] = *reinterpret_cast<const v4i*>(Alo + aoff + (uint64_t)(t - t0) * 32 * kp + 32 * k);
+        }
+    };
+    load_a(t0);
+    if (const uint32_t i = threadIdx.x; i < (t1 - t0) * 32) {
+        const int32_t sum = rpart[t0 * 32 + i];                              // one slab: K <= 1024
+        rterm[i] = make_int2(epi.row_bias(t0 * 32 + i) - (int32_t)(64 * K) + (sum >> 1), (sum & 1) << 7);
+    }
+    __syncthreads();
+    v4i bh[NK][PX], bl[NK][PX];
+    int32_t sh[PX], sl[PX], ch[PX], cl[PX];
+#pragma unroll
+    for (int j = 0; j < PX; j++) sh[j] = sl[j] = 0;
+#pragma unroll
+    for (int k = 0; k < NK; k++) px[k].planes(bh[k], bl[k], sh, sl, 32 * k + 16 * lh, K);
+#pragma unroll
+    for (int j = 0; j < PX; j++) {
+        int32_t s = (sh[j] << 8) + sl[j];
+        s += __shfl_xor(s, 32, 64);
+        s += (int32_t)(128 * K);                                             // x = 256 h + l + 128
+        ch[j] = s >> 1;
+        cl[j] = (s & 1) << 7;
+    }
+    int16_t* const yb = epi.y + img * epi.img + (uint64_t)(4 * lh) * epi.cs + p;
+    auto tiles = [&](auto m) {
+        constexpr uint32_t MODE = decltype(m)::value;
+        for (uint32_t t = t0; t < t1; t++) {
+            v16i hh[PX], mid[PX], ll[PX];
+#pragma unroll
+            for (int j = 0; j < PX; j++) hh[j] = mid[j] = ll[j] = v16i{};
+#pragma unroll
+            for (int k = 0; k < NK; k++) {
+#pragma unroll
+                for (int j = 0; j < PX; j++) {
+                    hh[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[k], bh[k][j], hh[j], 0, 0, 0);
+                    mid[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[k], bl[k][j], mid[j], 0, 0, 0);
+                    ll[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al[k], bl[k][j], ll[j], 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < PX; j++) mid[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al[k], bh[k][j], mid[j], 0, 0, 0);
+            }
+            if (t + 1 < t1) load_a(t + 1);
+            if (live) {
+                const bool flat = epi.cn == 0 && t * 32 + 32 <= epi.rows;    // uniform: rows cs apart, all inside
+                int16_t* const yl = yb + (uint64_t)t * 32 * epi.cs;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const uint32_t rl = 8 * (r / 4) + r % 4;
+                    int16_t* dst = yl + (uint64_t)rl * epi.cs;
+                    if (!flat) {
+                        dst = epi.row_ptr(img, t * 32 + 4 * lh + rl);
+                        if (dst == nullptr) continue;
+                        dst += p;
+                    }
+                    int32_t h[PX], m2[PX], l[PX];
+#pragma unroll
+                    for (int j = 0; j < PX; j++) h[j] = hh[j][r], m2[j] = mid[j][r], l[j] = ll[j][r];
+                    point_out<MODE, PX>(dst, h, m2, l, rterm[(t - t0) * 32 + 4 * lh + rl], ch, cl, epi.lo, epi.hi);
+                }
+            }
+        }
+    };
+    if (mode == kWrap) tiles(std::integral_constant<uint32_t, kWrap>{});
+    else tiles(std::integral_constant<uint32_t, kSatTiny>{});
 }
 
 // ---------------------------------------------------------------- standard conv, few taps
@@ -2830,21 +3005,69 @@ struct ConvGeom {
     uint32_t batch, in_ch, in_h, in_w, out_ch, out_h, out_w, kh, kw, sh, sw, dh, dw, pt, pl;
     uint32_t cs, cn, gs, wrap;          // the y pattern (cs = plane without one), int32 wrap
     uint32_t plane() const { return out_h * out_w; }
-    // 1x1 stride-1 unpadded, same plane in and out, no y pattern: the images fold into the
-    // GEMM's columns (one slice of batch * plane lines)
-    bool fold() const {
+    // 1x1 stride-1 unpadded, same plane in and out
+    bool pointwise() const {
         return kh == 1 && kw == 1 && sh == 1 && sw == 1 && pt == 0 && pl == 0 && out_h == in_h && out_w == in_w &&
-               cn == 0 && cs == plane() && (uint64_t)batch * plane() < ((uint64_t)1 << 31);
+               (uint64_t)batch * plane() < ((uint64_t)1 << 31);
     }
+    // and no y pattern: the images fold into the GEMM's columns (one slice of batch * plane lines)
+    bool fold() const { return pointwise() && cn == 0 && cs == plane(); }
 };
 
-// A folded 1x1 convolution whose workgroups split their own input (conv_direct_kernel) instead of the
-// fold split and the plane GEMM: at most 8 row tiles, each of which splits the input again.  Measured
-// at batch 32, us (both launches of the other form): 96 -> 24 at 56 x 56 15.7 (32.1), 144 -> 32 at 28 x 28
-// 9.3 (16.6), 64 -> 384 at 14 x 14 8.5 (11.5), 576 -> 96 at 14 x 14 11.6 (17.6), 960 -> 320 at 7 x 7 16.6
-// (18.0), 512 -> 512 at 28 x 28 61.7 (69.8); 96 -> 576 at 14 x 14 14.1 (13.7), 320 -> 1280 at 7 x 7 16.0
-// (13.6), 1024 -> 2048 at 14 x 14, batch 8, 41.7 (31.0).
-bool conv_direct(const ConvGeom& g) { return g.out_ch <= 8 * DT && g.plane() >= 4; }
+// The 1x1 convolutions whose waves take their operand straight from the pixels (conv_point*_kernel)
+// instead of the fold split and the plane GEMM: up to 64 input channels at any output, as a wave keeps
+// its pixels; otherwise, as every row tile splits the input again and each wave loads its own weights,
+// up to 1280 output channels and 2^19 weights, or two tiles a compute unit.  Measured us (both launches
+// of the other form): 24 -> 144 at 32 x 56 x 56 16.9 (46.8), 64 -> 256 at 16 x 56 x 56 17.1 (35.2), 960 -> 320 at
+// 32 x 7 x 7 11.9 (17.9), 512 -> 512 at 32 x 28 x 28 59.2 (71.9), 320 -> 1280 at 32 x 7 x 7 13.6 (13.7), 2048 -> 1000
+// at 1 x 7 x 7 9.7 (19.6); 512 -> 1024 at 32 x 7 x 7 16.1 (15.0), 2048 -> 512 at 32 x 7 x 7 28.8 (25.1).
+bool point_path(const ConvGeom& g, const DeviceState* st) {
+    if (!g.pointwise() || 2ull * g.in_ch * g.plane() > 0xFFFFFFFFull) return false;
+    if (g.in_ch <= 64) return true;
+    const uint64_t tiles = (uint64_t)ceil_div(g.out_ch, 32) * ceil_div((size_t)g.batch * g.plane(), 32);
+    return (g.out_ch <= 1280 && (uint64_t)g.in_ch * g.out_ch < (1u << 19)) || tiles <= 2ull * st->cus;
+}
+
+int point_launch(const int16_t* x, const Planes& A, const int16_t* bptr, int16_t* y, const ConvGeom& g, uint32_t batch,
+                  const DeviceState* st, hipStream_t s, int32_t lo, int32_t hi) {
+    const uint32_t plane = g.plane(), k = g.in_ch, cols = batch * plane, tr = ceil_div(g.out_ch, 32), tc = ceil_div(cols, 32);
+    const EpiConv epi{y, bptr, (uint64_t)g.out_ch * plane, g.out_ch, plane, g.cs, g.cn, g.gs, g.wrap, 0, 0, lo, hi};
+    const uint32_t mode = g.wrap ? kWrap : (k <= 256 ? kSatTiny : (k <= 8192 ? kSatNarrow : kSatWide));
+    const bool rag = k % 16 != 0;
+    const uint64_t tiles = (uint64_t)tr * tc, cus = st->cus;
+    if (k <= 64) {
+        // up to 3 row tiles a wave while two waves a SIMD remain (24 -> 144 at 32 x 56 x 56: 1 / 2 / 3 / 4 tiles
+        // 19.2 / 17.0 / 17.1 / 19.9 us; 64 -> 384 at 32 x 14 x 14, 2352 tiles: 6.3 / 7.1 / 7.4)
+        const uint32_t gt = (uint32_t)std::min<uint64_t>({kPointTiles, tr, std::max<uint64_t>(1, tiles / (8 * cus))});
+        const uint32_t br = ceil_div(tr, gt), bc = ceil_div(tc, 4);
+#define CM_WIDE(NK_, RAG_)                                                                                               \
+    CM_LAUNCH("conv_point_kernel", (conv_point_wide_kernel<NK_, RAG_>), dim3(br * bc), dim3(256), 0, s, A.hi, A.lo, \
+              A.part, x, k, plane, cols, br, bc, tr, gt, A.kp, mode, epi)
+        if (k <= 32) {
+            if (rag) { CM_WIDE(1, true); } else { CM_WIDE(1, false); }
+        } else {
+            if (rag) { CM_WIDE(2, true); } else { CM_WIDE(2, false); }
+        }
+#undef CM_WIDE
+        return CM_OK;
+    }
+    // two pixels a lane where that leaves three waves a compute unit (256 -> 256 at 8 x 28 x 28, 784 tiles of
+    // 64 pixels: 8.5 us against 10.0), else one: alone from 4 waves a unit up (160 -> 960 at 32 x 7 x 7, 1470
+    // tiles: 8.2 / 8.2 / 9.5 with 1 / 2 / 4 waves), two of them sharing the channels from 2.5 up (512 -> 512 at
+    // 8 x 14 x 14, 784 tiles: 10.6 / 10.1 / 10.9), four below (576 -> 160 at 32 x 7 x 7, 245 tiles: 8.4 / 6.7 / 6.3)
+#define CM_POINT1(PX_, KW_, RAG_)                                                                                        \
+    CM_LAUNCH("conv_point_kernel", (conv_point_kernel<PX_, KW_, RAG_>), dim3(tr * ceil_div(cols, 32 * PX_)), dim3(64 * KW_), \
+              0, s, A.hi, A.lo, A.part, A.lines_p, A.nsum(), x, k, plane, cols, tr, ceil_div(cols, 32 * PX_), A.kp, mode, epi)
+#define CM_POINT(PX_, KW_) \
+    if (rag) { CM_POINT1(PX_, KW_, true); } else { CM_POINT1(PX_, KW_, false); }
+    if (plane % 2 == 0 && (uint64_t)tr * ceil_div(cols, 64) >= 3 * cus) { CM_POINT(2, 1) }
+    else if (tiles >= 4 * cus) { CM_POINT(1, 1) }
+    else if (2 * tiles >= 5 * cus) { CM_POINT(1, 2) }
+    else { CM_POINT(1, 4) }
+#undef CM_POINT
+#undef CM_POINT1
+    return CM_OK;
+}
 
 // k of the GEMM: 16-channel tiles x kernel positions (the packed weight order), in BK steps.
 uint32_t conv_kp(uint32_t in_ch, uint32_t kh, uint32_t kw) {
@@ -2873,14 +3096,14 @@ int conv_gemm(const int16_t* x, const Planes& A, Planes& B, const int16_t* bptr,
               const DeviceState* st, hipStream_t s, int32_t lo, int32_t hi) {
     const uint32_t plane = g.plane();
     const uint64_t img = (uint64_t)g.out_ch * plane;
-    if (g.fold() && conv_direct(g)) {
-        const bool pairs = (reinterpret_cast<uintptr_t>(y) & 3) == 0 && (plane & 1) == 0;
-        const EpiConv epi{y, bptr, img, g.out_ch, plane, plane, 0, 0, g.wrap, pairs ? 1u : 0u, 0, lo, hi};
-        const uint32_t k = g.in_ch, mode = g.wrap ? kWrap : (k <= 8192 ? kSatNarrow : kSatWide);
-        const uint32_t tiles_r = ceil_div(g.out_ch, DT), tiles_c = ceil_div(plane, DT);
-        CM_LAUNCH("gemm_planes_kernel", (conv_direct_kernel<EpiConv>), dim3(tiles_r * tiles_c * g.batch), dim3(256), 0, s,
-                  A.hi, A.lo, A.part, A.lines_p, A.nsum(), x, (uint64_t)k * plane, k, plane,
-                  tiles_r, tiles_c, g.batch, A.kp, (int32_t)(64 * k), mode, epi);
+    if (point_path(g, st)) {
+        // images whose input stays below the kernels' 32-bit byte offsets, one launch each
+        const uint32_t per = (uint32_t)std::min<uint64_t>(g.batch, 0xFFFFFFFFull / (2ull * g.in_ch * plane));
+        for (uint32_t i = 0; i < g.batch; i += per) {
+            const int rc = point_launch(x + (uint64_t)i * g.in_ch * plane, A, bptr, y + i * img, g,
+                                        std::min(per, g.batch - i), st, s, lo, hi);
+            if (rc) return rc;
+        }
         return CM_OK;
     }
     if (g.fold()) {

@@ -962,10 +962,10 @@ class Simulator:
         if img is None:
             w = self._get(wt, raw).cpu().numpy().reshape(wt.shape)
             img = torch.from_numpy(conv_weight_image(w, sn.is_depthwise)).to(self.device)
-            # a pointwise one over few pixels runs faster on the GEMM than on the VALU path, whatever its
-            # taps (32 -> 192 at 32 x 28 x 28 12.2 us against 14.7; 24 -> 144 at 32 x 56 x 56 28.1 against 25.4)
+            # a pointwise one runs faster on the matrix units than on the VALU path, whatever its taps
+            # (24 -> 144 at 32 x 56 x 56 17.1 us against 25.4, 16 -> 96 at 32 x 112 x 112 28.2 against 35.0)
             pointwise = ((sn.kh, sn.kw, sn.stride_h, sn.stride_w, sn.pad_top, sn.pad_left) == (1, 1, 1, 1, 0, 0)
-                         and (sn.in_h, sn.in_w) == (sn.out_h, sn.out_w) and sn.batch * sn.out_h * sn.out_w <= 32768)
+                         and (sn.in_h, sn.in_w) == (sn.out_h, sn.out_w))
             if not sn.is_depthwise and wt.data is not None and (
                     pointwise or not units.conv_small(sn.in_ch, sn.kh, sn.kw, sn.out_ch, sn.batch)):
                 # a constant weight of a standard convolution on the GEMM: its operand split once

@@ -1,7 +1,8 @@
-"""1x1 convolutions whose workgroups split their own input (at most 512 output channels), bit for bit
-against the oracle: planes from 4 pixels up that end anywhere in a 64-pixel tile and in a group of
-4, channels at the edges of a 64-channel step and of the 16-channel weight tiles, one step and
-several, output channels at the edges of the row tiles and past 512, biases, RELU and RELU6, both output
+"""1x1 convolutions that take their operand straight from the pixels, bit for bit against the
+oracle: planes from one pixel up that end anywhere in a 32- or 64-pixel tile, channels at the edges of
+the 16-channel loads and the 32-channel steps, one step and several, output channels at the edges
+of the row tiles, the forms of one to three row tiles a wave, of one and two pixels a lane and of one,
+two and four waves an output tile, outputs on a y pattern, biases, RELU and RELU6, both output
 rules, full-range operands; the graph's choice of it over the few-tap path."""
 import numpy as np
 import pytest
@@ -25,8 +26,9 @@ def U():
 @pytest.mark.parametrize("batch,in_ch,h,w,out_ch", [
     (1, 8, 2, 2, 5), (3, 16, 1, 5, 64), (2, 63, 3, 3, 65), (1, 64, 7, 9, 17), (5, 65, 7, 7, 96), (2, 128, 8, 8, 64),
     (3, 129, 13, 5, 130), (2, 200, 14, 14, 33), (1, 320, 11, 11, 512), (2, 33, 9, 7, 520), (4, 96, 16, 12, 48),
-    (1, 640, 5, 13, 70)])
-def test_conv_direct(U, oracle_lib, batch, in_ch, h, w, out_ch, act, wrap, lim):
+    (1, 640, 5, 13, 70), (3, 16, 1, 1, 16), (2, 1, 3, 1, 3), (16, 9, 64, 64, 150), (16, 17, 64, 64, 64), (2, 34, 64, 64, 33),
+    (8, 72, 56, 56, 40), (8, 65, 33, 33, 128), (5, 100, 33, 33, 100), (1, 2048, 7, 7, 100), (3, 1025, 2, 2, 40)])
+def test_conv_point(U, oracle_lib, batch, in_ch, h, w, out_ch, act, wrap, lim):
     from cormorant_amd.packing import conv_weight_image
     rng = np.random.default_rng(batch + in_ch + 7 * h + out_ch + act)
     x = rng.integers(-lim, lim, batch * in_ch * h * w).astype(np.int16)
@@ -44,6 +46,27 @@ def test_conv_direct(U, oracle_lib, batch, in_ch, h, w, out_ch, act, wrap, lim):
     got = host(y)
     np.testing.assert_array_equal(got[:n], want)
     assert (got[n:] == 0x5A5A).all()
+
+
+@pytest.mark.parametrize("in_ch", [24, 96])
+@pytest.mark.parametrize("h,w", [(9, 7), (10, 6)])
+def test_conv_point_y_pattern(U, oracle_lib, in_ch, h, w):
+    """Output channel o of an image at (o % 4) cs + (o / 4) gs."""
+    from cormorant_amd.packing import conv_weight_image
+    rng = np.random.default_rng(in_ch + h)
+    batch, out_ch, plane = 1, 40, h * w
+    cs, cn, gs = 10 * (plane + 3), 4, plane + 3
+    x = rng.integers(-2000, 2000, batch * in_ch * plane).astype(np.int16)
+    img = np.asarray(conv_weight_image(rng.integers(-2000, 2000, (out_ch, in_ch, 1, 1)).astype(np.int16), False)).reshape(-1)
+    want = oracle_lib.conv(x, img, None, out_ch * plane, batch, in_ch, h, w, out_ch, h, w, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0)
+    y = poisoned16(40 * (plane + 3) + 8)
+    U.conv_planes(dev16(x, extra=0), U.conv_w_planes(dev16(img), out_ch, in_ch, 1, 1), None, y, batch, in_ch, h, w, out_ch,
+                  h, w, 1, 1, y_cs=cs, y_cn=cn, y_gs=gs)
+    full = np.full(40 * (plane + 3) + 8, 0x5A5A, np.int16)
+    for o in range(out_ch):
+        at = (o % cn) * cs + (o // cn) * gs
+        full[at:at + plane] = want[o * plane:(o + 1) * plane]
+    np.testing.assert_array_equal(host(y), full)
 
 
 @pytest.mark.parametrize("batch,hw", [(1, 6), (32, 33)])
