@@ -212,7 +212,7 @@ GRAPH_KERNELS = ("gemm_planes_kernel", "split_rows_kernel", "split_cols_kernel",
                  "split_fold_kernel", "split_fold_lds_kernel", "skinny_wrap_kernel", "skinny_reduce_kernel",
                  "skinny_planes_kernel", "skinny_mulact_kernel", "decode_attn_kernel", "decode_prep_kernel",
                  "attention_kernel", "embed_rows_kernel", "ro_fold_kernel",
-                 "ro_tload_kernel", "ro_xpose_kernel", "conv_small_kernel")
+                 "ro_tload_kernel", "ro_xpose_kernel", "conv_small_kernel", "conv_point_kernel")
 
 
 TIMED_REPLAYS = 10      # replays of the instrumented graph whose per-launch events are read

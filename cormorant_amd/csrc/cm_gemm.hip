@@ -1891,88 +1891,13 @@ __global__ __launch_bounds__(256) void conv_dw_kernel(const int16_t* __restrict_
     }
 }
 
-// Depthwise 3x3, dilation 1, stride SH x SW (the MobileNet blocks): each lane computes R
-// output rows of one column (a vertical strip) from the (R - 1) SH + 3 input rows' three
-// taps held in registers.  Lanes of a wavefront sit on neighbouring columns, so each load
-// is one contiguous run of an input row and the L1 serves the overlap between neighbours.
-// Sums are int32 where they are exact: the wrap path, or a channel whose bound
-// sum |w| 2^15 + |bias| 2^8 stays below 2^31; int64 otherwise.
-template <int SH, int SW, int R>
-__global__ __launch_bounds__(256) void conv_dw3_kernel(const int16_t* __restrict__ x, const int16_t* __restrict__ w,
-                                                       const int16_t* __restrict__ bias, int16_t* __restrict__ y,
-                                                       uint32_t items, uint32_t strips, uint32_t ch, uint32_t in_h,
-                                                       uint32_t in_w, uint32_t out_h, uint32_t out_w, uint32_t pt,
-                                                       uint32_t pl, uint32_t dws, uint32_t cs, uint32_t cn,
-                                                       uint32_t gs, uint32_t wrap, int32_t lo, int32_t hi) {
-    constexpr int NR = (R - 1) * SH + 3;
-    const uint32_t per_plane = strips * out_w;
-    for (uint32_t it = blockIdx.x * blockDim.x + threadIdx.x; it < items; it += gridDim.x * blockDim.x) {
-        const uint32_t p = it / per_plane, rem = it - p * per_plane;
-        const uint32_t sidx = rem / out_w, ow = rem - sidx * out_w;
-        const uint32_t nb = p / ch, c = p - nb * ch;
-        const int16_t* xp = x + (uint64_t)p * in_h * in_w;
-        const int16_t* wp = w + (uint64_t)c * dws;
-        int wv[9];
-        uint32_t wabs = 0;
-#pragma unroll
-        for (int i = 0; i < 9; i++) {
-            wv[i] = wp[i];
-            wabs += (uint32_t)(wv[i] < 0 ? -wv[i] : wv[i]);
-        }
-        const int b0 = bias ? (int)bias[c] : 0;
-        const int oh0 = (int)(sidx * R);
-        const int ih0 = oh0 * SH - (int)pt, iw0 = (int)(ow * SW) - (int)pl;
-        bool cv[3];
-#pragma unroll
-        for (int b = 0; b < 3; b++) cv[b] = (uint32_t)(iw0 + b) < in_w;
-        int v[NR][3];
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const int ih = ih0 + r;
-            const bool rv = (uint32_t)ih < in_h;
-            const int16_t* xr = xp + (int64_t)ih * in_w + iw0;
-#pragma unroll
-            for (int b = 0; b < 3; b++) v[r][b] = (rv && cv[b]) ? (int)xr[b] : 0;
-        }
-        const uint64_t bound = (uint64_t)wabs * 32768u + (uint64_t)(b0 < 0 ? -b0 : b0) * 256u;
-        int out[R];
-        if (wrap || bound < ((uint64_t)1 << 31)) {
-#pragma unroll
-            for (int i = 0; i < R; i++) {
-                uint32_t acc = (uint32_t)b0 << 8;
-#pragma unroll
-                for (int a = 0; a < 3; a++)
-#pragma unroll
-                    for (int b = 0; b < 3; b++) acc += (uint32_t)(v[i * SH + a][b] * wv[a * 3 + b]);
-                out[i] = clamp_i32((int)acc >> 8, lo, hi);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < R; i++) {
-                long long acc = (long long)b0 * 256;
-#pragma unroll
-                for (int a = 0; a < 3; a++)
-#pragma unroll
-                    for (int b = 0; b < 3; b++) acc += (long long)v[i * SH + a][b] * wv[a * 3 + b];
-                const long long q = acc >> 8;
-                out[i] = (int)(q > hi ? hi : (q < lo ? lo : q));
-            }
-        }
-        const uint64_t plane = (uint64_t)out_h * out_w;
-        const uint64_t base = cn ? (uint64_t)(c % cn) * cs + (uint64_t)(c / cn) * gs : (uint64_t)c * cs;
-        int16_t* yp = y + (uint64_t)nb * ch * plane + base + ow;
-#pragma unroll
-        for (int i = 0; i < R; i++)
-            if ((uint32_t)(oh0 + i) < out_h) yp[(uint64_t)(oh0 + i) * out_w] = (int16_t)out[i];
-    }
-}
-
 // Depthwise 3x3 stride 1 on rows of a multiple of 8 columns: a lane computes 8 columns x R
 // rows.  Per input row it loads the 16-byte word of its 8 columns and the dwords either side
 // (columns 8j - 2 .. 8j + 9, zero past the row), and every output takes its row's three
 // taps as two v_dot2_i32_i16 against packed weight pairs, so no 16-bit value is unpacked.
-// PL (the left pad, 0..2) fixes which pairs line up.  Exact int32 sums as in
-// conv_dw3_kernel; a channel whose bound leaves int32 takes int64 per value.
+// PL (the left pad, 0..2) fixes which pairs line up.  Sums are int32 where they are
+// exact: the wrap path, or a channel whose bound sum |w| 2^15 + |bias| 2^8 stays below 2^31; int64 a value
+// otherwise.
 typedef short cm_s16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ int dot2(uint32_t x, uint32_t w, int acc) {
@@ -2089,6 +2014,146 @@ __global__ __launch_bounds__(256) void conv_dw3v_kernel(const int16_t* __restric
             o.z = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pk_i16(q[4], q[5]));
             o.w = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pk_i16(q[6], q[7]));
             store_stream(yp + (uint64_t)(oh0 + i) * out_w, o);
+        }
+    }
+}
+
+// Depthwise 3x3, dilation 1, stride S both ways, at any width (the MobileNet blocks): a lane computes R rows
+// of 8 / S output columns from the 10 input columns 8 j - pad_left .. + 9 of every input row, loaded as 20
+// bytes at any alignment.  A load a tap kept the address unit busy: 27 two-byte loads for 4 outputs at
+// stride 2, 96 channels at 32 x 112 x 112 36.7 us, 20.7 this way (96 MB: 16.1 at 6 TB/s); 384 at 14 x 14
+// 7.1 and 5.4, 960 at 7 x 7 6.2 and 5.3.  Columns outside the plane are masked off; at the tensor's ends
+// the words move inside it and are shifted back.  Two rows: a longer strip saves loads where the planes
+// are large (20.0) but its code and its chain cost the small ones (4 rows: 384 at 14 x 14 7.0, one image
+// 4.5 against 3.5).  Rows of a multiple of 8 columns at stride 1 keep the aligned words above (144 channels
+// at 32 x 56 x 56 14.6 us, 18.6 here).  Taps and sums as conv_dw3v_kernel.
+template <int S, int R>
+__global__ __launch_bounds__(256) void conv_dw3_kernel(const int16_t* __restrict__ x, const int16_t* __restrict__ w,
+                                                       const int16_t* __restrict__ bias, int16_t* __restrict__ y,
+                                                       uint32_t items, uint32_t planes, uint32_t strips, uint32_t groups,
+                                                       uint32_t ch, uint32_t in_h, uint32_t in_w, uint32_t out_h,
+                                                       uint32_t out_w, uint32_t pt, uint32_t pl, uint32_t dws, uint32_t cs,
+                                                       uint32_t cn, uint32_t gs, uint32_t wrap, int32_t lo, int32_t hi) {
+    constexpr int T = 8 / S;                                         // output columns of a lane
+    const uint32_t per_plane = strips * groups, in_hw = in_h * in_w;
+    for (uint32_t it = blockIdx.x * blockDim.x + threadIdx.x; it < items; it += gridDim.x * blockDim.x) {
+        const uint32_t p = it / per_plane, rem = it - p * per_plane;
+        const uint32_t sidx = rem / groups, j = rem - sidx * groups;
+        const uint32_t nb = p / ch, c = p - nb * ch;
+        const int16_t* xp = x + (uint64_t)p * in_hw;
+        const int16_t* wp = w + (uint64_t)c * dws;
+        // the last lane of a row ends at the row's end (columns of the lane before it come out twice, the same)
+        const int oh0 = (int)(sidx * R), ow0 = (int)min(T * j, out_w - min((uint32_t)T, out_w));
+        const int ih0 = oh0 * S - (int)pt, iw0 = ow0 * S - (int)pl;
+        // the plane offsets at which the words of 10 columns stay inside the tensor (of 10 elements or more)
+        const int first = -(int)min((uint64_t)p * in_hw, (uint64_t)1 << 29);
+        const int last = (int)min((uint64_t)(planes - p) * in_hw, (uint64_t)1 << 30) - 10;
+        constexpr int NR = (R - 1) * S + 3;
+        uint32_t v[NR][5];
+        auto offset = [&](int r) { return min(max(ih0 + r, 0), (int)in_h - 1) * (int)in_w + iw0; };
+        int moved = 0;
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int o = offset(r), at = min(max(o, first), last);
+            moved = max(moved, max(o - at, at - o));
+            __builtin_memcpy(v[r], xp + at, 16);
+            __builtin_memcpy(v[r] + 4, xp + at + 8, 4);
+        }
+        int wv[9];
+        uint32_t wabs = 0;
+#pragma unroll
+        for (int i = 0; i < 9; i++) {
+            wv[i] = wp[i];
+            wabs += (uint32_t)(wv[i] < 0 ? -wv[i] : wv[i]);
+        }
+        const int b0 = bias ? (int)bias[c] : 0;
+        const uint64_t bound = (uint64_t)wabs * 32768u + (uint64_t)(b0 < 0 ? -b0 : b0) * 256u;
+        if (moved > 0) {
+            // at the tensor's ends: the words back to their columns, one element at a time (what comes in
+            // lies outside the plane and is masked below)
+#pragma unroll 1
+            for (int n = 0; n < min(moved, 10); n++) {
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    const int d = offset(r) - min(max(offset(r), first), last);
+                    if (d > n) {
+#pragma unroll
+                        for (int k = 0; k < 5; k++) v[r][k] = __builtin_amdgcn_alignbit(k < 4 ? v[r][k + 1 < 5 ? k + 1 : 4] : 0u, v[r][k], 16);
+                    } else if (-d > n) {
+#pragma unroll
+                        for (int k = 4; k >= 0; k--) v[r][k] = __builtin_amdgcn_alignbit(v[r][k], k > 0 ? v[r][k - 1 > 0 ? k - 1 : 0] : 0u, 16);
+                    }
+                }
+            }
+        }
+        uint32_t m[5];
+#pragma unroll
+        for (int k = 0; k < 5; k++)
+            m[k] = ((uint32_t)(iw0 + 2 * k) < in_w ? 0xFFFFu : 0u) | ((uint32_t)(iw0 + 2 * k + 1) < in_w ? 0xFFFF0000u : 0u);
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const bool in = (uint32_t)(ih0 + r) < in_h;
+#pragma unroll
+            for (int k = 0; k < 5; k++) v[r][k] &= in ? m[k] : 0u;
+        }
+        const uint64_t plane = (uint64_t)out_h * out_w;
+        const uint64_t base = cn ? (uint64_t)(c % cn) * cs + (uint64_t)(c / cn) * gs : (uint64_t)c * cs;
+        int16_t* yp = y + (uint64_t)nb * ch * plane + base + ow0;
+        const int nv = (int)min(out_w, (uint32_t)T);                 // the columns inside
+        if (!wrap && bound >= ((uint64_t)1 << 31)) {
+            // int64 a value (weights too large for an int32 bound): each tap loaded alone
+#pragma unroll 1
+            for (int n = 0; n < R * T; n++) {
+                const int i = n / T, t = n % T, oh = oh0 + i;
+                if (oh >= (int)out_h || t >= nv) continue;
+                long long acc = (long long)b0 * 256;
+#pragma unroll 1
+                for (int k = 0; k < 9; k++) {
+                    const int ih = ih0 + i * S + k / 3, iw = iw0 + t * S + k % 3;
+                    if ((uint32_t)ih < in_h && (uint32_t)iw < in_w) acc += (long long)xp[ih * (int)in_w + iw] * wp[k];
+                }
+                const long long f = acc >> 8;
+                yp[(uint64_t)oh * out_w + t] = (int16_t)(f > hi ? hi : (f < lo ? lo : f));
+            }
+            continue;
+        }
+        int q[R][T];
+#pragma unroll
+        for (int i = 0; i < R; i++)
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                int acc = b0 * 256;
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    const uint32_t* vr = v[i * S + a];
+                    // weight pairs for an even first column (w0, w1), (w2, 0), an odd one (0, w0), (w1, w2)
+                    if ((t * S & 1) == 0) {
+                        acc = dot2(vr[t * S >> 1], pack16(wv[3 * a], wv[3 * a + 1]), acc);
+                        acc = dot2(vr[(t * S >> 1) + 1], pack16(wv[3 * a + 2], 0), acc);
+                    } else {
+                        acc = dot2(vr[t * S >> 1], pack16(0, wv[3 * a]), acc);
+                        acc = dot2(vr[(t * S >> 1) + 1], pack16(wv[3 * a + 1], wv[3 * a + 2]), acc);
+                    }
+                }
+                q[i][t] = acc >> 8;
+            }
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            if ((uint32_t)(oh0 + i) >= out_h) break;
+            uint32_t o[T / 2];
+#pragma unroll
+            for (int t = 0; t < T; t += 2)
+                o[t / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pk_i16(clamp_i32(q[i][t], lo, hi), clamp_i32(q[i][t + 1], lo, hi)));
+            int16_t* dst = yp + (uint64_t)(oh0 + i) * out_w;
+            if (nv == T) {
+                __builtin_memcpy(dst, o, 2 * T);
+            } else {
+#pragma unroll
+                for (int t = 0; t < T - 1; t += 2) {
+                    if (t + 1 < nv) __builtin_memcpy(dst + t, &o[t / 2], 4);
+                    else if (t < nv) dst[t] = (int16_t)o[t / 2];
+                }
+            }
         }
     }
 }
@@ -3199,21 +3264,19 @@ int conv_run(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y
             return CM_OK;
         }
     }
-    if (dw3 && stride_h == stride_w && stride_h <= 2) {
-        const uint32_t R = stride_h == 1 ? 8 : 4;
-        const uint32_t strips = (out_h + R - 1) / R;
-        const uint64_t items = (uint64_t)batch * out_ch * strips * out_w;
+    if (dw3 && stride_h == stride_w && stride_h <= 2 && (uint64_t)in_h * in_w < (1u << 29) && (uint64_t)batch * out_ch * in_h * in_w >= 10 && out_h < (1u << 27) && out_w < (1u << 27) &&
+        pad_top < (1u << 28) && pad_left < (1u << 28) && (uint64_t)batch * out_ch < (1u << 31)) {
+        constexpr uint32_t R = 2;
+        const uint32_t strips = ceil_div(out_h, R), groups = ceil_div((size_t)out_w * stride_w, 8);
+        const uint64_t items = (uint64_t)batch * out_ch * strips * groups;
         if (items < ((uint64_t)1 << 31)) {
             const unsigned blocks = (unsigned)std::min<uint64_t>((items + 255) / 256, 65536ull * 8);
-            if (stride_h == 1) {
-                CM_LAUNCH("conv_dw3_kernel", (conv_dw3_kernel<1, 1, 8>), dim3(blocks), dim3(256), 0, s, x, w, bptr, y,
-                          (uint32_t)items, strips, out_ch, in_h, in_w, out_h, out_w, pad_top, pad_left, 16u, cs, y_cn,
-                          y_gs, wrap32 ? 1u : 0u, lo, hi);
-            } else {
-                CM_LAUNCH("conv_dw3_kernel", (conv_dw3_kernel<2, 2, 4>), dim3(blocks), dim3(256), 0, s, x, w, bptr, y,
-                          (uint32_t)items, strips, out_ch, in_h, in_w, out_h, out_w, pad_top, pad_left, 16u, cs, y_cn,
-                          y_gs, wrap32 ? 1u : 0u, lo, hi);
-            }
+#define CM_DW3(S_)                                                                                              \
+    CM_LAUNCH("conv_dw3_kernel", (conv_dw3_kernel<S_, R>), dim3(blocks), dim3(256), 0, s, x, w, bptr, y, (uint32_t)items, \
+              batch * out_ch, strips, groups, out_ch, in_h, in_w, out_h, out_w, pad_top, pad_left, 16u, cs, y_cn, y_gs, \
+              wrap32 ? 1u : 0u, lo, hi)
+            if (stride_h == 1) { CM_DW3(1); } else { CM_DW3(2); }
+#undef CM_DW3
             return CM_OK;
         }
     }
