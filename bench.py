@@ -299,11 +299,11 @@ def step_fields(args, ms):
             "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "int16"}
 
 
-def gemm_roofline(per_kernel, macs):
-    gemm_ms = per_kernel.get(GEMM_KERNEL, {}).get("ms", float("nan"))
+def gemm_roofline(per_kernel, macs, kernel=GEMM_KERNEL):
+    gemm_ms = per_kernel.get(kernel, {}).get("ms", float("nan"))
     achieved = 8.0 * macs / (gemm_ms * 1e-3) / 1e12
     return {"bound": "mfma", "achieved": round(achieved, 1), "peak": I8_PEAK_TOPS, "unit": "TFLOP/s",
-            "frac": round(achieved / I8_PEAK_TOPS, 4), "traffic": None, "kernel": GEMM_KERNEL,
+            "frac": round(achieved / I8_PEAK_TOPS, 4), "traffic": None, "kernel": kernel,
             "kernel_ms_per_step": gemm_ms, "ops_per_step": 8 * macs}
 
 
@@ -430,10 +430,18 @@ def conv_pointwise(sn) -> bool:
             and (sn.in_h, sn.in_w) == (sn.out_h, sn.out_w))
 
 
-def conv_on_gemm(sn) -> bool:
-    """A convolution the library runs on the plane GEMM (not depthwise, not a few-tap one)."""
+def conv_kernel(sn, cus: int) -> str:
+    """The kernel a graph's standard convolution runs on: a pointwise one straight from its pixels
+    (conv_point_kernel; past 64 input channels while its weights or its tiles are few), other
+    few-tap ones on the VALU, the rest on the plane GEMM."""
     from cormorant_amd import units
-    return not sn.is_depthwise and not units.conv_small(sn.in_ch, sn.kh, sn.kw, sn.out_ch, sn.batch)
+    if conv_pointwise(sn):
+        tiles = -(-sn.out_ch // 32) * -(-sn.batch * sn.out_h * sn.out_w // 32)
+        if sn.in_ch <= 64 or (sn.out_ch <= 1280 and sn.in_ch * sn.out_ch < 1 << 19) or tiles <= 2 * cus:
+            return "conv_point_kernel"
+        return "gemm_planes_kernel"
+    small = units.conv_small(sn.in_ch, sn.kh, sn.kw, sn.out_ch, sn.batch)
+    return "conv_small_kernel" if small else "gemm_planes_kernel"
 
 
 def matmul_on_skinny(sn) -> bool:
@@ -446,15 +454,20 @@ def matmul_on_skinny(sn) -> bool:
 
 def write_conv_roofline(path, g, per_kernel, batch, ms):
     """A markdown table of every convolution and product launch of one forward against its own
-    roofline: the GEMM launches (and the fold split before each folded 1x1) against
+    roofline: the matrix-unit launches (and the fold split before a 1x1 on the plane GEMM) against
     max(i8-MFMA time, HBM time) of their algorithmic work and bytes, the few-tap convolutions
     (VALU) against their HBM time.  Algorithmic bytes: each operand once at int16, the output
-    once.  The i-th GEMM / fold / few-tap launch is the i-th node of the graph that makes one."""
-    gemm = per_kernel.get("gemm_planes_kernel", {}).get("each", [])
-    fold = per_kernel.get("split_fold_kernel", {}).get("each", [])
-    small = per_kernel.get("conv_small_kernel", {}).get("each", [])
+    once.  The i-th launch of a kernel is the i-th node of the graph that makes one."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    each = {k: iter(per_kernel.get(k, {}).get("each", []))
+            for k in ("gemm_planes_kernel", "split_fold_kernel", "conv_point_kernel", "conv_small_kernel")}
+
+    def next_us(kern):
+        return next(each[kern], float("nan")) * 1e3
+
     skinny = per_kernel.get("skinny_planes_kernel", {}).get("each", [])
-    gi = fi = si = ki = 0
+    ki = 0
     rows = []
     for sn in g.nodes:
         kind = type(sn).__name__
@@ -463,18 +476,9 @@ def write_conv_roofline(path, g, per_kernel, batch, ms):
             k = sn.in_ch * sn.kh * sn.kw
             byt = 2 * (sn.out_ch * k + sn.batch * sn.in_ch * sn.in_h * sn.in_w + sn.out_ch * n)
             shape = f"{sn.in_ch}x{sn.in_h}x{sn.in_w} -> {sn.out_ch}, {sn.kh}x{sn.kw} s{sn.stride_h}"
-            if conv_on_gemm(sn):
-                split_us = None
-                if conv_pointwise(sn):
-                    split_us = fold[fi] * 1e3 if fi < len(fold) else float("nan")
-                    fi += 1
-                us = gemm[gi] * 1e3 if gi < len(gemm) else float("nan")
-                gi += 1
-                rows.append((sn.output.onnx_name, shape, "gemm_planes_kernel", us, conv_macs(sn), byt, split_us))
-            else:
-                us = small[si] * 1e3 if si < len(small) else float("nan")
-                si += 1
-                rows.append((sn.output.onnx_name, shape, "conv_small_kernel", us, conv_macs(sn), byt, None))
+            kern = conv_kernel(sn, cus)
+            split_us = next_us("split_fold_kernel") if kern == "gemm_planes_kernel" and conv_pointwise(sn) else None
+            rows.append((sn.output.onnx_name, shape, kern, next_us(kern), conv_macs(sn), byt, split_us))
         elif kind == "MatmulNode":
             a, b = sn.inputs
             n, kk, m = int(a.shape[-2]), int(a.shape[-1]), int(b.shape[-1])
@@ -484,16 +488,15 @@ def write_conv_roofline(path, g, per_kernel, batch, ms):
                 ki += launches
                 kern = "skinny_planes_kernel" if launches == 1 else f"skinny_planes_kernel x {launches}"
             else:
-                us = gemm[gi] * 1e3 if gi < len(gemm) else float("nan")
-                gi += 1
                 kern = "gemm_planes_kernel"
+                us = next_us(kern)
             rows.append((sn.output.onnx_name, f"{n}x{kk} . {kk}x{m}", kern, us, n * kk * m,
                          2 * (n * kk + kk * m + n * m), None))
     tot_us = tot_bound = 0.0
     lines = [f"| output | shape (batch {batch}) | kernel | us | G MAC | MB | MFMA-bound us | HBM-bound us | "
              "of roofline | fold split us (HBM-bound us) |", "|---|---|---|---|---|---|---|---|---|---|"]
     for name, shape, kern, us, macs, byt, split_us in rows:
-        t_mfma = 8.0 * macs / (I8_PEAK_TOPS * 1e12) * 1e6 if kern.startswith(("gemm", "skinny")) else 0.0
+        t_mfma = 8.0 * macs / (I8_PEAK_TOPS * 1e12) * 1e6 if kern.startswith(("gemm", "conv_point", "skinny")) else 0.0
         t_hbm = byt / (HBM_PEAK_GBS * 1e9) * 1e6
         bound = max(t_mfma, t_hbm)
         split = ""
@@ -530,7 +533,7 @@ def mobilenet_bench(args, torch, np):
     sim = Simulator(g)
     out_name = g.output_tensors[0].onnx_name
     x = sim._to_device(sim._tensor("input"), inputs["input"])
-    each = (("gemm_planes_kernel", "split_fold_kernel", "conv_small_kernel", "skinny_planes_kernel")
+    each = (("gemm_planes_kernel", "split_fold_kernel", "conv_point_kernel", "conv_small_kernel", "skinny_planes_kernel")
             if args.per_launch else ())
     ms, per_kernel, out = run_graph(args, torch, sim, {"input": x}, out_name, each=each)
     if args.per_launch:
@@ -549,13 +552,13 @@ def mobilenet_bench(args, torch, np):
                    "batch": batch, "res": 224, "macs_per_step": macs},
         "kernels_ms_per_step": per_kernel,
     }
-    # the GEMM's share of the MACs: the standard / pointwise convolutions it runs (the few-tap
-    # convolutions run on the VALU, the classifier on the skinny products)
-    off_mfma = sum(conv_macs(sn) for sn in g.nodes if type(sn).__name__ == "ConvNode" and not conv_on_gemm(sn))
-    off_mfma += sum(int(sn.inputs[0].shape[-2]) * int(sn.inputs[0].shape[-1]) * int(sn.inputs[1].shape[-1])
-                    for sn in g.nodes if type(sn).__name__ == "MatmulNode" and matmul_on_skinny(sn))
-    result["roofline"] = gemm_roofline(per_kernel, macs - off_mfma)
-    result["roofline"]["macs_on_mfma"] = macs - off_mfma
+    # the pointwise convolutions' share of the MACs (the depthwise and the few-tap ones run on the VALU,
+    # the classifier on the skinny products, what is left on the plane GEMM)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    point = sum(conv_macs(sn) for sn in g.nodes if type(sn).__name__ == "ConvNode" and not sn.is_depthwise
+                and conv_kernel(sn, cus) == "conv_point_kernel")
+    result["roofline"] = gemm_roofline(per_kernel, point, "conv_point_kernel")
+    result["roofline"]["macs_on_mfma"] = point
     ok = None
     if not args.no_cpu_baseline:
         from oracle import graph_sim
