@@ -376,9 +376,12 @@ __global__ __launch_bounds__(64 * NW) void ro_norm_fast_kernel(Job j, const uint
 // row leaves each lane a long serial chain of 64-bit arithmetic over several units at a few
 // wavefronts per SIMD; here a lane holds one or two units and a row has TPR / 64 wavefronts.
 // ADDX and PL as in ro_norm_fast_kernel: the residual add's int32 output formed in registers,
-// stored and normalised; the output's byte planes and per-slab row sums for the next GEMM.
+// stored and normalised; the output's byte planes and per-slab row sums for the next GEMM.  The
+// bounds hold four wavefronts a SIMD (the launch's four workgroups a CU): ADDX without PL would take
+// 132 registers and three (19204 x 1520 with the residual add, RMS: 112.7 us, 84.7 at four).
 template <int AK, int UPL, bool ADDX, bool PL, int TPR>
-__global__ __launch_bounds__(TPR) void ro_norm_wg_kernel(Job j, const uint8_t* __restrict__ params, uint8_t* pram_dst,
+__global__ __launch_bounds__(TPR, UPL > 1 ? 2 : (ADDX && PL ? 3 : 4)) void ro_norm_wg_kernel(
+                                                         Job j, const uint8_t* __restrict__ params, uint8_t* pram_dst,
                                                          uint32_t p_entries, bool bcast,
                                                          const uint8_t* __restrict__ tab, Job ja,
                                                          const uint8_t* __restrict__ pa, bool bca, APlanes po) {
