@@ -2660,31 +2660,55 @@ int run_split(const Src& src, uint64_t src_slice, Planes& pl, hipStream_t s) {
 }
 
 // k slices of a wrap-mode product of `tiles` tiles of a plan: as many as fill the workgroup slots
-// once, at least 12 k steps each (a slice's partials cost a round trip to the coherence point:
-// 128 x 3072 x 768 on 64 x 64 tiles takes 11.9 us in 2 slices, 9.7 in 4 (12 steps), 10.6 in 8).
+// once, each of at least 12 k steps of a 64 x 64 tile or 8 of a larger one (a slice's partials cost a
+// round trip to the coherence point: 128 x 3072 x 768 on 64 x 64 tiles takes 11.9 us in 2 slices, 9.7 in 4
+// of 12 steps, 10.6 in 8; 1280 x 1536 x 2048 on 128 x 128 tiles 31.9 unsplit, 30.7 in 3 of 8).
 uint32_t gemm_slices(const GemmPlan& pl, uint64_t tiles, uint32_t nk, uint32_t cus) {
-    return (uint32_t)std::min<uint64_t>((uint64_t)cus * pl.per_cu / tiles, nk / 12);
+    return (uint32_t)std::min<uint64_t>((uint64_t)cus * pl.per_cu / tiles, nk / (pl.tm == 64 ? 12 : 8));
 }
 
 // The tile of an n x m output of `batch` slices and nk k steps, where a product by the int32-wrap
 // rule (`wrap`) may be split over k; measured (us, k = 768 unless given):
 //   - 64 x 64 tiles on the four-stage ring while they fit the slots once (two workgroups a unit):
 //     128 x 2304 6.9 (128 x 128 tiles, two stages: 13.2), 1040 x 768 7.7 (15.2), 512 x 3072 10.0
-//     (13.6), 1536 x 768 of k 3072 24.5 (25.7 split in 3); and for outputs of at most 64 rows at any
-//     width: 24 x 100352 of k 192 18.9 (64 x 128 tiles, two stages: 23.6);
+//     (13.6); and for outputs of at most 64 rows at any width: 24 x 100352 of k 192 18.9 (64 x 128
+//     tiles, two stages: 23.6);
+//   - but 128 x 128 tiles, split over k, for a wrap product whose 64 x 64 tiles would take at most 2 slices
+//     of 48 steps or more: they read half the bytes a product (in 3 slices or more the 64 x 64 tiles stay
+//     ahead: 384 x 1024 of k 16384 45.3 in 5, 57.1).  On the ring, one workgroup a unit, where its slices fill
+//     the units no worse than two a unit of the two-stage kernel do and have under 64 steps: 512 x 4096 of k
+//     4096 43.8 in 2 (64 x 64 48.8; two stages, in 4, 44.5), 640 x 2048 of k 8192 56.1 in 3 (77.0; in 6, 56.5),
+//     1024 x 1024 of k 8192 49.4 in 4 (54.6; in 8, 52.2), 256 x 4096 of k 4096, 32 steps a slice, 30.5 in 4 (31.0).
+//     Else the two stages: 1536 x 1024 of k 4096 41.6 in 5 (44.9; the ring in 2, 43.7), 2048 x 1024 of k 16384
+//     143.5 in 4 (171.3; 151.2);
 //   - 128 x 128 tiles on the ring with 8 waves while they fit one to a unit: 1040 x 2304 15.1 (two
 //     stages 16.7), 576 x 6272 of k 128 8.0 (11.8), 3072 x 768 14.4 (14.3); but a wrap product that
 //     splits in 3 or more keeps the two-stage kernel, two workgroups a unit: 3072 x 768 of k 3072
-//     37.1 (ring unsplit 42.6), while 4992 x 768 of k 3072 takes 48.8 on the ring, 50.6 split in 2;
+//     45.0 (ring unsplit 52.6), while 3072 x 1024 of k 4096 takes 68.3 on the ring, 70.1 split in 2; in 2
+//     slices of 48 steps or more where they fill 15 of 16 slots: 2048 x 2048 of k 8192 129.2 (142.4), of
+//     k 4096 73.2 (72.7);
 //   - above, 256 x 128 tiles (one workgroup of 8 waves a unit, three stages) where their rounds
 //     over the units cost no more than the 128 x 128 tiles' (a round of them takes 22 - 25, of 128
-//     x 128 tiles 12.6 per tile a unit): 3072 x 2304 24.7 (26.7), 3072 x 3072 44.2 (37.8).
+//     x 128 tiles 12.6 per tile a unit): 3072 x 2304 24.7 (26.7), 3072 x 3072 44.2 (37.8); of 8 steps or
+//     fewer, where a workgroup alone on its unit pays its start and its stores in full, only a single round
+//     without a padded half tile: 1024 x 8192 of k 512 26.2 (26.8), 640 x 8192 of k 512 26.3 (24.2), 4096 x 6000 of
+//     k 256 50.4 (45.0).
 GemmPlan gemm_plan(uint32_t n, uint32_t m, uint32_t batch, uint32_t nk, bool wrap, uint32_t cus) {
     auto tiles = [&](const GemmPlan& pl) { return (uint64_t)ceil_div(n, pl.tm) * ceil_div(m, pl.tn) * batch; };
-    if (n <= 64 || tiles(kRing64) <= 2ull * cus) return kRing64;
-    const uint64_t t128 = tiles(kPlan128);
-    if (t128 <= cus) return wrap && gemm_slices(kPlan128, t128, nk, cus) >= 3 ? kPlan128 : kRing128;
-    return 2 * ((tiles(kPlan256) + cus - 1) / cus) <= (t128 + cus - 1) / cus ? kPlan256 : kPlan128;
+    auto slices = [&](const GemmPlan& pl) { return std::max(1u, gemm_slices(pl, tiles(pl), nk, cus)); };
+    const uint64_t t128 = tiles(kPlan128), t256 = tiles(kPlan256);
+    if (n <= 64 || tiles(kRing64) <= 2ull * cus) {
+        const uint32_t few = slices(kRing64);
+        if (n <= 64 || !wrap || few > 2 || nk / few < 48) return kRing64;
+        const uint32_t two = slices(kPlan128), ring = slices(kRing128);
+        return 2 * ring >= two && nk / ring < 64 ? kRing128 : kPlan128;
+    }
+    if (t128 <= cus) {
+        const uint32_t two = slices(kPlan128);
+        return wrap && (two >= 3 || (two == 2 && nk >= 96 && 16 * t128 >= 15ull * cus)) ? kPlan128 : kRing128;
+    }
+    if (2 * ((t256 + cus - 1) / cus) > (t128 + cus - 1) / cus) return kPlan128;
+    return nk > 8 || (t256 <= cus && 2 * t256 == t128) ? kPlan256 : kPlan128;
 }
 
 // Tile columns of the strips tile_pos walks: the square root of an XCD's share of the tiles.

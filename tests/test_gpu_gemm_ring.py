@@ -27,7 +27,10 @@ SHAPES = [(33, 64 * s, 65, 1) for s in range(1, 11)] + [(130, 64 * s - 24, 66, 2
     (2048, 136, 1024, 1), (2049, 136, 1024, 1),           # 512 tiles of 64 x 64, then one row more
     (2048, 72, 2048, 1), (2048, 72, 2049, 1),             # 256 tiles of 128 x 128, then past one a unit
     (2050, 72, 4100, 1), (513, 72, 2050, 5),              # rounds of 256-row tiles, a batch
-    (64, 1600, 72, 1), (300, 2500, 200, 1), (2100, 2560, 1100, 1)]   # wrap products split over k
+    (64, 1600, 72, 1), (300, 2500, 200, 1), (2100, 2560, 1100, 1),   # wrap products split over k
+    (1100, 3100, 1050, 1), (1500, 3100, 1000, 1),         # past 48 steps: 128 x 128 tiles on the ring in 3, two stages in 5
+    (330, 6500, 1025, 2), (1270, 1500, 2040, 1),          # the ring in 4 of 26 steps; two stages in 3 of 8
+    (600, 500, 8100, 1), (1024, 300, 8190, 1)]            # at most 8 steps: 128-row tiles, one round of 256-row ones
 
 
 @pytest.mark.parametrize("wrap", [0, 1])
