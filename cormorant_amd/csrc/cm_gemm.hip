@@ -2025,6 +2025,82 @@ __global__ __launch_bounds__(256) void conv_dw3v_kernel(const int16_t* __restric
     }
 }
 
+// Depthwise 3x3, dilation 1, stride S both ways, over so few columns that the launch is its latency, or
+// over rows of at most 5: each lane computes R output rows of one column (a vertical strip) from the (R - 1) S + 3 input rows' three
+// taps, a load a tap with no edge to mend.  One workgroup a unit or fewer, us (conv_dw3_kernel): one
+// image of 96 channels at 14 x 14, stride 2 3.9 (4.3), of 960 at 7 x 7 4.0 (4.25), 32 images of 32 at 3 x 3 3.8
+// (5.3).  Sums as conv_dw3v_kernel.
+template <int S, int R>
+__global__ __launch_bounds__(256) void conv_dw3_strip_kernel(const int16_t* __restrict__ x, const int16_t* __restrict__ w,
+                                                             const int16_t* __restrict__ bias, int16_t* __restrict__ y,
+                                                             uint32_t items, uint32_t strips, uint32_t ch,
+                                                             uint32_t in_h, uint32_t in_w, uint32_t out_h,
+                                                             uint32_t out_w, uint32_t pt, uint32_t pl, uint32_t dws,
+                                                             uint32_t cs, uint32_t cn, uint32_t gs, uint32_t wrap,
+                                                             int32_t lo, int32_t hi) {
+    constexpr int NR = (R - 1) * S + 3;
+    const uint32_t per_plane = strips * out_w;
+    for (uint32_t it = blockIdx.x * blockDim.x + threadIdx.x; it < items; it += gridDim.x * blockDim.x) {
+        const uint32_t p = it / per_plane, rem = it - p * per_plane;
+        const uint32_t sidx = rem / out_w, ow = rem - sidx * out_w;
+        const uint32_t nb = p / ch, c = p - nb * ch;
+        const int16_t* xp = x + (uint64_t)p * in_h * in_w;
+        const int16_t* wp = w + (uint64_t)c * dws;
+        int wv[9];
+        uint32_t wabs = 0;
+#pragma unroll
+        for (int i = 0; i < 9; i++) {
+            wv[i] = wp[i];
+            wabs += (uint32_t)(wv[i] < 0 ? -wv[i] : wv[i]);
+        }
+        const int b0 = bias ? (int)bias[c] : 0;
+        const int oh0 = (int)(sidx * R);
+        const int ih0 = oh0 * S - (int)pt, iw0 = (int)(ow * S) - (int)pl;
+        bool cv[3];
+#pragma unroll
+        for (int b = 0; b < 3; b++) cv[b] = (uint32_t)(iw0 + b) < in_w;
+        int v[NR][3];
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int ih = ih0 + r;
+            const bool rv = (uint32_t)ih < in_h;
+            const int16_t* xr = xp + (int64_t)ih * in_w + iw0;
+#pragma unroll
+            for (int b = 0; b < 3; b++) v[r][b] = (rv && cv[b]) ? (int)xr[b] : 0;
+        }
+        const uint64_t bound = (uint64_t)wabs * 32768u + (uint64_t)(b0 < 0 ? -b0 : b0) * 256u;
+        int out[R];
+        if (wrap || bound < ((uint64_t)1 << 31)) {
+#pragma unroll
+            for (int i = 0; i < R; i++) {
+                uint32_t acc = (uint32_t)b0 << 8;
+#pragma unroll
+                for (int a = 0; a < 3; a++)
+#pragma unroll
+                    for (int b = 0; b < 3; b++) acc += (uint32_t)(v[i * S + a][b] * wv[a * 3 + b]);
+                out[i] = clamp_i32((int)acc >> 8, lo, hi);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < R; i++) {
+                long long acc = (long long)b0 * 256;
+#pragma unroll
+                for (int a = 0; a < 3; a++)
+#pragma unroll
+                    for (int b = 0; b < 3; b++) acc += (long long)v[i * S + a][b] * wv[a * 3 + b];
+                const long long q = acc >> 8;
+                out[i] = (int)(q > hi ? hi : (q < lo ? lo : q));
+            }
+        }
+        const uint64_t plane = (uint64_t)out_h * out_w;
+        const uint64_t base = cn ? (uint64_t)(c % cn) * cs + (uint64_t)(c / cn) * gs : (uint64_t)c * cs;
+        int16_t* yp = y + (uint64_t)nb * ch * plane + base + ow;
+#pragma unroll
+        for (int i = 0; i < R; i++)
+            if ((uint32_t)(oh0 + i) < out_h) yp[(uint64_t)(oh0 + i) * out_w] = (int16_t)out[i];
+    }
+}
+
 // Depthwise 3x3, dilation 1, stride S both ways, at any width (the MobileNet blocks): a lane computes R rows
 // of 8 / S output columns from the 10 input columns 8 j - pad_left .. + 9 of every input row, loaded as 20
 // bytes at any alignment.  A load a tap kept the address unit busy: 27 two-byte loads for 4 outputs at
@@ -3295,7 +3371,24 @@ int conv_run(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y
             return CM_OK;
         }
     }
-    if (dw3 && stride_h == stride_w && stride_h <= 2 && (uint64_t)in_h * in_w < (1u << 29) && (uint64_t)batch * out_ch * in_h * in_w >= 10 && out_h < (1u << 27) && out_w < (1u << 27) &&
+    if (dw3 && stride_h == stride_w && stride_h <= 2) {
+        // one workgroup a unit or fewer (at 1.3 a unit 384 channels of 32 images at 7 x 7 take 4.65 us, 4.49 below),
+        // or rows that fill no more than half of a lane's 10 columns (960 channels of 64 images, us, and below:
+        // 12 x 3 8.4, 9.3; 3 x 3 4.9, 6.4; 5 x 5 6.85, 7.05)
+        const uint32_t R = stride_h == 1 ? 8 : 4, strips = ceil_div(out_h, R);
+        const uint64_t items = (uint64_t)batch * out_ch * strips * out_w;
+        if (items < (1ull << 31) && (in_w <= 5 || items <= 256ull * st->cus)) {
+#define CM_DW3S(S_, R_)                                                                                         \
+    CM_LAUNCH("conv_dw3_kernel", (conv_dw3_strip_kernel<S_, R_>), dim3(std::min(ceil_div(items, 256), 65536u * 8)), dim3(256), 0, s, x, w, \
+              bptr, y, (uint32_t)items, strips, out_ch, in_h, in_w, out_h, out_w, pad_top, pad_left, 16u, cs, y_cn, y_gs, \
+              wrap32 ? 1u : 0u, lo, hi)
+            if (stride_h == 1) { CM_DW3S(1, 8); } else { CM_DW3S(2, 4); }
+#undef CM_DW3S
+            return CM_OK;
+        }
+    }
+    if (dw3 && stride_h == stride_w && stride_h <= 2 && (uint64_t)in_h * in_w < (1u << 29) &&
+        (uint64_t)batch * out_ch * in_h * in_w >= 10 && out_h < (1u << 27) && out_w < (1u << 27) &&
         pad_top < (1u << 28) && pad_left < (1u << 28) && (uint64_t)batch * out_ch < (1u << 31)) {
         constexpr uint32_t R = 2;
         const uint32_t strips = ceil_div(out_h, R), groups = ceil_div((size_t)out_w * stride_w, 8);

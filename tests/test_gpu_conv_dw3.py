@@ -1,7 +1,8 @@
-"""The depthwise 3x3 strips of 8 input columns, bit for bit against the oracle: rows that end anywhere in
-a lane's columns, output rows past its strip, planes too small for its words, one plane and many (the
-words beyond a plane's ends belong to its neighbours), paddings up to one past the kernel, both strides,
-both output rules, activations, weights past the int32 bound, outputs on a y pattern."""
+"""The depthwise 3x3 kernels of strides 1 and 2, bit for bit against the oracle: few planes (a strip of one
+column a lane) and as many as take the lanes of 8 input columns, rows that end anywhere in a lane's
+columns, output rows past its strip, planes too small for its words, one plane and many (the words
+beyond a plane's ends belong to its neighbours), paddings up to one past the kernel, both strides, both
+output rules, activations, weights past the int32 bound, outputs on a y pattern."""
 import numpy as np
 import pytest
 
@@ -20,15 +21,26 @@ def U():
     return units
 
 
+def _past_strips(batch, ch, oh, ow, stride):
+    """The least channel count of at least ``ch`` past one workgroup a compute unit of the strip kernel
+    (256 lanes, a lane one column of 8 output rows, 4 at stride 2)."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return max(ch, 256 * cus // (batch * -(-oh // (8 if stride == 1 else 4)) * ow) + 1)
+
+
+@pytest.mark.parametrize("many", [False, True])
 @pytest.mark.parametrize("act,wrap,lim", [(0, 0, 32768), (2, 0, 3000), (1, 1, 32768)])
 @pytest.mark.parametrize("stride", [1, 2])
 @pytest.mark.parametrize("batch,ch,h,w,pt,pl,pb,pr", [
     (1, 1, 1, 1, 1, 1, 1, 1), (1, 3, 2, 2, 1, 1, 1, 1), (2, 5, 3, 3, 0, 0, 0, 0), (1, 2, 3, 9, 1, 0, 0, 1),
     (2, 7, 7, 7, 1, 1, 1, 1), (1, 4, 14, 14, 1, 1, 1, 1), (3, 2, 15, 8, 0, 1, 1, 0), (1, 3, 9, 17, 2, 2, 2, 2),
     (1, 2, 8, 16, 1, 1, 1, 1), (1, 3, 6, 13, 2, 1, 2, 3), (2, 3, 28, 28, 1, 1, 1, 1), (1, 2, 56, 40, 0, 0, 1, 1), (1, 2, 5, 6, 3, 4, 3, 4), (1, 1, 4, 33, 1, 12, 1, 12)])
-def test_dw3(U, oracle_lib, batch, ch, h, w, pt, pl, pb, pr, stride, act, wrap, lim):
+def test_dw3(U, oracle_lib, batch, ch, h, w, pt, pl, pb, pr, stride, act, wrap, lim, many):
     from cormorant_amd.packing import conv_weight_image
     oh, ow = (h + pt + pb - 3) // stride + 1, (w + pl + pr - 3) // stride + 1
+    if many:
+        ch = _past_strips(batch, ch, oh, ow, stride)
     rng = np.random.default_rng(ch + 7 * h + w + act + stride)
     x = rng.integers(-lim, lim, batch * ch * h * w).astype(np.int16)
     wt = rng.integers(-lim, lim, (ch, 1, 3, 3)).astype(np.int16)
@@ -46,13 +58,15 @@ def test_dw3(U, oracle_lib, batch, ch, h, w, pt, pl, pb, pr, stride, act, wrap, 
     assert (got[n:] == 0x5A5A).all()
 
 
+@pytest.mark.parametrize("many", [False, True])
 @pytest.mark.parametrize("h,w", [(9, 7), (10, 16)])
-def test_dw3_y_pattern(U, oracle_lib, h, w):
+def test_dw3_y_pattern(U, oracle_lib, h, w, many):
     """Output channel o at (o % 2) cs + (o / 2) gs."""
     from cormorant_amd.packing import conv_weight_image
     rng = np.random.default_rng(w)
-    ch, plane = 6, h * w
-    cs, cn, gs = 3 * (plane + 5), 2, plane + 5
+    ch = _past_strips(1, 6, h, w, 1) + 1 & ~1 if many else 6
+    plane = h * w
+    cs, cn, gs = ch // 2 * (plane + 5), 2, plane + 5
     x = rng.integers(-2000, 2000, ch * plane).astype(np.int16)
     img = np.asarray(conv_weight_image(rng.integers(-2000, 2000, (ch, 1, 3, 3)).astype(np.int16), True)).reshape(-1)
     want = oracle_lib.conv(x, img, None, ch * plane, 1, ch, h, w, ch, h, w, 3, 3, 1, 1, 1, 1, 1, 1, 0, 1)
