@@ -194,8 +194,10 @@ __device__ __forceinline__ void stage_addx_params(uint4* lds, const uint8_t* par
         const uint32_t w = (uint32_t)q.sa | ((uint32_t)q.sb << 8) | ((uint32_t)q.sc << 16) |
                            ((base && q.sb <= 30) ? 1u << 24 : 0u) | ((base && q.sb <= 46) ? 1u << 25 : 0u);
         const u64 bs = bq_sh <= 40 ? (u64)(q.bq * ((i64)1 << bq_sh) + norm_half((uint32_t)q.sc)) : 0;
-        const bool plain = bq_sh <= 40 && q.sa == 0 && q.sc == 0 && q.sb <= 15 && bs + (1u << 30) < (1ull << 31);
-        lds[pslot(i, units)] = make_uint4(w | (plain ? 1u << 26 : 0u), (uint32_t)q.g, (uint32_t)bs, (uint32_t)(bs >> 32));
+        // sa = sc = 0, sb <= 15 and the bias (|bs| < 2^62) in 31 bits as one test, bq_sh where it is used: tested one by
+        // one it took the staging of 4096 columns from 8.7 to 9.4 us
+        const uint32_t far = (w & 0x3F303Fu) | (uint32_t)((bs + (1u << 30)) >> 31);
+        lds[pslot(i, units)] = make_uint4(w | (far == 0 ? 1u << 26 : 0u), (uint32_t)q.g, (uint32_t)bs, (uint32_t)(bs >> 32));
     });
 }
 
@@ -228,7 +230,7 @@ __device__ __forceinline__ void addx_unit(const int (&x)[8], const int (&y)[8], 
             e[l] = ro_lds[bcast ? 0u : l * units + u];
             all &= e[l].x;
         }
-        if (__all(all != 0) && !scale) {
+        if (__all(all != 0) && !scale && j.bq_sh <= 40) {
 #pragma unroll
             for (int l = 0; l < 8; l++) {
                 const int t = (BEN ? (int)((uint32_t)y[l] << ((e[l].x >> 8) & 15)) : 0) + (int)e[l].z;

@@ -1,7 +1,8 @@
 """NORM and the residual add at the edges of their short arithmetic, bit for bit against the oracle:
 row magnitudes on both sides of the short sums' bound (2^21 .. 2^23 and far past it), one row short
 and the next long in one call, output shifts on both sides of 32 / 33 and at 61, ties, both signs of
-saturation; residual adds with and without the plain form (shifts, biases past 2^30, RELU)."""
+saturation; residual adds with and without the plain form (shifts, biases past 2^30
+and shifted past the staged form's 40, RELU)."""
 import numpy as np
 import pytest
 
@@ -63,7 +64,7 @@ def test_norm_magnitudes(U, oracle_lib, rows, n, mag, sc, rms):
 @pytest.mark.parametrize("rows,n,sa,sb,sc,bq,bq_sh,relu", [
     (300, 768, 0, 2, 0, 1 << 20, 5, False), (20, 768, 0, 15, 0, 1 << 18, 12, True), (300, 512, 0, 3, 0, 1 << 21, 11, False),
     (300, 768, 0, 16, 0, 1 << 10, 0, False), (9, 256, 1, 2, 0, 1 << 12, 0, False), (9, 256, 0, 2, 1, 1 << 12, 3, True),
-    (3100, 768, 0, 4, 0, 1 << 16, 0, False)])
+    (3100, 768, 0, 4, 0, 1 << 16, 0, False), (9, 256, 0, 2, 0, 1 << 21, 40, False), (20, 512, 0, 2, 0, 3, 41, True)])
 def test_residual_add_then_norm(U, oracle_lib, rows, n, sa, sb, sc, bq, bq_sh, relu):
     from cormorant_amd import rowops_nodes as rn
     rng = np.random.default_rng(rows + n + sb)
