@@ -192,7 +192,7 @@ class Simulator:
                 i += 1
                 continue
             chain = self._attn_chain(i - 1)
-            if chain is not None:
+            if chain is not None and all(self._aligned(t, raw) for t in (chain[0].inputs[0], chain[2].inputs[1])):
                 # a prompt's attention, group by group: one launch, the merged output alone
                 self._attn_chain_run(chain, raw)
                 i += 3 * chain[0].KV
@@ -647,6 +647,8 @@ class Simulator:
             if out is not None:
                 raw[name] = out.reshape(-1)
         elif isinstance(sn, AttentionNode):
+            if sn.seq not in self._ATT_SEQ and not self._aligned(sn.inputs[0], raw):
+                return False
             # o itself only where something besides the output projection's planes reads it
             self._attention(sn, raw, planes=planes, write_o=not self._planes_only(name))
             if self._attention_out is not None:
@@ -1254,7 +1256,8 @@ class Simulator:
                 return o
             units.attention(x, o, B, T, H, hd, ld, sn.q_off, sn.k_off, sn.v_off, cols, sn.cm, sn.cfg)
             return o
-        if self._att_any(sn) and ld % 8 == 0 and sn.q_off % 8 == 0 and sn.k_off % 8 == 0 and sn.v_off % 8 == 0:
+        if (self._att_any(sn) and ld % 8 == 0 and sn.q_off % 8 == 0 and sn.k_off % 8 == 0 and sn.v_off % 8 == 0
+                and self._aligned(xt, raw)):
             view = lambda off: (off, ld, T * ld, hd)                                     # noqa: E731
             units.attention_strided(x, x, x, o, T, T, B * H, H, view(sn.q_off), view(sn.k_off), view(sn.v_off),
                                     (0, cols, T * cols, hd), sn.cm, sn.cfg, T, planes=planes, planes_rows=B * T)
@@ -1288,6 +1291,11 @@ class Simulator:
         """An AttentionNode cm_attention_strided takes (other lengths than _ATT_SEQ)."""
         return (sn.head_dim == 64 and sn.seq % 16 == 0 and 0 < sn.seq <= 1024 and sn.batch * sn.heads <= 65535
                 and 0 < (sn.cfg >> 8) & 31)
+
+    def _aligned(self, t: TensorInfo, raw) -> bool:
+        """A tensor's device image starts on a 16-byte word, as the fused attention reads it (a caller's own
+        buffer may not: its attention then runs node by node)."""
+        return self._get(t, raw).data_ptr() % 16 == 0
 
     def _attn_chain(self, i: int):
         """The attention of a prompt (or an encoder's prep chain) that starts at node ``i``: per KV group,

@@ -124,3 +124,55 @@ def test_encoder_odd_length(U, batch, seq):
     got = Simulator(g)._forward_pass(inputs)
     for name, v in got.items():
         np.testing.assert_array_equal(v, want[name].reshape(v.shape), err_msg=name)
+
+
+def _off_word(t):
+    """The same values in a buffer that starts two bytes past a 16-byte word."""
+    import torch
+    v = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")[1:1 + t.numel()]
+    return v.copy_(t.reshape(-1))
+
+
+@pytest.mark.parametrize("keep", [None, []])
+@pytest.mark.parametrize("planes", [False, True])
+def test_encoder_unaligned_input(U, oracle_lib, keep, planes):
+    """A caller's buffer off a 16-byte word, at a length only the strided kernel takes fused: the node by
+    node pass, also where the next MatMul takes the output's planes."""
+    import torch
+    from cormorant_amd.graph import AttentionNode, Graph, MatmulNode, TensorInfo
+    from cormorant_amd.simulate import Simulator
+    rng = np.random.default_rng(5)
+    B, T, H = 3, 48, 2
+    x, o = TensorInfo("x", [B * T, 3 * 64 * H], exp=8), TensorInfo("o", [B * T, 64 * H], exp=8)
+    nodes, out = [AttentionNode([x], o, batch=B, seq=T, heads=H, k_off=64 * H, v_off=128 * H)], o
+    if planes:
+        w = TensorInfo("w", [64 * H, 72], data=rng.integers(-40, 40, (64 * H, 72)) / 256.0, exp=8)
+        out = TensorInfo("y", [B * T, 72], exp=8)
+        nodes.append(MatmulNode([o, w], out))
+    g = Graph(nodes=nodes, input_tensors=[x], output_tensors=[out])
+    d = dev16(rint16(rng, x.numel, -2500, 2500), extra=0)
+    want = Simulator(g).forward_raw({"x": d}, keep=keep)[out.onnx_name]
+    got = Simulator(g).forward_raw({"x": _off_word(d)}, keep=keep)[out.onnx_name]
+    assert torch.equal(got, want)
+
+
+def test_prompt_unaligned_caches(U):
+    """The attention chain alone over a caller's caches off a 16-byte word."""
+    import torch
+    from cormorant_amd import models
+    from cormorant_amd.graph import AttnMergeNode, AttnSoftmaxNode, Graph, LlmAttnConvNode
+    from cormorant_amd.simulate import Simulator
+    S = models.LlamaShape(layers=1, batch=1, d=256, heads=4, kv=2, hd=64, ff=256, vocab=512, ctx=128)
+    w = models.smollm2_weights(S, 5)
+    _, _, exps = models.smollm2_decode(S, seed=5, weights=w)
+    nodes = [nd for nd in models.smollm2_prefill(S, 32, exps, w).nodes
+             if isinstance(nd, (LlmAttnConvNode, AttnSoftmaxNode, AttnMergeNode))]
+    kc, qx, vc = nodes[0].inputs[0], nodes[0].inputs[1], nodes[2].inputs[1]
+    g = Graph(nodes=nodes, input_tensors=[kc, qx, vc] + list(nodes[0].inputs[2:]), output_tensors=[nodes[-1].output])
+    rng = np.random.default_rng(8)
+    d = {t.onnx_name: dev16(rint16(rng, t.numel, -3000, 3000), extra=0) for t in (kc, qx, vc)}
+    host_in = {"pos": np.array([37]), "n": np.array([32])}
+    sim = Simulator(g)
+    want = sim.forward_raw({**d, **host_in}, keep=[])[nodes[-1].output.onnx_name]
+    got = sim.forward_raw({**{k: _off_word(v) for k, v in d.items()}, **host_in}, keep=[])[nodes[-1].output.onnx_name]
+    assert torch.equal(got.reshape(-1), want.reshape(-1))
