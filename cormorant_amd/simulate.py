@@ -960,19 +960,22 @@ class Simulator:
         xt, wt, ot = sn.inputs[0], sn.inputs[1], sn.output
         bias_t = sn.inputs[2] if sn.has_bias else None
         x = self._get(xt, raw)
-        img = self._images.get(wt.onnx_name)
+        # a pointwise one runs faster on the matrix units than on the VALU path, whatever its taps
+        # (24 -> 144 at 32 x 56 x 56 17.1 us against 25.4, 16 -> 96 at 32 x 112 x 112 28.2 against 35.0)
+        pointwise = ((sn.kh, sn.kw, sn.stride_h, sn.stride_w, sn.pad_top, sn.pad_left) == (1, 1, 1, 1, 0, 0)
+                     and (sn.in_h, sn.in_w) == (sn.out_h, sn.out_w))
+        # a constant weight of a standard convolution on the matrix units: its operand split once; a weight
+        # that another node reads on the VALU path has both images
+        planes = not sn.is_depthwise and wt.data is not None and (
+            pointwise or not units.conv_small(sn.in_ch, sn.kh, sn.kw, sn.out_ch, sn.batch))
+        key = wt.onnx_name + "#conv_planes" if planes else wt.onnx_name
+        img = self._images.get(key)
         if img is None:
             w = self._get(wt, raw).cpu().numpy().reshape(wt.shape)
             img = torch.from_numpy(conv_weight_image(w, sn.is_depthwise)).to(self.device)
-            # a pointwise one runs faster on the matrix units than on the VALU path, whatever its taps
-            # (24 -> 144 at 32 x 56 x 56 17.1 us against 25.4, 16 -> 96 at 32 x 112 x 112 28.2 against 35.0)
-            pointwise = ((sn.kh, sn.kw, sn.stride_h, sn.stride_w, sn.pad_top, sn.pad_left) == (1, 1, 1, 1, 0, 0)
-                         and (sn.in_h, sn.in_w) == (sn.out_h, sn.out_w))
-            if not sn.is_depthwise and wt.data is not None and (
-                    pointwise or not units.conv_small(sn.in_ch, sn.kh, sn.kw, sn.out_ch, sn.batch)):
-                # a constant weight of a standard convolution on the GEMM: its operand split once
+            if planes:
                 img = units.conv_w_planes(img, sn.out_ch, sn.in_ch, sn.kh, sn.kw)
-            self._images[wt.onnx_name] = img
+            self._images[key] = img
         bias = None
         if bias_t is not None:
             key = bias_t.onnx_name + "#bias"
@@ -981,7 +984,7 @@ class Simulator:
                 bias = torch.from_numpy(conv_bias_image(self._get(bias_t, raw).cpu().numpy())).to(self.device)
                 self._images[key] = bias
         y = self._new(ot if out_t is None else out_t)
-        if img.dtype == torch.uint8:
+        if planes:
             units.conv_planes(x.reshape(-1).contiguous(), img, bias, y, sn.batch, sn.in_ch, sn.in_h, sn.in_w,
                               sn.out_ch, sn.out_h, sn.out_w, sn.kh, sn.kw, sn.stride_h, sn.stride_w, sn.dilation_h,
                               sn.dilation_w, sn.pad_top, sn.pad_left, int(bias is not None),

@@ -81,3 +81,32 @@ def test_graph_pointwise(U, batch, hw):
     g = G.Graph([G.ConvNode([x, w], y)], [x], [y])
     feeds = {"x": np.round(rng.uniform(-4, 4, (batch, 24, hw, hw)) * 256) / 256}
     np.testing.assert_array_equal(Simulator(g).simulate(feeds)["y"], graph_sim.forward(g, feeds)["y"])
+
+
+def test_shared_weight_keeps_both_images(U, oracle_lib, monkeypatch):
+    """One weight read by a pointwise and by a stride-2 node of few taps, in either order: the one on the
+    matrix units, the other on its few-tap path."""
+    from cormorant_amd import units
+    from cormorant_amd.graph import ConvNode, Graph, TensorInfo
+    from cormorant_amd.packing import conv_weight_image
+    from cormorant_amd.simulate import Simulator
+    rng = np.random.default_rng(3)
+    x = TensorInfo("x", [2, 24, 6, 6])
+    w = TensorInfo("w", [40, 24, 1, 1], data=rng.integers(-300, 300, (40, 24, 1, 1)) / 256.0)
+    nodes = [ConvNode([x, w], TensorInfo("a", [2, 40, 6, 6])),
+             ConvNode([x, w], TensorInfo("b", [2, 40, 3, 3]), stride_h=2, stride_w=2)]
+    xr = rng.integers(-3000, 3000, x.numel).astype(np.int16)
+    img = np.asarray(conv_weight_image((w.data * 256).astype(np.int16), False)).reshape(-1)
+    want = {nd.output.onnx_name: oracle_lib.conv(xr, img, None, nd.output.numel, 2, 24, 6, 6, 40, nd.out_h, nd.out_w, 1, 1,
+                                                 nd.stride_h, nd.stride_w, 1, 1, 0, 0, 0, 0) for nd in nodes}
+    calls = []
+    for name in ("conv", "conv_planes"):
+        fn = getattr(units, name)
+        monkeypatch.setattr(units, name, lambda *a, fn=fn, name=name, **k: (calls.append(name), fn(*a, **k))[1])
+    for order in (nodes, nodes[::-1]):
+        calls.clear()
+        got = Simulator(Graph(nodes=list(order), input_tensors=[x], output_tensors=[n.output for n in order])).forward_raw(
+            {"x": dev16(xr, extra=0)})
+        assert calls == ["conv_planes" if nd is nodes[0] else "conv" for nd in order]
+        for k, v in want.items():
+            np.testing.assert_array_equal(host(got[k]).reshape(-1), v)
