@@ -3263,21 +3263,25 @@ int conv_split_w(const int16_t* w, Planes& A, uint32_t out_ch, uint32_t in_ch, u
     return run_split<SrcConvW, true>(SrcConvW{w, out_ch, in_ch, kh, kw, tiles, per_m, last}, 0, A, s);
 }
 
+// A 1x1 convolution from its pixels with the weights' planes A (point_path): no planes of the input.
+int conv_point(const int16_t* x, const Planes& A, const int16_t* bptr, int16_t* y, const ConvGeom& g,
+               const DeviceState* st, hipStream_t s, int32_t lo, int32_t hi) {
+    const uint32_t plane = g.plane();
+    // images whose input stays below the kernels' 32-bit byte offsets, one launch each
+    const uint32_t per = (uint32_t)std::min<uint64_t>(g.batch, 0xFFFFFFFFull / (2ull * g.in_ch * plane));
+    for (uint32_t i = 0; i < g.batch; i += per) {
+        const int rc = point_launch(x + (uint64_t)i * g.in_ch * plane, A, bptr, y + (uint64_t)i * g.out_ch * plane, g,
+                                    std::min(per, g.batch - i), st, s, lo, hi);
+        if (rc) return rc;
+    }
+    return CM_OK;
+}
+
 // The input's planes (im2col, or the folded 1x1 form) and the GEMM with the weights' planes A.
 int conv_gemm(const int16_t* x, const Planes& A, Planes& B, const int16_t* bptr, int16_t* y, const ConvGeom& g,
               const DeviceState* st, hipStream_t s, int32_t lo, int32_t hi) {
     const uint32_t plane = g.plane();
     const uint64_t img = (uint64_t)g.out_ch * plane;
-    if (point_path(g, st)) {
-        // images whose input stays below the kernels' 32-bit byte offsets, one launch each
-        const uint32_t per = (uint32_t)std::min<uint64_t>(g.batch, 0xFFFFFFFFull / (2ull * g.in_ch * plane));
-        for (uint32_t i = 0; i < g.batch; i += per) {
-            const int rc = point_launch(x + (uint64_t)i * g.in_ch * plane, A, bptr, y + i * img, g,
-                                        std::min(per, g.batch - i), st, s, lo, hi);
-            if (rc) return rc;
-        }
-        return CM_OK;
-    }
     if (g.fold()) {
         const uint32_t cols = g.batch * plane;
         if (B.lines_p / 64 >= 4 * st->cus) {
@@ -3448,16 +3452,18 @@ int conv_run(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y
     const ConvGeom g{batch, in_ch, in_h, in_w, out_ch, out_h, out_w, kh, kw, stride_h, stride_w, dilation_h,
                      dilation_w, pad_top, pad_left, cs, y_cn, y_gs, wrap32 ? 1u : 0u};
     const uint32_t kp = conv_kp(in_ch, kh, kw);
-    Planes B = conv_b_planes(g, kp);
-    Planes A = make_a_planes(out_ch, kp, 1, conv_plan(g, B, st));
+    const bool point = point_path(g, st);
+    Planes B = point ? Planes{} : conv_b_planes(g, kp);
+    Planes A = point ? make_planes(out_ch, kp, 1) : make_a_planes(out_ch, kp, 1, conv_plan(g, B, st));
     void* ws;
-    rc = workspace(st, A.bytes() + B.bytes(), &ws, s);
+    rc = workspace(st, A.bytes() + (point ? 0 : B.bytes()), &ws, s);
     if (rc) return rc;
     char* p = static_cast<char*>(ws);
     A.carve(p);
-    B.carve(p);
     rc = conv_split_w(w, A, out_ch, in_ch, kh, kw, s);
     if (rc) return rc;
+    if (point) return conv_point(x, A, bptr, y, g, st, s, lo, hi);
+    B.carve(p);
     return conv_gemm(x, A, B, bptr, y, g, st, s, lo, hi);
 }
 
@@ -3539,17 +3545,19 @@ int conv_planes_run(const int16_t* x, const void* w_planes, const int16_t* bias,
     const ConvGeom g{batch, in_ch, in_h, in_w, out_ch, out_h, out_w, kh, kw, stride_h, stride_w, dilation_h,
                      dilation_w, pad_top, pad_left, y_cs ? y_cs : plane, y_cn, y_gs, wrap32 ? 1u : 0u};
     const uint32_t kp = conv_kp(in_ch, kh, kw);
-    Planes B = conv_b_planes(g, kp);
+    const int16_t* bptr = has_bias ? bias : nullptr;
     Planes A = make_planes(out_ch, kp, 1, 256);
     char* q = static_cast<char*>(const_cast<void*>(w_planes));
     A.carve(q);
+    if (point_path(g, st)) return conv_point(x, A, bptr, y, g, st, s, lo, hi);
+    Planes B = conv_b_planes(g, kp);
     A.plan = conv_plan(g, B, st);
     void* ws;
     rc = workspace(st, B.bytes(), &ws, s);
     if (rc) return rc;
     char* p = static_cast<char*>(ws);
     B.carve(p);
-    return conv_gemm(x, A, B, has_bias ? bias : nullptr, y, g, st, s, lo, hi);
+    return conv_gemm(x, A, B, bptr, y, g, st, s, lo, hi);
 }
 
 }  // namespace

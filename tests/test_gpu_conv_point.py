@@ -110,3 +110,25 @@ def test_shared_weight_keeps_both_images(U, oracle_lib, monkeypatch):
         assert calls == ["conv_planes" if nd is nodes[0] else "conv" for nd in order]
         for k, v in want.items():
             np.testing.assert_array_equal(host(got[k]).reshape(-1), v)
+
+
+def test_no_workspace(U, oracle_lib):
+    """Captured before any other call of its size (the workspace cannot grow during a capture): a 1x1
+    convolution from its pixels has no planes of its input (412 MB of them here) to put there."""
+    import torch
+    rng = np.random.default_rng(11)
+    batch, h, out_ch = 64, 224, 3
+    n = batch * out_ch * h * h
+    x = rng.integers(-3000, 3000, batch * h * h).astype(np.int16)
+    from cormorant_amd.packing import conv_weight_image
+    img = np.asarray(conv_weight_image(rng.integers(-3000, 3000, (out_ch, 1, 1, 1)).astype(np.int16), False)).reshape(-1)
+    want = oracle_lib.conv(x, img, None, n, batch, 1, h, h, out_ch, h, h, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0)
+    planes, dx, y = U.conv_w_planes(dev16(img), out_ch, 1, 1, 1), dev16(x, extra=0), poisoned16(n)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        U.conv_planes(dx, planes, None, y, batch, 1, h, h, out_ch, h, h, 1, 1)
+    for _ in range(2):
+        y.fill_(0x5A5A)
+        graph.replay()
+        np.testing.assert_array_equal(host(y), want)
