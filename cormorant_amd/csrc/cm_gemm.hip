@@ -51,20 +51,15 @@ __device__ __forceinline__ uint32_t pack_lo(const int16_t* v) {   // 4 low bytes
 }
 
 // ---------------------------------------------------------------- operand sources
-// B side: columns of the output; B(kk, j) of the matmul images (the GEMV image of more than one
-// column group; the others have their own kernels).
-struct SrcMatB {
+// B side: columns of the output; B(kk, j) of the GEMV image of more than one column group (the other
+// matmul images have their own kernels).
+struct SrcGemvB {
     const int16_t* p;
-    uint32_t cols, k, m, layout, kw;   // layout 0 row-major, 1 packed, 2 gemv, 3 transposed [m][k]
-    __device__ bool real(uint32_t j, uint32_t kk) const { return j < cols && kk < k; }
+    uint32_t k, m, kw;
+    __device__ bool real(uint32_t j, uint32_t kk) const { return j < m && kk < k; }
     __device__ int16_t at(uint32_t j, uint32_t kk) const {
-        if (layout == 1) return p[((uint64_t)(j >> 5) * k + kk) * 32 + (j & 31)];
-        if (layout == 3) return p[(uint64_t)j * k + kk];
-        if (layout == 2 && kw > 1) {
-            uint32_t c = (kk / (16 * kw)) * 16 + (kk & 15), jj = (kk >> 4) % kw;
-            return p[((uint64_t)c * m + j) * kw + jj];
-        }
-        return p[(uint64_t)kk * m + j];
+        uint32_t c = (kk / (16 * kw)) * 16 + (kk & 15), jj = (kk >> 4) % kw;
+        return p[((uint64_t)c * m + j) * kw + jj];
     }
 };
 // Conv weights in the packed tile-major layout (ConvKernel.h:136-159) as GEMM rows:
@@ -1116,7 +1111,7 @@ __global__ __launch_bounds__(128 * WR, 8 / (2 * WR)) void gemm_planes_kernel(
 // network's 7 x 7 and 14 x 14 planes), where the kernel above is bound by latency: its two-stage
 // ring gives a copy less than one k step to arrive, a wavefront's fragment reads stall its own
 // MFMAs, and its 128 x 128 tiles leave most compute units idle.  Here a workgroup of WR x WC
-// waves computes (32 RB WR) x (32 CB WC) outputs over a ring of NST stages:
+// waves computes (32 RB WR) x (32 CB WC) outputs over a ring of NST = 4 stages:
 //   - copies run NST - 1 steps ahead, so that with few steps nearly all of k is in flight at once;
 //   - a wavefront reads the next step's fragments (both 32-k substeps) while its MFMAs of this step
 //     run, from a stage that landed one step earlier: one barrier a step, and no MFMA waits on LDS.
@@ -1136,7 +1131,7 @@ __device__ __forceinline__ void wait_steps(uint32_t later) {
     else wait_steps<NC, MAX - 1>(later);
 }
 
-template <int RB, int CB, int WR, int WC, int NST, class Epi>
+template <int RB, int CB, int WR, int WC, class Epi>
 __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_ring_kernel(
     const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
     uint64_t a_slice, uint64_t rp_slice, uint32_t a_lines, const int8_t* __restrict__ Bhi,
@@ -1144,17 +1139,15 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_ring_kernel(
     uint32_t b_lines, uint32_t nslab, uint32_t nsum_a, uint32_t tiles_r, uint32_t tiles_c, uint32_t xw, uint32_t kp, int32_t k64,
     uint32_t mode, int32_t* __restrict__ pout, uint32_t ksteps, uint32_t* __restrict__ tcnt, Epi epi) {
     constexpr int TM = 32 * RB * WR, TN = 32 * CB * WC;
+    constexpr int NST = 4;                             // stages (even: the fragment registers alternate)
     constexpr int NW = WR * WC, NT = 64 * NW;
     constexpr int A_T = TM * BK, B_T = TN * BK;        // plane tile bytes
     constexpr int STAGE = 2 * A_T + 2 * B_T;           // Ah, Al, Bh, Bl
     constexpr int NC = STAGE / 1024 / NW;              // copies per wave and step
     static_assert(STAGE % (1024 * NW) == 0, "equal copies per wave");
-    static_assert(NST >= 4 && NST <= 8 && (NST & 1) == 0, "an even ring (the fragment registers alternate)");
     static_assert(NC * (NST - 1) < 64, "vmcnt is six bits");
     // separate arrays: the compiler then tells the copies in flight from the fragment reads
     __shared__ __attribute__((aligned(1024))) int8_t sm0[STAGE], sm1[STAGE], sm2[STAGE], sm3[STAGE];
-    __shared__ __attribute__((aligned(1024))) int8_t sm4[NST > 4 ? STAGE : 16], sm5[NST > 4 ? STAGE : 16];
-    __shared__ __attribute__((aligned(1024))) int8_t sm6[NST > 6 ? STAGE : 16], sm7[NST > 6 ? STAGE : 16];
     __shared__ int2 rterm[TM], cterm[TN];              // (h, l) halves
     __shared__ uint32_t ticket;                        // kSplitFix: the tile's arrival ticket
 
@@ -1216,15 +1209,10 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_ring_kernel(
             for (int i = 4; i < TP; i++) tpart[q][i] = pp[(uint64_t)min((uint32_t)i, ns - 1) * stride];
         }
     }
-#define CM_ST(i) ((i) % NST == 0 ? sm0 : (i) % NST == 1 ? sm1 : (i) % NST == 2 ? sm2 : (i) % NST == 3 ? sm3 \
-                  : (i) % NST == 4 ? sm4 : (i) % NST == 5 ? sm5 : (i) % NST == 6 ? sm6 : sm7)
+#define CM_ST(i) ((i) % NST == 0 ? sm0 : (i) % NST == 1 ? sm1 : (i) % NST == 2 ? sm2 : sm3)
     issue(sm0, 0);
     if (1 < nk) issue(sm1, 1);
     if (2 < nk) issue(sm2, 2);
-    if (NST > 4 && 3 < nk) issue(sm3, 3);
-    if (NST > 4 && 4 < nk) issue(sm4, 4);
-    if (NST > 6 && 5 < nk) issue(sm5, 5);
-    if (NST > 6 && 6 < nk) issue(sm6, 6);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < TE; q++) {
@@ -1316,14 +1304,6 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void gemm_ring_kernel(
         CM_RSTEP(1, f1, f0)
         CM_RSTEP(2, f0, f1)
         CM_RSTEP(3, f1, f0)
-        if constexpr (NST > 4) {
-            CM_RSTEP(4, f0, f1)
-            CM_RSTEP(5, f1, f0)
-        }
-        if constexpr (NST > 6) {
-            CM_RSTEP(6, f0, f1)
-            CM_RSTEP(7, f1, f0)
-        }
     }
 #undef CM_RSTEP
 #undef CM_ST
@@ -1593,17 +1573,16 @@ __global__ __launch_bounds__(256, NK > 1 ? 3 : 4) void conv_point_wide_kernel(
     const int8_t* __restrict__ Ahi, const int8_t* __restrict__ Alo, const int32_t* __restrict__ rpart,
     const int16_t* __restrict__ x, uint32_t K, uint32_t plane, uint32_t cols, uint32_t blocks_r, uint32_t blocks_c,
     uint32_t tiles_r, uint32_t gt, uint32_t kp, uint32_t mode, EpiConv epi) {
-    constexpr int PX = 1;                                                    // two pixels a lane measured the same
     __shared__ int2 rterm[kPointTiles * 32];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, lh = lane >> 5;
     const TilePos tp = tile_pos(blockIdx.x, blocks_r, blocks_c, 1);
     const uint32_t t0 = tp.tr * gt, t1 = min(t0 + gt, tiles_r);
-    const uint32_t col = ((tp.tc * 4 + wave) * 32 + l32) * PX;               // pixels over all images
+    const uint32_t col = (tp.tc * 4 + wave) * 32 + l32;      // a pixel a lane, over all images (two measured the same)
     const bool live = col < cols;
-    const uint32_t c = min(col, cols - PX), img = c / plane, p = c - img * plane;
+    const uint32_t c = min(col, cols - 1), img = c / plane, p = c - img * plane;
     const uint32_t pix = 2 * (img * K * plane + p), row = 2 * plane;
     const uint64_t aoff = (uint64_t)(t0 * 32 + l32) * kp + 16 * lh;
-    PointPx<PX, RAG> px[NK];
+    PointPx<1, RAG> px[NK];
 #pragma unroll
     for (int k = 0; k < NK; k++) px[k].load(x, pix, row, 32 * k + 16 * lh, K);
     v4i ah[NK], al[NK];
@@ -1620,37 +1599,25 @@ __global__ __launch_bounds__(256, NK > 1 ? 3 : 4) void conv_point_wide_kernel(
         rterm[i] = make_int2(epi.row_bias(t0 * 32 + i) - (int32_t)(64 * K) + (sum >> 1), (sum & 1) << 7);
     }
     __syncthreads();
-    v4i bh[NK][PX], bl[NK][PX];
-    int32_t sh[PX], sl[PX], ch[PX], cl[PX];
-#pragma unroll
-    for (int j = 0; j < PX; j++) sh[j] = sl[j] = 0;
+    v4i bh[NK][1], bl[NK][1];
+    int32_t sh[1] = {0}, sl[1] = {0};
 #pragma unroll
     for (int k = 0; k < NK; k++) px[k].planes(bh[k], bl[k], sh, sl, 32 * k + 16 * lh, K);
-#pragma unroll
-    for (int j = 0; j < PX; j++) {
-        int32_t s = (sh[j] << 8) + sl[j];
-        s += __shfl_xor(s, 32, 64);
-        s += (int32_t)(128 * K);                                             // x = 256 h + l + 128
-        ch[j] = s >> 1;
-        cl[j] = (s & 1) << 7;
-    }
+    int32_t s = (sh[0] << 8) + sl[0];
+    s += __shfl_xor(s, 32, 64);
+    s += (int32_t)(128 * K);                                                 // x = 256 h + l + 128
+    const int32_t ch[1] = {s >> 1}, cl[1] = {(s & 1) << 7};
     int16_t* const yb = epi.y + img * epi.img + (uint64_t)(4 * lh) * epi.cs + p;
     auto tiles = [&](auto m) {
         constexpr uint32_t MODE = decltype(m)::value;
         for (uint32_t t = t0; t < t1; t++) {
-            v16i hh[PX], mid[PX], ll[PX];
-#pragma unroll
-            for (int j = 0; j < PX; j++) hh[j] = mid[j] = ll[j] = v16i{};
+            v16i hh = v16i{}, mid = v16i{}, ll = v16i{};
 #pragma unroll
             for (int k = 0; k < NK; k++) {
-#pragma unroll
-                for (int j = 0; j < PX; j++) {
-                    hh[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[k], bh[k][j], hh[j], 0, 0, 0);
-                    mid[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[k], bl[k][j], mid[j], 0, 0, 0);
-                    ll[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al[k], bl[k][j], ll[j], 0, 0, 0);
-                }
-#pragma unroll
-                for (int j = 0; j < PX; j++) mid[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(al[k], bh[k][j], mid[j], 0, 0, 0);
+                hh = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[k], bh[k][0], hh, 0, 0, 0);
+                mid = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[k], bl[k][0], mid, 0, 0, 0);
+                ll = __builtin_amdgcn_mfma_i32_32x32x32_i8(al[k], bl[k][0], ll, 0, 0, 0);
+                mid = __builtin_amdgcn_mfma_i32_32x32x32_i8(al[k], bh[k][0], mid, 0, 0, 0);
             }
             if (t + 1 < t1) load_a(t + 1);
             if (live) {
@@ -1665,10 +1632,8 @@ __global__ __launch_bounds__(256, NK > 1 ? 3 : 4) void conv_point_wide_kernel(
                         if (dst == nullptr) continue;
                         dst += p;
                     }
-                    int32_t h[PX], m2[PX], l[PX];
-#pragma unroll
-                    for (int j = 0; j < PX; j++) h[j] = hh[j][r], m2[j] = mid[j][r], l[j] = ll[j][r];
-                    point_out<MODE, PX>(dst, h, m2, l, rterm[(t - t0) * 32 + 4 * lh + rl], ch, cl, epi.lo, epi.hi);
+                    const int32_t h[1] = {hh[r]}, m2[1] = {mid[r]}, l[1] = {ll[r]};
+                    point_out<MODE, 1>(dst, h, m2, l, rterm[(t - t0) * 32 + 4 * lh + rl], ch, cl, epi.lo, epi.hi);
                 }
             }
         }
@@ -1679,10 +1644,10 @@ __global__ __launch_bounds__(256, NK > 1 ? 3 : 4) void conv_point_wide_kernel(
 
 // ---------------------------------------------------------------- standard conv, few taps
 // A standard convolution whose taps per output (in_ch kh kw <= 80) are few -- a network's stem
-// over its 1 .. 4 input channels, the 1x1 convolutions of up to 80 channels -- straight on the
-// VALU instead of im2col + GEMM (which would pad each kernel position to 16 channels, and
-// whose folded 1x1 operand costs a transposing split; such products are bound by their output
-// bytes, not by the multiplies): a lane per output pixel over OG output channels, its
+// over its 1 .. 4 input channels, the 1x1 convolutions of up to 80 channels whose weights come packed
+// with the call (split once, they run from their pixels, above) -- straight on the VALU instead of
+// im2col + GEMM (which would pad each kernel position to 16 channels; such products are bound by
+// their output bytes, not by the multiplies): a lane per output pixel over OG output channels, its
 // taps gathered once (zero outside the input) and packed in pairs, each channel's sum by
 // v_dot2_i32_i16 against the channel's pairs staged in LDS (read by every lane at one
 // address).  The sum is int32 where that is exact -- the wrap path (the int32 wrap is its
@@ -2816,8 +2781,8 @@ int run_gemm(const Planes& A, const Planes& B, uint32_t batch, uint32_t k, Epi e
               A.kp, (int32_t)(64 * k), mode, pout, ksteps, tcnt, epi)
     switch (pl.id) {
     case kPlan256.id: CM_GEMM(512, gemm_planes_kernel<4, 3, Epi>); break;
-    case kRing64.id: CM_GEMM(256, gemm_ring_kernel<1, 1, 2, 2, 4, Epi>); break;
-    case kRing128.id: CM_GEMM(512, gemm_ring_kernel<1, 2, 4, 2, 4, Epi>); break;
+    case kRing64.id: CM_GEMM(256, gemm_ring_kernel<1, 1, 2, 2, Epi>); break;
+    case kRing128.id: CM_GEMM(512, gemm_ring_kernel<1, 2, 4, 2, Epi>); break;
     default: CM_GEMM(256, gemm_planes_kernel<2, 2, Epi>); break;
     }
 #undef CM_GEMM
@@ -2898,7 +2863,7 @@ int split_b(const int16_t* b, uint64_t b_slice, uint32_t k, uint32_t m, uint32_t
                   B.nslab);
         return CM_OK;
     }
-    return run_split<SrcMatB, false>(SrcMatB{b, m, k, m, layout, gemv_kw}, b_slice, B, s);
+    return run_split<SrcGemvB, false>(SrcGemvB{b, k, m, gemv_kw}, b_slice, B, s);
 }
 
 // The skinny path of cm_matmul (wrap32, n <= 32): slices of kSkinnyKc k.
