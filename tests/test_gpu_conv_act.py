@@ -1,6 +1,6 @@
 """A convolution with the RELU / RELU6 that follows it fused (cm_conv_act, cm_conv_planes_act)
 against the oracle's two unit calls -- the convolution, then VectorOP op 4 / 5 on its raw
-output -- on every conv path (the folded 1x1 GEMM, im2col, the three depthwise kernels), with
+output -- on every conv path (1x1 from their pixels and folded, im2col, few-tap, the depthwise kernels), with
 full-range operands so that both bounds bite; and MobileNetV2's forward with only its logits
 kept (every conv + RELU6 pair fused) against the oracle's graph."""
 import numpy as np

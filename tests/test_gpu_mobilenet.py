@@ -1,6 +1,6 @@
 """MobileNetV2 (Q8.8) on the GPU (Simulator) against the value-domain restatement of the
-reference simulator (oracle_graph), every tensor bit for bit: the stem and pointwise
-convolutions on the plane GEMM, the depthwise 3x3 kernels at strides 1 and 2, RELU6 and the
+reference simulator (oracle_graph), every tensor bit for bit: the stem, the pointwise
+convolutions from their pixels, the depthwise 3x3 kernels at strides 1 and 2, RELU6 and the
 residual ADD on VectorOP, the global average pool and the classifier MatMul."""
 import numpy as np
 import pytest
@@ -12,8 +12,8 @@ from oracle import graph_sim as oracle_graph
 pytestmark = pytest.mark.gpu
 
 
-# (32, 224): the configuration's own batch -- the 1x1 convolutions fold 32 images into their
-# GEMM columns (up to 401 408 lines), every image compared
+# (32, 224): the configuration's own batch -- the 1x1 convolutions over the pixels of 32 images
+# (up to 401 408), every image compared
 @pytest.mark.parametrize("batch,res,seed", [(1, 32, 0), (2, 64, 1), (1, 224, 2), (32, 224, 5)])
 def test_mobilenet_every_tensor(batch, res, seed):
     g, inputs, _ = models.mobilenet_v2(batch=batch, res=res, seed=seed)

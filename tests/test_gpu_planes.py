@@ -238,7 +238,7 @@ def test_vectorop_planes(U, rows, k, act, arity):
     np.testing.assert_array_equal(part2, rsum)
 
 
-@pytest.mark.parametrize("B,T,H", [(2, 128, 3), (1, 384, 12)])
+@pytest.mark.parametrize("B,T,H", [(2, 128, 3), (1, 384, 12), (13, 64, 5), (10, 128, 5), (9, 256, 3), (6, 384, 3)])
 def test_attention_planes(U, B, T, H):
     """The fused attention's o with its planes (per-head partial sums): o as cm_attention
     writes it, the split, the output projection over the planes."""

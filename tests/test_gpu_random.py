@@ -493,6 +493,8 @@ def _attention_regs():
     (2, 384, 2, 2, 3000),        # BERT-like scores
     (1, 256, 1, 3, 32768),
     (1, 384, 1, 1, 32768),
+    # past 384 blocks of 16 queries (256 at 64 keys): a workgroup of 64 queries a (sequence, head) pair
+    (5, 64, 13, 0, 32768), (7, 128, 7, 1, 32768), (5, 256, 5, 3, 3000), (3, 384, 6, 2, 32768),
 ])
 def test_attention_random(U, oracle_lib, B, T, H, regs, lim):
     """cm_attention against the oracle's chain per (sequence, head): s = K . Q^T (int32 wrap,
@@ -573,8 +575,8 @@ CONV_CASES = [  # batch, C, H, W, M, kh, kw, sh, sw, dh, dw, pt, pl, pb, pr, bia
     (1, 8, 12, 16, 8, 3, 3, 1, 1, 1, 1, 2, 2, 0, 0, 1, 1, True, False),
     (1, 8, 20, 56, 8, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, True, False),
     (2, 8, 9, 32, 8, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, True, True),
-    # 1x1 stride 1 unpadded: the images folded into the GEMM's columns (even / odd planes,
-    # line groups across images, 1280 rows, two k slabs), and 1x1 convs that do not fold
+    # 1x1 stride 1 unpadded, from their pixels (even / odd planes, tiles across images, 1280 rows,
+    # two k slabs), few-tap ones, and 1x1 convs that are not pointwise
     (32, 24, 14, 14, 144, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, False, False),
     (5, 96, 7, 7, 160, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, True, False),
     (2, 320, 8, 8, 1280, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, False, True),
@@ -582,8 +584,8 @@ CONV_CASES = [  # batch, C, H, W, M, kh, kw, sh, sw, dh, dw, pt, pl, pb, pr, bia
     (3, 16, 33, 35, 24, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, False, False),
     (2, 16, 9, 9, 24, 1, 1, 2, 2, 1, 1, 0, 0, 0, 0, 1, 0, False, False),
     (2, 16, 9, 9, 24, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 0, False, False),
-    # folded 1x1 with 2^16 lines and more (the LDS-tiled split): an even and an odd plane (the
-    # first two run on the VALU as few-tap convolutions, the other two on the GEMM)
+    # 1x1 with 2^16 pixels and more: an even and an odd plane (the first two run on the VALU as
+    # few-tap convolutions, the other two from their pixels)
     (4, 24, 128, 128, 40, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, False, False),
     (3, 20, 151, 149, 24, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, True, False),
     (4, 96, 128, 128, 160, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, False, False),
@@ -603,11 +605,22 @@ CONV_CASES = [  # batch, C, H, W, M, kh, kw, sh, sw, dh, dw, pt, pl, pb, pr, bia
     (3, 40, 9, 10, 50, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, True, False),
     (1, 80, 7, 7, 130, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, True, True),
     (2, 20, 9, 9, 24, 2, 2, 1, 1, 1, 1, 1, 0, 0, 1, 1, 0, False, False),
-    # GEMM convolutions of few output tiles and long k: MobileNetV2's 7 x 7 960 -> 160 (folded),
-    # 3 x 3 over 128 channels (im2col) at full range, 1100 channels wrapped
+    # few output tiles and long k: MobileNetV2's 7 x 7 960 -> 160 and 1100 channels wrapped (from their
+    # pixels), 3 x 3 over 128 channels (im2col) at full range
     (4, 960, 7, 7, 160, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, False, False),
     (2, 128, 8, 8, 64, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, 0, True, False),
     (2, 1100, 7, 7, 320, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, True, True),
+    # folded 1x1: past 64 input channels, 1280 output channels or 2^19 weights, and two tiles a unit; few
+    # lines (16 a workgroup, on 128- and 64-row ring tiles), 2^14 of them (a wave per 64 k), 2^16 (the
+    # LDS-tiled split), 256-row tiles; even and odd planes, both output rules
+    (32, 72, 7, 7, 1300, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, True, False),
+    (12, 520, 12, 10, 1010, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, False, False),
+    (12, 520, 11, 11, 1010, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, True, True),
+    (8, 66, 46, 46, 1284, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, True, False),
+    (9, 80, 43, 43, 1290, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, False, True),
+    (2, 68, 182, 182, 1281, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, False, False),
+    (3, 65, 149, 149, 1283, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 0, True, True),
+    (16, 600, 18, 18, 1290, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 1, 0, True, False),
 ]
 
 

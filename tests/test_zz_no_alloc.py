@@ -1,7 +1,7 @@
 """cm_matmul_noalloc (the matmul entry point that allocates nothing) against cm_matmul, bit for
 bit, through the C ABI: the plane GEMM (Q8.8 saturate, batched A, packed B), the wrap-mode
-split over k (partials in the scratch) and the skinny path (split-k partials in the scratch),
-each as two calls in a row, the second smaller, so the second reads a scratch the first left
+split over k (partials in the scratch), products whose first plan does not fit the scratch and
+the skinny path (split-k partials in the scratch), each as two calls in a row, the second smaller, so the second reads a scratch the first left
 behind; and a call past the scratch maximum refused."""
 import numpy as np
 import pytest
@@ -35,6 +35,9 @@ def _both(a, b, n, k, m, batch, a_bs, b_packed, wrap32):
 CASES = {
     "plane_gemm_q88": [(512, 2048, 1024, 2, 1, 1, False), (96, 320, 160, 1, 0, 0, False)],
     "wrap_split_k": [(128, 2048, 256, 1, 0, 0, True), (64, 1024, 128, 1, 0, 1, True)],
+    # planes and partials, or rows rounded up to a tile, past the scratch: 64-row tiles without a split
+    "replanned_split": [(1536, 8192, 1024, 1, 0, 0, True), (65, 200, 70, 1, 0, 0, True)],
+    "replanned_rows": [(130, 384, 130, 350, 1, 0, False), (33, 130, 40, 3, 1, 0, False)],
     "skinny_split_k": [(16, 960, 2560, 1, 0, 2, True), (3, 256, 64, 1, 0, 0, True)],
 }
 
