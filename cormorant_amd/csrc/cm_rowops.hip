@@ -205,6 +205,9 @@ __device__ __forceinline__ void stage_addx_params(uint4* lds, const uint8_t* par
 // bounds), from the job's own parameter block in global memory.
 __device__ __forceinline__ void addx_unit_wide(const int (&x)[8], const int (&y)[8], bool ben, int ck, uint32_t u,
                                             uint32_t bq_sh, bool scale, const uint8_t* praw, bool bcast, int (&r)[8]) {
+    // keeps the entries' addresses of this rare path out of a caller's row loop: hoisted, they took two registers a
+    // column and spilled (twelve-wavefront ADDX + NORM with planes: 10 spilled at 168 registers, 147 without)
+    asm volatile("" : "+v"(u));
     for (int l = 0; l < 8; l++) {
         const Param q = ld_param(praw, 8 * u + l, bcast);
         const i128 s = ((i128)x[l] << q.sa) + ((i128)(ben ? y[l] : 0) << q.sb) + ((i128)q.bq << bq_sh);
@@ -379,8 +382,8 @@ __global__ __launch_bounds__(64 * NW) void ro_norm_fast_kernel(Job j, const uint
 // wavefronts per SIMD; here a lane holds one or two units and a row has TPR / 64 wavefronts.
 // ADDX and PL as in ro_norm_fast_kernel: the residual add's int32 output formed in registers,
 // stored and normalised; the output's byte planes and per-slab row sums for the next GEMM.  The
-// bounds hold four wavefronts a SIMD (the launch's four workgroups a CU): ADDX without PL would take
-// 132 registers and three (19204 x 1520 with the residual add, RMS: 112.7 us, 84.7 at four).
+// bounds hold four wavefronts a SIMD (the launch's four workgroups a CU; 19204 x 1520 with the residual
+// add, RMS: 84.7 us at four, 112.7 at three).
 template <int AK, int UPL, bool ADDX, bool PL, int TPR>
 __global__ __launch_bounds__(TPR, UPL > 1 ? 2 : (ADDX && PL ? 3 : 4)) void ro_norm_wg_kernel(
                                                          Job j, const uint8_t* __restrict__ params, uint8_t* pram_dst,
