@@ -2715,15 +2715,17 @@ uint32_t gemm_slices(const GemmPlan& pl, uint64_t tiles, uint32_t nk, uint32_t c
 //     (13.6); and for outputs of at most 64 rows at any width: 24 x 100352 of k 192 18.9 (64 x 128
 //     tiles, two stages: 23.6);
 //   - but 128 x 128 tiles, split over k, for a wrap product whose 64 x 64 tiles would take at most 2 slices
-//     of 48 steps or more: they read half the bytes a product (in 3 slices or more the 64 x 64 tiles stay ahead:
-//     384 x 1024 of k 16384 45.3 in 5, 57.1; so do they below 96 steps where the larger tiles pad more than an
-//     eighth: 3606 x 317 of k 11696 takes 112 on those, 145 on 64 x 64).  On the ring, one workgroup a unit
-//     (A's planes given): 2000 x 1000 of k 3072 33.6 in 2 (64 x 64 34.5; two stages, in 4, 38.8), 2112 x 768 of k
-//     3072 31.4 (31.5; in 5, 35.8), 1250 x 1000 of k 4096 31.2 in 3 (36.2; in 6, 37.4), 640 x 2048 of k 8192 56.1 in 3
-//     (77.0; in 6, 56.5).  On the two stages, two workgroups a unit, where they fill the units better or a slice of
-//     the ring is long, from 64 steps over whole tiles (1536 x 1024 of k 4096 35.9 in 5, the ring in 2 36.5; 2048 x
-//     1024 of k 16384 143.5 in 4, 151.2), from 80 over ragged ones, whose stores cost them more (1500 x 1024 of k
-//     4096 39.0 and 37.0, of k 6144 50.1 and 50.6);
+//     of 48 steps or more: they read half the bytes a product (in 3 slices or more the 64 x 64 tiles stay
+//     ahead: 384 x 1024 of k 16384 45.3 in 5, 57.1; so do they below 96 steps where the larger tiles pad
+//     more than an eighth: 3606 x 317 of k 11696 takes 112 on those, 145 on 64 x 64; and below 64 where two
+//     slices fill less than 7 of 8 units: an encoder layer of 12 x 176 tokens, 2112 x 768 of k 3072 in it,
+//     162.2 on 64 x 64, 164.8).  On the ring, one workgroup a unit (A's planes given): 2000 x 1000 of k
+//     3072 33.6 in 2 (64 x 64 34.5; two stages, in 4, 38.8), 1250 x 1000 of k 4096 31.2 in 3 (36.2; in 6,
+//     37.4), 640 x 2048 of k 8192 56.1 in 3 (77.0; in 6, 56.5).  On the two stages, two workgroups a unit,
+//     where they fill the units better or a slice of the ring is long, from 64 steps over whole tiles (1536
+//     x 1024 of k 4096 35.9 in 5, the ring in 2 36.5; 2048 x 1024 of k 16384 143.5 in 4, 151.2), from 80
+//     over ragged ones, whose stores cost them more (1500 x 1024 of k 4096 39.0 and 37.0, of k 6144 50.1
+//     and 50.6);
 //   - 128 x 128 tiles on the ring with 8 waves while they fit one to a unit: 1040 x 2304 15.1 (two
 //     stages 16.7), 576 x 6272 of k 128 8.0 (11.8), 3072 x 768 14.4 (14.3); but a wrap product that
 //     splits in 3 or more keeps the two-stage kernel, two workgroups a unit: 3072 x 768 of k 3072
@@ -2744,6 +2746,7 @@ GemmPlan gemm_plan(uint32_t n, uint32_t m, uint32_t batch, uint32_t nk, bool wra
         const uint32_t few = slices(kRing64), ring = slices(kRing128), two = slices(kPlan128);
         if (n <= 64 || !wrap || few > 2 || nk / few < 48) return kRing64;
         if (nk / few < 96 && (ring < 2 || 32 * t128 > 9 * tiles(kRing64))) return kRing64;
+        if (nk / few < 64 && ring == 2 && 8 * t128 < 7 * (cus / 2)) return kRing64;
         const uint32_t steps = n % 128 == 0 && m % 128 == 0 ? 64 : 80;
         return nk >= steps && (nk / ring >= steps || 2 * ring < two) ? kPlan128 : kRing128;
     }
