@@ -1991,7 +1991,7 @@ __global__ __launch_bounds__(256) void conv_dw3v_kernel(const int16_t* __restric
 }
 
 // Depthwise 3x3, dilation 1, stride S both ways, over so few columns that the launch is its latency, or
-// over rows of at most 5: each lane computes R output rows of one column (a vertical strip) from the (R - 1) S + 3 input rows' three
+// over the narrowest rows: each lane computes R output rows of one column (a vertical strip) from the (R - 1) S + 3 input rows' three
 // taps, a load a tap with no edge to mend.  One workgroup a unit or fewer, us (conv_dw3_kernel): one
 // image of 96 channels at 14 x 14, stride 2 3.9 (4.3), of 960 at 7 x 7 4.0 (4.25), 32 images of 32 at 3 x 3 3.8
 // (5.3).  Sums as conv_dw3v_kernel.
@@ -3347,12 +3347,19 @@ int conv_run(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y
         }
     }
     if (dw3 && stride_h == stride_w && stride_h <= 2) {
-        // one workgroup a unit or fewer (at 1.3 a unit 384 channels of 32 images at 7 x 7 take 4.65 us, 4.49 below),
-        // or rows that fill no more than half of a lane's 10 columns (960 channels of 64 images, us, and below:
-        // 12 x 3 8.4, 9.3; 3 x 3 4.9, 6.4; 5 x 5 6.85, 7.05)
+        // Lanes a unit up to which the strips win, from both kernels over 9 plane counts of 45 shapes (us, and
+        // conv_dw3_kernel's): one workgroup, 2048 planes of 7 x 7 4.0 (4.2), 12288 at 1.3 4.65 (4.49); more over
+        // rows that fill less than half of a lane's 10 columns (12288 of 12 x 3 3.9 and 5.2, 61440 of 40 x 3 12
+        // % behind), any over rows of 4 at stride 1 (131072 of 20 x 4 20.9 and 24.4) and over planes of at most
+        // 5 x 5 (30720 of 3 x 3 4.2 and 5.4; 131072 of 5 x 5 4 % behind); none at stride 2 over rows of 4 or 8
+        // columns in whole strips (2048 of 8 x 8 5.4 and 4.6)
+        uint64_t most = 256;
+        if ((in_w <= 5 && in_h <= 5) || (in_w == 4 && stride_h == 1)) most = (1ull << 31) / st->cus;
+        else if (stride_h == 2 && (in_w == 4 || in_w == 8) && out_h % 4 == 0) most = 0;
+        else if (in_w <= 3) most = stride_h == 1 ? 1200 : 512;
         const uint32_t R = stride_h == 1 ? 8 : 4, strips = ceil_div(out_h, R);
         const uint64_t items = (uint64_t)batch * out_ch * strips * out_w;
-        if (items < (1ull << 31) && (in_w <= 5 || items <= 256ull * st->cus)) {
+        if (items < (1ull << 31) && items <= most * st->cus) {
 #define CM_DW3S(S_, R_)                                                                                         \
     CM_LAUNCH("conv_dw3_kernel", (conv_dw3_strip_kernel<S_, R_>), dim3(std::min(ceil_div(items, 256), 65536u * 8)), dim3(256), 0, s, x, w, \
               bptr, y, (uint32_t)items, strips, out_ch, in_h, in_w, out_h, out_w, pad_top, pad_left, 16u, cs, y_cn, y_gs, \

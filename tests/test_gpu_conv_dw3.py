@@ -21,12 +21,14 @@ def U():
     return units
 
 
-def _past_strips(batch, ch, oh, ow, stride):
-    """The least channel count of at least ``ch`` past one workgroup a compute unit of the strip kernel
-    (256 lanes, a lane one column of 8 output rows, 4 at stride 2)."""
+def _past_strips(batch, ch, w, oh, ow, stride):
+    """The least channel count of at least ``ch`` past the lanes of the strip kernel (a lane one column of 8
+    output rows, 4 at stride 2): 256 a compute unit, more over rows of at most 3 columns (over rows of 4 at
+    stride 1 and planes of 5 x 5 there is no such count: many of its lanes)."""
     import torch
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    return max(ch, 256 * cus // (batch * -(-oh // (8 if stride == 1 else 4)) * ow) + 1)
+    most = (1200 if stride == 1 else 512) if w <= 3 else 256
+    return max(ch, most * cus // (batch * -(-oh // (8 if stride == 1 else 4)) * ow) + 1)
 
 
 @pytest.mark.parametrize("many", [False, True])
@@ -40,7 +42,7 @@ def test_dw3(U, oracle_lib, batch, ch, h, w, pt, pl, pb, pr, stride, act, wrap, 
     from cormorant_amd.packing import conv_weight_image
     oh, ow = (h + pt + pb - 3) // stride + 1, (w + pl + pr - 3) // stride + 1
     if many:
-        ch = _past_strips(batch, ch, oh, ow, stride)
+        ch = _past_strips(batch, ch, w, oh, ow, stride)
     rng = np.random.default_rng(ch + 7 * h + w + act + stride)
     x = rng.integers(-lim, lim, batch * ch * h * w).astype(np.int16)
     wt = rng.integers(-lim, lim, (ch, 1, 3, 3)).astype(np.int16)
@@ -64,7 +66,7 @@ def test_dw3_y_pattern(U, oracle_lib, h, w, many):
     """Output channel o at (o % 2) cs + (o / 2) gs."""
     from cormorant_amd.packing import conv_weight_image
     rng = np.random.default_rng(w)
-    ch = _past_strips(1, 6, h, w, 1) + 1 & ~1 if many else 6
+    ch = _past_strips(1, 6, w, h, w, 1) + 1 & ~1 if many else 6
     plane = h * w
     cs, cn, gs = ch // 2 * (plane + 5), 2, plane + 5
     x = rng.integers(-2000, 2000, ch * plane).astype(np.int16)
