@@ -270,12 +270,12 @@ __device__ __forceinline__ void addx_unit(const int (&x)[8], const int (&y)[8], 
 // One NORM row of the fast path (norm_row_vals), its int16 results to rc (null: not written) and, with PL, their
 // byte planes and row sums per 1024 columns (unit u in sum u / 128 = k / 2) as row `prow` of
 // `po`.  Wavefront-uniform control.
-template <int UPL, bool PL>
+template <int UPL, bool PL, bool ADDX>
 __device__ __forceinline__ void norm_row(const Job& j, const int (&x)[UPL][8], uint8_t* rc, const uint4* ro_lds,
                                          bool bcast, const uint8_t* tab, uint32_t lane, uint32_t units, bool ln,
                                          bool high, const APlanes& po, u64 prow) {
     int4 o[UPL];
-    norm_row_vals<UPL>(j.n, j.eps, x, ro_lds, bcast, tab, lane, units, ln, high, o);
+    norm_row_vals<UPL, ADDX>(j.n, j.eps, x, ro_lds, bcast, tab, lane, units, ln, high, o);
     int32_t ps[UPL];
 #pragma unroll
     for (int k = 0; k < UPL; k++) {
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(64 * NW) void ro_norm_fast_kernel(Job j, const uint
                 for (int l = 0; l < 8; l++) x[k][l] = r[l];
             }
         }
-        norm_row<UPL, PL>(j, x, j.c != nullptr ? j.c + (u64)i2 * j.c_s2 + (u64)i1 * j.c_s1 : nullptr, ro_lds, bcast, tab,
+        norm_row<UPL, PL, ADDX>(j, x, j.c != nullptr ? j.c + (u64)i2 * j.c_s2 + (u64)i1 * j.c_s1 : nullptr, ro_lds, bcast, tab,
                           lane, units, ln, high, po, row);
         if (row + stride < rows) load_row(row + stride);
     }
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(TPR, UPL > 1 ? 2 : (ADDX && PL ? 3 : 4)) void ro_no
                 for (int l = 0; l < 8; l++) x[k][l] = r[l];
             }
         }
-        NormSums ts = norm_sums_of_wave<UPL>(x);
+        NormSums ts = norm_sums_of_wave<UPL, ADDX>(x);
         if constexpr (SELF) {
             if (it == 0) {
 #pragma unroll

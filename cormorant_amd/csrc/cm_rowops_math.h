@@ -264,9 +264,10 @@ struct NormSums {
     uint32_t amax;
 };
 
-template <int UPL>
-__device__ __forceinline__ NormSums norm_sums(const int (&x)[UPL][8]) {
-    NormSums t{0, 0, 0, 0};
+// A lane's sums at any values; with MAX their maximum too, else the wavefront's, found before.
+template <int UPL, bool MAX>
+__device__ __forceinline__ NormSums norm_sums(const int (&x)[UPL][8], uint32_t amax) {
+    NormSums t{0, 0, 0, MAX ? 0 : amax};
 #pragma unroll
     for (int k = 0; k < UPL; k++) {
 #pragma unroll
@@ -276,8 +277,10 @@ __device__ __forceinline__ NormSums norm_sums(const int (&x)[UPL][8]) {
             const u64 sq = (u64)(v * v);                 // |x| <= 2^31: x^2 <= 2^62
             t.lo += sq;
             t.hi += t.lo < sq ? 1 : 0;
-            const uint32_t av = (uint32_t)(v < 0 ? -v : v);
-            t.amax = av > t.amax ? av : t.amax;
+            if constexpr (MAX) {
+                const uint32_t av = (uint32_t)(v < 0 ? -v : v);
+                t.amax = av > t.amax ? av : t.amax;
+            }
         }
     }
     return t;
@@ -291,15 +294,17 @@ __device__ __forceinline__ void norm_sums_add(NormSums& a, const NormSums& b) {
     a.amax = b.amax > a.amax ? b.amax : a.amax;
 }
 
-// The wavefront's total in every lane.
+// The wavefront's total in every lane (without MAX, amax is the same in every lane already).
+template <bool MAX>
 __device__ __forceinline__ void norm_sums_wave(NormSums& t) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         NormSums o;
         o.s1 = (i64)shfl64((u64)t.s1, off);
         o.lo = shfl64(t.lo, off);
-        o.hi = shfl64(t.hi, off);
-        o.amax = (uint32_t)__shfl_xor((int)t.amax, off, 64);
+        // hi without MAX in one word: 64 lanes x 64 elements of 2^62 at most, 2^10
+        o.hi = MAX ? shfl64(t.hi, off) : (uint32_t)__shfl_xor((int)(uint32_t)t.hi, off, 64);
+        o.amax = MAX ? (uint32_t)__shfl_xor((int)t.amax, off, 64) : t.amax;
         norm_sums_add(t, o);
     }
 }
@@ -320,8 +325,11 @@ constexpr uint32_t kNormShort = 1u << (UPL == 1 ? 23 : UPL == 2 ? 23 : 21);
 // The wavefront's sums (norm_sums, then norm_sums_wave).  Where every |x| is below kNormShort (the
 // residual stream at 2^-15: |value| < 256) a lane adds its elements in int32 and their squares in one
 // 64-bit multiply-add each, the 16 lanes of a row meet over DPP and the four rows in scalar registers,
-// instead of 128-bit carries and seven LDS shuffles a step.
-template <int UPL>
+// instead of 128-bit carries and seven LDS shuffles a step.  Larger values pay for the test; without MAX
+// (a norm by itself) their sums take its maximum (RMS norm of 3072 x 1024: 9.5 us, 9.9 with MAX).  After a
+// residual add MAX stays: without it the compiler orders the next row's loads behind a wait (24576 x 1520
+// with values below the bound 149 us, 165).
+template <int UPL, bool MAX>
 __device__ __forceinline__ NormSums norm_sums_of_wave(const int (&x)[UPL][8]) {
     static_assert(UPL <= 8, "kNormShort");
     int mx = 0, mn = 0;
@@ -340,8 +348,8 @@ __device__ __forceinline__ NormSums norm_sums_of_wave(const int (&x)[UPL][8]) {
     auto row = [](uint32_t v, int r) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 16 * r); };
     const uint32_t amax = max(max(row(am, 0), row(am, 1)), max(row(am, 2), row(am, 3)));
     if (amax >= kNormShort<UPL>) {
-        NormSums t = norm_sums<UPL>(x);
-        norm_sums_wave(t);
+        NormSums t = norm_sums<UPL, MAX>(x, amax);
+        norm_sums_wave<MAX>(t);
         return t;
     }
     int s1 = 0;
@@ -490,11 +498,11 @@ __device__ __forceinline__ void norm_row_finish(uint32_t n, i64 eps, const NormS
 }
 
 // A NORM row held by one wavefront: x[k] = unit lane + 64 k.
-template <int UPL>
+template <int UPL, bool ADDX>
 __device__ __forceinline__ void norm_row_vals(uint32_t n, i64 eps, const int (&x)[UPL][8], const uint4* ro_lds,
                                               bool bcast, const uint8_t* tab, uint32_t lane, uint32_t units, bool ln,
                                               bool high, int4 (&o)[UPL]) {
-    const NormSums t = norm_sums_of_wave<UPL>(x);
+    const NormSums t = norm_sums_of_wave<UPL, ADDX>(x);
     norm_row_finish<UPL>(n, eps, t, x, ro_lds, bcast, tab, lane, 64, units, ln, high, o);
 }
 

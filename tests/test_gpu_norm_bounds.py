@@ -48,7 +48,8 @@ def _run(U, lib, jobs, out_bytes):
 @pytest.mark.parametrize("rows,n,mag,sc", [
     (7, 768, 1 << 20, (34, 43)), (300, 768, (1 << 23) - 1, (33, 33)), (300, 512, 1 << 23, (40, 40)), (9, 520, 1 << 24, (36, 40)),
     (20, 2048, (1 << 21) - 1, (33, 61)), (20, 2304, 1 << 22, (38, 39)), (5, 4096, (1 << 31) - 1, (44, 50)),
-    (40, 768, 1 << 18, (30, 34)), (33, 768, 1 << 18, (32, 32)), (300, 64, 5, (33, 40)), (16, 960, 1 << 12, (62, 63))])
+    (40, 768, 1 << 18, (30, 34)), (33, 768, 1 << 18, (32, 32)), (300, 64, 5, (33, 40)), (16, 960, 1 << 12, (62, 63)),
+    (300, 1024, 1 << 31, (44, 50)), (5, 4096, 1 << 31, (44, 50)), (5, 2048, 1 << 31, (44, 50))])     # a row of -2^31
 def test_norm_magnitudes(U, oracle_lib, rows, n, mag, sc, rms):
     from cormorant_amd import rowops_nodes as rn
     rng = np.random.default_rng(rows + n + sc[0])
